@@ -847,13 +847,31 @@ int xnn_scan_counts(int32_t* row_ptr, int64_t n, void* workspace, xnn_stream_t s
  * (E,3) -> int32 src, dst, packed shift; receiver CSR (ptr_dst, perm_dst) and
  * sender CSR (ptr_src, perm_src), both stable (edge order within a row).
  * Mirrors the orderings of common/models/csr.py:20-51. Shift fields outside
- * [-512, 511] fail with XNN_ECAPACITY (flag written to *overflow on device). */
+ * [-512, 511] fail with XNN_ECAPACITY (flag written to *overflow on device: bit 0 a shift
+ * out of range, bit 1 an index out of [0, N), bit 2 edges not grouped by receiver). */
 size_t xnn_edge_plan_workspace_bytes(int64_t n_edges, int64_t n_nodes);
 int xnn_edge_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t n_edges,
                   int64_t n_nodes, int32_t* src, int32_t* dst, int32_t* shift,
                   int32_t* ptr_dst, int32_t* perm_dst, int32_t* ptr_src, int32_t* perm_src,
                   int32_t* overflow, void* workspace, size_t workspace_bytes,
                   xnn_stream_t stream);
+
+/* The same with the structures' layout and an order of the atoms, in the same launches:
+ * batch (N) int64 (nullable: one structure) -> batch32 (N), n_atoms (B) int64 (nullable
+ * for B = 1) -> node_ptr (B+1); visit (N, nullable): the atoms along a Morton curve of
+ * bins of each structure (fractional coordinates of cell (B,3,3), or positions; ties in
+ * atom order), an ordering hint for the force reductions. pos and cell in geom_dtype.
+ * *flags (device): the bits of xnn_edge_plan, bit 3 batch not sorted, bit 4 batch outside
+ * [0, B), bit 5 n_atoms not summing to N. */
+size_t xnn_graph_plan_workspace_bytes(int64_t n_edges, int64_t n_nodes, int64_t n_graphs,
+                                      int32_t with_visit);
+int xnn_graph_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t n_edges,
+                   int64_t n_nodes, const int64_t* batch, const int64_t* n_atoms,
+                   int64_t n_graphs, int32_t* batch32, int64_t* node_ptr, int geom_dtype,
+                   const void* pos, const void* cell, int32_t* visit, int32_t* src, int32_t* dst,
+                   int32_t* shift, int32_t* ptr_dst, int32_t* perm_dst, int32_t* ptr_src,
+                   int32_t* perm_src, int32_t* flags, void* workspace, size_t workspace_bytes,
+                   xnn_stream_t stream);
 
 /* D3 reference weights (N,7): w_r = exp(-wf (cn - cnref_r)^2) normalized over the
  * species' nref references (a zero norm: weight 1 on the largest-cnref references).

@@ -1,0 +1,88 @@
+"""The edge plan (``xnn_graph_plan``): both CSR orderings, the structures' layout and the
+atom order against NumPy's stable sorts, at the edges of its row sorts and scans."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _lists(name, rng):
+    """``(senders, receivers, atoms)`` of one case."""
+    def random(n, e):
+        return rng.integers(0, n, e), rng.integers(0, n, e), n
+
+    if name == "empty":
+        return np.zeros(0, int), np.zeros(0, int), 5
+    if name == "one":
+        return np.array([0]), np.array([0]), 1
+    if name == "ungrouped":                      # rows of about 40, many waves a row's edge
+        return random(3001, 120_007)
+    if name == "grouped":
+        s, d, n = random(3001, 120_007)
+        return s, np.sort(d), n
+    if name == "two_tiles":                      # more rows than one scan block takes
+        return random(20_011, 33_333)
+    if name == "rows_64_65":
+        d = np.repeat(np.arange(4), [63, 64, 65, 128])
+        return rng.permutation(d), rng.permutation(d), 4
+    if name == "rows_1024_1025":                 # the last row of each sort
+        d = np.repeat(np.arange(5), [1023, 1024, 1025, 0, 5000])
+        return rng.permutation(d), d, 5
+    if name == "sorted_hub":                     # long runs of one sender
+        return np.sort(random(50, 60_000)[0]), random(50, 60_000)[1], 50
+    assert name == "library"                     # mean rows above 8,192
+    return random(3, 30_000)
+
+
+@pytest.mark.parametrize("name", ["empty", "one", "ungrouped", "grouped", "two_tiles", "rows_64_65",
+                                  "rows_1024_1025", "sorted_hub", "library"])
+def test_plan_orderings_are_stable_sorts(name):
+    from xnn_amd.plan import build_plan
+    rng = np.random.default_rng(3)
+    src, dst, n = _lists(name, rng)
+    shift = rng.integers(-512, 512, (len(src), 3))
+    pos = rng.uniform(-20, 20, (n, 3))
+    cut = n // 3
+    plan = build_plan(torch.tensor(np.stack([src, dst]), device=DEV), torch.tensor(shift, device=DEV), n,
+                      torch.tensor(np.arange(n) >= cut, device=DEV).long(),
+                      torch.tensor([cut, n - cut], device=DEV), torch.tensor(pos, device=DEV))
+    assert np.array_equal(plan.src.cpu(), src) and np.array_equal(plan.dst.cpu(), dst)
+    packed = plan.shift.cpu().numpy().astype(np.int64)
+    for a in range(3):
+        field = (packed >> (10 * a)) & 1023
+        assert np.array_equal(np.where(field > 511, field - 1024, field), shift[:, a])
+    for key, ptr, perm in ((src, plan.ptr_src, plan.perm_src), (dst, plan.ptr_dst, plan.perm_dst)):
+        assert np.array_equal(ptr.cpu(), np.concatenate([[0], np.cumsum(np.bincount(key, minlength=n))]))
+        order = np.argsort(key, kind="stable")
+        got = np.arange(len(key)) if perm is None else perm.cpu().numpy()
+        assert np.array_equal(got, order)
+    assert (plan.perm_dst is None) == bool((np.diff(dst) >= 0).all())
+    assert plan.node_ptr.tolist() == [0, cut, n]
+    assert np.array_equal(plan.batch32.cpu(), np.arange(n) >= cut)
+    visit = plan.visit.cpu().numpy()
+    assert np.array_equal(np.sort(visit), np.arange(n))
+    assert (np.diff((visit >= cut).astype(int)) >= 0).all()           # structure by structure
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+def test_visit_order_follows_the_cell(dtype):
+    """Atoms of one bin stay together for any lattice: the cubes of a 16^3 crystal of 8 atoms
+    each are visited one whole cube after another, also from images outside the cell and with
+    a position that is not finite."""
+    from xnn_amd.plan import build_plan
+    rng = np.random.default_rng(1)
+    cell = np.array([[16.0, 0, 0], [3.0, 15.0, 0], [-2.0, 1.0, 17.0]])
+    cube = rng.permutation(np.repeat(np.arange(16 ** 3), 8))
+    frac = (np.stack([cube // 256, cube // 16 % 16, cube % 16], 1) + rng.uniform(.2, .8, (len(cube), 3))) / 16
+    pos = (frac + rng.integers(-2, 3, frac.shape)) @ cell
+    n = len(pos)
+    none = torch.zeros((2, 0), dtype=torch.long, device=DEV)
+    t = torch.tensor(pos, device=DEV, dtype=dtype)
+    c = torch.tensor(cell, device=DEV, dtype=dtype)[None]
+    visit = build_plan(none, None, n, pos=t, cell=c).visit.cpu().numpy()
+    assert (cube[visit].reshape(-1, 8) == cube[visit].reshape(-1, 8)[:, :1]).all()
+    t[5, 1] = float("nan")
+    assert np.array_equal(np.sort(build_plan(none, None, n, pos=t, cell=c).visit.cpu().numpy()),
+                          np.arange(n))

@@ -218,9 +218,13 @@ _SIGNATURES = {
     "xnn_scan_counts": [vp, i64, vp, vp],
     "xnn_edge_plan_workspace_bytes": [i64, i64],
     "xnn_edge_plan": [vp, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp],
+    "xnn_graph_plan_workspace_bytes": [i64, i64, i64, i32],
+    "xnn_graph_plan": [vp, vp, i64, i64, vp, vp, i64, vp, vp, c_int, vp, vp, vp, vp, vp, vp, vp,
+                       vp, vp, vp, vp, vp, sz, vp],
 }
 _RESTYPES = {"xnn_last_error": ctypes.c_char_p, "xnn_scan_workspace_bytes": sz,
-             "xnn_edge_plan_workspace_bytes": sz, "xnn_segment_reduce_workspace_bytes": sz,
+             "xnn_edge_plan_workspace_bytes": sz, "xnn_graph_plan_workspace_bytes": sz,
+             "xnn_segment_reduce_workspace_bytes": sz,
              "xnn_d4_workspace_bytes": sz, "xnn_virial_reduce_workspace_bytes": sz,
              "xnn_d4_plan_bytes": sz, "xnn_edge_force_reduce_virial_workspace_bytes": sz,
              "xnn_energy_stress_max_nodes": i64,

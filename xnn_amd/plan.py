@@ -49,9 +49,16 @@ class EdgePlan:
         return self.ptr_dst.device
 
 
+def _int64(t: Tensor, device) -> Tensor:
+    return t.to(device=device, dtype=torch.int64).contiguous()
+
+
 def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
-               batch: Optional[Tensor] = None, n_atoms: Optional[Tensor] = None) -> EdgePlan:
-    """Build the plan of an edge list on its (GPU) device.
+               batch: Optional[Tensor] = None, n_atoms: Optional[Tensor] = None,
+               pos: Optional[Tensor] = None, cell: Optional[Tensor] = None) -> EdgePlan:
+    """Build the plan of an edge list on its (GPU) device, in one call of the library and
+    one host read (of the checks). With ``pos`` (N, 3) the plan also orders the atoms along
+    a space-filling curve (:attr:`EdgePlan.visit`; ``cell`` (B, 3, 3) or None).
 
     Raises ``ValueError`` for edge indices outside ``[0, n_nodes)``, image
     shifts outside ``[-512, 511]`` or atoms not grouped by structure.
@@ -60,86 +67,55 @@ def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
     if device.type != "cuda":
         raise ValueError("edge plans live on the GPU; move the graph to the device first")
     n_edges = int(edge_index.shape[1])
-    edge_index = edge_index.to(torch.int64).contiguous()
-    if cell_shifts is None or cell_shifts.numel() == 0:
-        shifts = None
+    edge_index = _int64(edge_index, device)
+    shifts = None
+    if cell_shifts is not None and cell_shifts.numel() > 0:
+        shifts = _int64(cell_shifts, device)
+    batch = None if batch is None else _int64(batch, device)
+    n_atoms = None if n_atoms is None else _int64(n_atoms, device)
+    n_graphs = 1 if n_atoms is None else int(n_atoms.shape[0])
+    if pos is not None and n_nodes > 0 and n_graphs > 0:
+        pos = pos.detach().contiguous()
+        if pos.dtype not in (torch.float32, torch.float64):
+            pos = pos.double()
+        geom = _lib.dtype_code(pos.dtype)
+        if cell is not None:
+            cell = cell.detach().reshape(-1, 3, 3).to(device=device, dtype=pos.dtype).contiguous()
+            cell = cell if cell.shape[0] == n_graphs else None
     else:
-        shifts = cell_shifts.to(torch.int64).contiguous()
-    i32 = dict(dtype=torch.int32, device=device)
-    src = torch.empty(n_edges, **i32)
-    dst = torch.empty(n_edges, **i32)
-    shift = torch.empty(n_edges, **i32)
-    ptr_dst = torch.empty(n_nodes + 1, **i32)
-    ptr_src = torch.empty(n_nodes + 1, **i32)
-    perm_dst = torch.empty(n_edges, **i32)
-    perm_src = torch.empty(n_edges, **i32)
-    flag = torch.empty(1, **i32)
-    ws_bytes = int(_lib.load().xnn_edge_plan_workspace_bytes(n_edges, n_nodes))
+        geom, pos, cell = _lib.XNN_F64, None, None
+    want_visit = pos is not None
+    # the int32 arrays of the plan, one allocation (each view keeps it alive)
+    sizes = [n_edges] * 5 + [n_nodes + 1] * 2 + [n_nodes] * (2 if want_visit else 1) + [1]
+    views = torch.empty(sum(sizes), dtype=torch.int32, device=device).split(sizes)
+    src, dst, shift, perm_dst, perm_src, ptr_dst, ptr_src, batch32 = views[:8]
+    visit = views[8] if want_visit else None
+    flags = views[-1]
+    node_ptr = torch.empty(n_graphs + 1, dtype=torch.int64, device=device)
+    ws_bytes = int(_lib.load().xnn_graph_plan_workspace_bytes(n_edges, n_nodes, n_graphs,
+                                                              int(want_visit)))
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=device)
-    _lib.call("xnn_edge_plan", _lib.ptr(edge_index), _lib.ptr(shifts), n_edges, n_nodes,
-              _lib.ptr(src), _lib.ptr(dst), _lib.ptr(shift), _lib.ptr(ptr_dst), _lib.ptr(perm_dst),
-              _lib.ptr(ptr_src), _lib.ptr(perm_src), _lib.ptr(flag), _lib.ptr(ws), ws_bytes,
-              _lib.stream(device))
-    if batch is None:
-        batch = torch.zeros(n_nodes, dtype=torch.int64, device=device)
-    batch = batch.to(device)
-    if n_atoms is None:
-        n_atoms = torch.tensor([n_nodes], dtype=torch.int64, device=device)
-    n_atoms = n_atoms.to(device=device, dtype=torch.int64)
-    node_ptr = torch.zeros(n_atoms.shape[0] + 1, dtype=torch.int64, device=device)
-    node_ptr[1:] = torch.cumsum(n_atoms, 0)
-    # one host read: overflow flag, receiver grouping, structure grouping, atom count
-    checks = [flag[0].to(torch.int64),
-              (dst[1:] >= dst[:-1]).all().to(torch.int64) if n_edges > 1 else
-              torch.ones((), dtype=torch.int64, device=device),
-              (batch[1:] >= batch[:-1]).all().to(torch.int64) if n_nodes > 1 else
-              torch.ones((), dtype=torch.int64, device=device),
-              node_ptr[-1],
-              ((batch >= 0) & (batch < n_atoms.shape[0])).all().to(torch.int64) if n_nodes > 0
-              else torch.ones((), dtype=torch.int64, device=device)]
-    overflow, grouped, batch_sorted, total, batch_ok = torch.stack(checks).tolist()
-    if overflow & 2:
+    _lib.call("xnn_graph_plan", _lib.ptr(edge_index), _lib.ptr(shifts), n_edges, n_nodes,
+              _lib.ptr(batch), _lib.ptr(n_atoms), n_graphs, _lib.ptr(batch32), _lib.ptr(node_ptr),
+              geom, _lib.ptr(pos), _lib.ptr(cell), _lib.ptr(visit), _lib.ptr(src), _lib.ptr(dst),
+              _lib.ptr(shift), _lib.ptr(ptr_dst), _lib.ptr(perm_dst), _lib.ptr(ptr_src),
+              _lib.ptr(perm_src), _lib.ptr(flags), _lib.ptr(ws), ws_bytes, _lib.stream(device))
+    bits = int(flags.item())
+    if bits & 2:
         raise ValueError(f"edge_index holds atom indices outside [0, {n_nodes})")
-    if overflow & 1:
+    if bits & 1:
         raise ValueError("cell_shifts outside [-512, 511]: the packed int32 shifts cannot hold "
                          "them (wrap the positions into the cell first)")
-    if not batch_ok:
+    if bits & 16:
         raise ValueError("batch holds structure indices outside [0, B)")
-    if not batch_sorted:
+    if bits & 8:
         raise ValueError("the atoms of a batch must be grouped by structure (as collate does)")
-    if total != n_nodes:
-        raise ValueError(f"n_atoms sums to {total}, the graph has {n_nodes} atoms")
-    return EdgePlan(n_nodes=n_nodes, n_edges=n_edges, n_graphs=int(n_atoms.shape[0]), src=src,
-                    dst=dst, shift=shift, ptr_dst=ptr_dst, perm_dst=None if grouped else perm_dst,
-                    ptr_src=ptr_src, perm_src=perm_src, batch32=batch.to(torch.int32),
-                    node_ptr=node_ptr)
-
-
-def _spread10(q: Tensor) -> Tensor:
-    """The 10 low bits of ``q`` (int64) spread to every third bit (Morton interleave)."""
-    q = (q | (q << 16)) & 0x030000FF
-    q = (q | (q << 8)) & 0x0300F00F
-    q = (q | (q << 4)) & 0x030C30C3
-    return (q | (q << 2)) & 0x09249249
-
-
-def spatial_order(pos: Tensor, cell: Optional[Tensor], batch: Tensor, n_graphs: int) -> Tensor:
-    """The atoms sorted along a Morton (Z-order) curve of their positions, structure by
-    structure, int32: fractional coordinates of the cell for one periodic structure, else
-    the batch's bounding box, 10 bits per axis. Neighbours in space end up near one another
-    in the order; an ordering hint only (nothing computed depends on it)."""
-    p = pos.detach().to(torch.float64)
-    if cell is not None and n_graphs == 1 and bool(torch.isfinite(p).all()):
-        c = cell.detach().reshape(-1, 3, 3)[0].to(torch.float64)
-        frac = p @ torch.linalg.inv(c)
-        frac = frac - torch.floor(frac)
-    else:
-        lo, hi = p.min(0).values, p.max(0).values
-        frac = (p - lo) / (hi - lo).clamp(min=1e-9)
-    q = (frac * 1024.0).to(torch.int64).clamp(0, 1023)
-    code = _spread10(q[:, 0]) | (_spread10(q[:, 1]) << 1) | (_spread10(q[:, 2]) << 2)
-    key = (batch.to(torch.int64) << 30) | code
-    return torch.argsort(key, stable=True).to(torch.int32)
+    if bits & 32:
+        raise ValueError(f"n_atoms sums to {int(node_ptr[-1])}, the graph has {n_nodes} atoms")
+    return EdgePlan(n_nodes=n_nodes, n_edges=n_edges, n_graphs=n_graphs, src=src, dst=dst,
+                    shift=shift, ptr_dst=ptr_dst, perm_dst=perm_dst if bits & 4 else None,
+                    ptr_src=ptr_src, perm_src=perm_src, batch32=batch32, node_ptr=node_ptr,
+                    visit=visit)
 
 
 def plan_for(graph) -> EdgePlan:
@@ -151,9 +127,7 @@ def plan_for(graph) -> EdgePlan:
             and cached[2] == graph.num_nodes):
         return cached[3]
     plan = build_plan(graph.edge_index, graph.cell_shifts, graph.num_nodes, graph.batch,
-                      graph.n_atoms)
-    if plan.n_nodes > 0:
-        plan.visit = spatial_order(graph.pos, graph.cell, plan.batch32, plan.n_graphs)
+                      graph.n_atoms, graph.pos, graph.cell)
     object.__setattr__(graph, "_xnn_plan",
                        (graph.edge_index, graph.cell_shifts, graph.num_nodes, plan))
     return plan
