@@ -1117,31 +1117,52 @@ def triple_graph(pos: Tensor, cell64: Optional[Tensor], pbc: Optional[Tensor], c
     radius graph per structure) and their vectors in bohr,
     ``(pos[dst] - pos[src] + shift @ cell) / bohr``, differentiable in ``pos`` and the
     cell (d4.py:1201-1207 with the in-cutoff mask of 1277)."""
-    from .data import build_neighbor_list
-    eis, vecs = [], []
-    s0 = 0
-    for b, n in enumerate(counts):
-        p = pos[s0:s0 + n]
-        cell_b = None if cell64 is None else cell64[b]
-        pbc_b = None
-        if cell_b is not None:
-            pbc_b = (torch.ones(3, dtype=torch.bool) if pbc is None
-                     else pbc.reshape(-1, 3)[b].detach().cpu().bool())
-            if not bool(pbc_b.any()):
-                cell_b = None
-        if cell_b is None:
-            ei, _ = build_neighbor_list(p.detach(), cutoff_aa)
-            v = p[ei[1]] - p[ei[0]]
-        else:
-            ei, sh = build_neighbor_list(p.detach(), cutoff_aa, cell_b.detach(), pbc_b)
-            v = p[ei[1]] - p[ei[0]] + sh.to(pos.dtype) @ cell_b
-        eis.append(ei + s0)
-        vecs.append(v)
-        s0 += n
-    if not eis:
+    from .data import batched_neighbor_list, build_neighbor_list
+    if not counts or pos.shape[0] == 0:
         return (torch.zeros((2, 0), dtype=torch.long, device=pos.device),
                 pos.new_zeros((0, 3)))
-    return torch.cat(eis, 1), torch.cat(vecs) / BOHR
+    dev, p = pos.device, pos.detach()
+    flags = None
+    if cell64 is not None:
+        flags = (torch.ones((len(counts), 3), dtype=torch.bool) if pbc is None
+                 else pbc.reshape(-1, 3).detach().cpu().bool())
+    if len(counts) > 1 and max(counts) <= 1024 and (flags is None or not bool(flags.any())):
+        # a batch of molecules: one pass
+        ei, sh = batched_neighbor_list(p, torch.tensor(counts), cutoff_aa)
+    else:
+        eis, shs = [], []
+        s0 = 0
+        for b, n in enumerate(counts):
+            if flags is None or not bool(flags[b].any()):
+                e, h = build_neighbor_list(p[s0:s0 + n], cutoff_aa)
+            else:
+                e, h = build_neighbor_list(p[s0:s0 + n], cutoff_aa, cell64[b].detach(), flags[b])
+            eis.append(e + s0 if s0 else e)
+            shs.append(h)
+            s0 += n
+        ei, sh = (eis[0], shs[0]) if len(eis) == 1 else (torch.cat(eis, 1), torch.cat(shs))
+    return ei, _triple_vectors(pos / BOHR, None if cell64 is None else cell64 / BOHR, ei, sh, counts)
+
+
+def _triple_vectors(pos: Tensor, cell: Optional[Tensor], ei: Tensor, sh: Tensor,
+                    counts: List[int]) -> Tensor:
+    """``pos[dst] - pos[src] + shift @ cell`` on the edge kernels: the derivative in the cell
+    is a sum per atom and one over the atoms, where ``shift^T g`` as a matrix product of 3
+    by E by 3 runs on one workgroup (75.7 of the 163 ms of a 700-atom cell's evaluation with
+    2.2 million edges), and the atoms' sums follow the orderings instead of an index sort."""
+    from .ops import edge_vectors
+    from .plan import build_plan
+    node_ptr, batch32 = _batch_tensors(counts, pos.device)
+    try:
+        plan = build_plan(ei, sh if cell is not None else None, pos.shape[0], batch32,
+                          node_ptr[1:] - node_ptr[:-1])
+    except ValueError:
+        # shifts beyond the plan's 10 bits (positions hundreds of cells away)
+        v = pos[ei[1]] - pos[ei[0]]
+        if cell is None:
+            return v
+        return v + (sh.to(pos.dtype)[:, None, :] @ cell[batch32.long()[ei[0]]])[:, 0]
+    return edge_vectors(pos, cell, plan)
 
 
 # --------------------------------------------------------------------------- potentials
