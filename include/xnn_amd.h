@@ -619,6 +619,37 @@ int xnn_eeq_real_apply(const double* pos, int64_t n_nodes, const double* cell, c
                        int32_t nrhs, double* out, void* work, size_t work_bytes,
                        xnn_stream_t stream);
 
+/* The real-space matrix of the conjugate-gradient regime kept packed in 128 x 128 tiles,
+ * for sizes whose pairs in reach fit the memory (8.2 bytes each, an unordered pair once).
+ * All device memory, nt = ceil(N / 128). */
+typedef struct xnn_eeq_tiles {
+  int64_t n_tiles;
+  const int32_t* tile_ij; /* (n_tiles, 2): row and column block, I >= J */
+  const int32_t* index;   /* (nt, nt): a tile's place in the list or -1 (I >= J read) */
+  uint64_t* mask;         /* (n_tiles, 128, 2): the stored columns of each half row */
+  uint32_t* off;          /* (n_tiles, 128, 2): its first value within the tile */
+  const int64_t* base;    /* (n_tiles): the tile's first value */
+} xnn_eeq_tiles;
+
+/* flags (nt, nt) int32: 1 for the tiles (I >= J) with a lattice image within the cutoff;
+ * spheres (nt, 4) the bounding spheres of 128 consecutive atoms (as in
+ * xnn_eeq_real_apply), or NULL for every lower tile. cell: host memory. */
+int xnn_eeq_store_meet(const double* spheres, int64_t n_nodes, const double* cell, double cutoff,
+                       int32_t* flags, xnn_stream_t stream);
+/* Two steps: with counts (n_tiles) int64, mask and off are written and each tile's values
+ * counted; with values, the entries of xnn_eeq_real_matrix with an image within the cutoff
+ * are written from tiles->base on. cell: host memory. */
+int xnn_eeq_store_tiles(const double* pos, int64_t n_nodes, const double* cell, const double* rad,
+                        double alpha, double cutoff, const xnn_eeq_tiles* tiles, int64_t* counts,
+                        double* values, xnn_stream_t stream);
+
+/* out (N, nrhs) = matrix v for v (N, nrhs) row-major, nrhs 1 or 2, from the packed values,
+ * each read once. work: device, of the queried size. Deterministic. */
+int xnn_eeq_store_apply_work_size(int64_t n_tiles, int32_t nrhs, size_t* bytes);
+int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_t n_nodes,
+                        const double* v, int32_t nrhs, double* out, void* work, size_t work_bytes,
+                        xnn_stream_t stream);
+
 /* One diagonal block of the blocked Cholesky factorization of the assembled operator
  * (replaces the factorization of EEQSystem._solve_lu, common/models/eeq.py:312-323, which
  * LU-factors the augmented matrix; the operator is symmetric positive definite and the

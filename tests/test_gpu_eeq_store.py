@@ -1,0 +1,62 @@
+"""The stored real-space product of the EEQ conjugate-gradient regime
+(``xnn_eeq_store_apply``) against the formed matrix, at the tiles' edges."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _system(n, seed=0):
+    gen = torch.Generator().manual_seed(seed)
+    box = 4.0 * max(n, 2) ** (1 / 3)
+    cell = (torch.eye(3) * box + 0.05 * box * torch.rand((3, 3), generator=gen)).double()
+    pos = (torch.rand((n, 3), generator=gen).double() @ cell).to(DEV)
+    rad = (0.8 + torch.rand(n, generator=gen)).double().to(DEV)
+    v = torch.randn((n, 2), generator=gen, dtype=torch.float64).to(DEV)
+    return pos.contiguous(), cell.to(DEV), rad, v
+
+
+@pytest.mark.parametrize("n", [1, 64, 127, 128, 129, 257, 1000])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_stored_tiles_match_the_formed_matrix(n, periodic):
+    from xnn_amd import eeq as E
+    pos, cell, rad, v = _system(n)
+    # a range longer than the small cells (own images) and shorter than the largest
+    cutoff = 30.0 if periodic else float("inf")
+    alpha = E.ewald_alpha(cutoff) if periodic else 0.0
+    host = E._host_cell(cell) if periodic else None
+    R = E.real_matrix(pos, cell if periodic else None, rad, alpha, cutoff)
+    store = E.RealTiles.build(pos, host, rad, alpha, cutoff)
+    # n products of magnitude |R| |v|, each rounded once, and kernel values to a few ulps
+    bound = (n + 16) * 2.3e-16 * (R.abs() @ v.abs())
+    for cols in (slice(0, 1), slice(0, 2)):
+        got = store.apply(v[:, cols].contiguous())
+        assert bool(((got - R @ v[:, cols]).abs() <= bound[:, cols] + 1e-300).all())
+        assert torch.equal(store.apply(v[:, cols].contiguous()), got)
+
+
+def test_far_tiles_are_left_out_and_the_fallback_agrees(monkeypatch):
+    """Two clusters out of each other's reach: their tiles are not stored; without room for
+    the tiles the regime evaluates its pairs at every product, to the same charges."""
+    from xnn_amd import eeq as E
+    gen = torch.Generator().manual_seed(4)
+    n, cutoff = 512, 20.0
+    cell = torch.diag(torch.tensor([30.0, 30.0, 400.0], dtype=torch.float64))
+    pos = torch.rand((n, 3), generator=gen).double() * torch.tensor([30.0, 30.0, 30.0])
+    pos[n // 2:, 2] += 200.0        # the most significant axis of the order
+    pos, cell = pos.to(DEV), cell.to(DEV)
+    rad = torch.full((n,), 1.2, dtype=torch.float64, device=DEV)
+    diag = torch.full((n,), 3.0, dtype=torch.float64, device=DEV)
+    x = torch.randn(n, generator=gen, dtype=torch.float64).to(DEV)
+    alpha = E.ewald_alpha(cutoff)
+    system = E.IterativeEEQSystem(pos, cell, rad, diag, alpha, cutoff)
+    assert system.store is not None and system.store.tiles.n_tiles < 4 * 5 // 2
+    zero = torch.zeros((), dtype=torch.float64, device=DEV)
+    q, mu = system.solve_augmented(x, zero)
+    monkeypatch.setattr(E, "STORE_BYTES", 0)
+    free = E.IterativeEEQSystem(pos, cell, rad, diag, alpha, cutoff)
+    assert free.store is None
+    q2, mu2 = free.solve_augmented(x, zero)
+    # both to a residual of 1e-12 |x|, the operator's smallest eigenvalue of order one
+    assert float((q - q2).abs().max()) <= 2e-11 * float(x.norm())

@@ -46,6 +46,12 @@ class GridPlan(ctypes.Structure):
                 ("workspace_bytes", sz)]
 
 
+class EeqTiles(ctypes.Structure):
+    """``xnn_eeq_tiles``."""
+    _fields_ = [("n_tiles", i64), ("tile_ij", vp), ("index", vp), ("mask", vp), ("off", vp),
+                ("base", vp)]
+
+
 class D4CnParams(ctypes.Structure):
     """``xnn_d4_cn_params``."""
     _fields_ = [("cutoff_cn", dbl), ("cutoff_eeq_cn", dbl), ("kcn", dbl), ("k4", dbl),
@@ -198,6 +204,10 @@ _SIGNATURES = {
     "xnn_eeq_real_grad": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp],
     "xnn_eeq_cholesky_block": [vp, i64, i64, i64, vp, vp, vp],
     "xnn_eeq_cholesky_solve": [vp, i64, vp, vp, i32, vp, vp],
+    "xnn_eeq_store_meet": [vp, i64, vp, dbl, vp, vp],
+    "xnn_eeq_store_tiles": [vp, i64, vp, vp, dbl, dbl, ctypes.POINTER(EeqTiles), vp, vp, vp],
+    "xnn_eeq_store_apply_work_size": [i64, i32, ctypes.POINTER(ctypes.c_size_t)],
+    "xnn_eeq_store_apply": [vp, ctypes.POINTER(EeqTiles), i64, vp, i32, vp, vp, sz, vp],
     "xnn_eeq_real_apply_work_size": [i64, c_int, ctypes.POINTER(ctypes.c_size_t)],
     "xnn_eeq_real_apply": [vp, i64, vp, vp, dbl, dbl, vp, vp, c_int, vp, vp, ctypes.c_size_t, vp],
     "xnn_segment_reduce_f64_noalloc": [c_int, vp, i64, i64, vp, i64, vp, vp],

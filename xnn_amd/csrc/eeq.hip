@@ -315,6 +315,261 @@ __global__ __launch_bounds__(256) void eeq_sum_splits_kernel(const double* __res
   out[k] = s;
 }
 
+// ------------------------------------------------------------------ stored product
+// The same product from the real-space matrix evaluated once (the conjugate-gradient regime
+// multiplies it some fifty times): its lower 128 x 128 tiles, packed. Of each row of a tile
+// that has an image within the cutoff, a bit per column and the values of the set ones (8.2
+// bytes per unordered pair in reach), each read once per product and used for both of its
+// atoms. A block takes a tile, its waves 32 rows each, a lane the columns l and l + 64; the
+// wave holds its 64 half rows' bits and places in its lanes and hands them out as scalars.
+// The column sums stay in the lane, the row sums of 32 (row, side) pairs at a time go
+// through a reduce-scatter over the wave (31 exchanges instead of six butterfly steps a
+// row). Both are written per tile and summed per row by eeq_tiles_sum_kernel in tile order
+// (bitwise reproducible). Bound by reading the values: two columns at 24,000 atoms and 60
+// bohr (1.3 GB) take 331 us = 4.0 TB/s and 35 us of sums, where evaluating the 5.8e8 pairs
+// takes 4,800 us; forming the values takes 4,000 us once.
+constexpr int kStoreTile = 128;
+
+// the lane's place among the lanes of mask below it
+__device__ __forceinline__ uint32_t lanes_below(uint64_t mask) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
+                                   __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+}
+
+// v[l] kept from the halving over lane bit M: lanes with the bit take hi, the others lo, each
+// adding its partner's value of the same slot
+template <int M>
+__device__ __forceinline__ double halve_lanes(double lo, double hi, int lane) {
+  const bool up = lane & M;
+  const double keep = up ? hi : lo;
+  const double give = up ? lo : hi;
+  if constexpr (M == 8) {
+    const int a = __builtin_amdgcn_mov_dpp(__double2loint(give), 0x128, 0xF, 0xF, false);
+    const int b = __builtin_amdgcn_mov_dpp(__double2hiint(give), 0x128, 0xF, 0xF, false);
+    return keep + __hiloint2double(b, a);
+  } else {
+    return keep + xor_lanes<M>(give);
+  }
+}
+
+// the two halves (M = 32) or the 16-lane rows of each half (M = 16): lo stays with the lanes
+// without the bit, hi with the others (row-swap permutes, no selects)
+template <int M>
+__device__ __forceinline__ double halve_swap(double lo, double hi) {
+  const unsigned a0 = (unsigned)__double2loint(lo), a1 = (unsigned)__double2hiint(lo);
+  const unsigned b0 = (unsigned)__double2loint(hi), b1 = (unsigned)__double2hiint(hi);
+  const auto x = M == 32 ? __builtin_amdgcn_permlane32_swap(a0, b0, false, false)
+                         : __builtin_amdgcn_permlane16_swap(a0, b0, false, false);
+  const auto y = M == 32 ? __builtin_amdgcn_permlane32_swap(a1, b1, false, false)
+                         : __builtin_amdgcn_permlane16_swap(a1, b1, false, false);
+  return __hiloint2double((int)y[0], (int)x[0]) + __hiloint2double((int)y[1], (int)x[1]);
+}
+
+// the wave-wide sums of 32 per-lane values: lanes 2k and 2k + 1 return the total of value k
+__device__ __forceinline__ double reduce_scatter32(double (&p)[32], int lane) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) p[k] = halve_swap<32>(p[k], p[k + 16]);
+#pragma unroll
+  for (int k = 0; k < 8; ++k) p[k] = halve_swap<16>(p[k], p[k + 8]);
+#pragma unroll
+  for (int k = 0; k < 4; ++k) p[k] = halve_lanes<8>(p[k], p[k + 4], lane);
+#pragma unroll
+  for (int k = 0; k < 2; ++k) p[k] = halve_lanes<4>(p[k], p[k + 2], lane);
+  p[0] = halve_lanes<2>(p[0], p[1], lane);
+  return p[0] + xor_lanes<1>(p[0]);
+}
+
+template <int NRHS>
+__global__ __launch_bounds__(256) void eeq_tiles_apply_kernel(
+    const double* __restrict__ values, const int32_t* __restrict__ tile_ij,
+    const uint64_t* __restrict__ mask, const uint32_t* __restrict__ off,
+    const int64_t* __restrict__ base, int64_t n, const double* __restrict__ v,
+    double* __restrict__ part) {
+  constexpr int kRows = 32 / NRHS;                 // rows per reduce-scatter
+  __shared__ double sv[kStoreTile * NRHS];         // v of the row block
+  __shared__ double sc[4][kStoreTile * NRHS];      // the waves' column sums
+  const int64_t id = blockIdx.x;
+  const int64_t I = tile_ij[2 * id], J = tile_ij[2 * id + 1];
+  const int lane = threadIdx.x % kWave, w = wave_in_block();
+  // half row 64 w + lane of the tile: row 32 w + lane / 2, columns 64 (lane % 2) + 0..63
+  const int64_t half_row = id * (2 * kStoreTile) + 64 * w + lane;
+  const uint64_t my_mask = mask[half_row];
+  const int my_off = (int)off[half_row];
+  const int mask_lo = (int)(uint32_t)my_mask, mask_hi = (int)(uint32_t)(my_mask >> 32);
+  const double* vals = values + base[id];
+  for (int k = threadIdx.x; k < kStoreTile * NRHS; k += 256) {
+    const int64_t at = I * kStoreTile * NRHS + k;
+    sv[k] = at < n * NRHS ? v[at] : 0.0;
+  }
+  double vj[2][NRHS], col[2][NRHS];
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) {
+      const int64_t j = J * kStoreTile + lane + 64 * h;
+      vj[h][r] = j < n ? v[j * NRHS + r] : 0.0;
+      col[h][r] = 0.0;
+    }
+  __syncthreads();
+  double* out = part + id * (2 * kStoreTile * NRHS);
+  for (int b = 0; b < 32; b += kRows) {
+    double a[kRows][2];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = 2 * (b + q) + h;
+        const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mask_lo, k) |
+                           (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mask_hi, k) << 32;
+        const int at = __builtin_amdgcn_readlane(my_off, k) + (int)lanes_below(m);
+        // every lane loads (an unset column the next value of the tile or, past its last
+        // one, its first), so that no load waits for a branch
+        const double x = vals[(m >> lane) & 1 ? at : 0];
+        a[q][h] = (m >> lane) & 1 ? x : 0.0;
+      }
+    double p[32];
+#pragma unroll
+    for (int q = 0; q < kRows; ++q)
+#pragma unroll
+      for (int r = 0; r < NRHS; ++r) {
+        p[q * NRHS + r] = fma(a[q][1], vj[1][r], a[q][0] * vj[0][r]);
+        const double vi = sv[(32 * w + b + q) * NRHS + r];
+        col[0][r] = fma(a[q][0], vi, col[0][r]);
+        col[1][r] = fma(a[q][1], vi, col[1][r]);
+      }
+    const double t = reduce_scatter32(p, lane);
+    if ((lane & 1) == 0) out[(32 * w + b) * NRHS + lane / 2] = t;
+  }
+#pragma unroll
+  for (int h = 0; h < 2; ++h)
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) sc[w][(lane + 64 * h) * NRHS + r] = col[h][r];
+  __syncthreads();
+  for (int k = threadIdx.x; k < kStoreTile * NRHS; k += 256)
+    out[kStoreTile * NRHS + k] = ((sc[0][k] + sc[1][k]) + sc[2][k]) + sc[3][k];
+}
+
+// out of row block I: the row sums of its tiles (I, J <= I) and the column sums of the tiles
+// (K > I, I), 1024 / (128 NRHS) partial sums over the blocks taken in turn, added in order
+template <int NRHS>
+__global__ __launch_bounds__(1024) void eeq_tiles_sum_kernel(const double* __restrict__ part,
+                                                             const int32_t* __restrict__ index,
+                                                             int64_t n, int64_t nt,
+                                                             double* __restrict__ out) {
+  constexpr int kW = kStoreTile * NRHS, kGroups = 1024 / kW, kAhead = 8;
+  __shared__ double sums[kGroups][kW];
+  const int64_t I = blockIdx.x;
+  const int k = threadIdx.x % kW, g = threadIdx.x / kW;
+  double s = 0.0;
+  for (int64_t K0 = g; K0 < nt; K0 += kGroups * kAhead) {
+    double x[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int64_t K = K0 + u * kGroups;
+      const int64_t hi = K > I ? K : I, lo = K > I ? I : K;
+      const int64_t id = K < nt ? (int64_t)index[hi * nt + lo] : -1;
+      x[u] = id >= 0 ? part[(id * 2 + (K > I ? 1 : 0)) * kW + k] : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) s += x[u];
+  }
+  sums[g][k] = s;
+  __syncthreads();
+  if (g != 0) return;
+#pragma unroll
+  for (int q = 1; q < kGroups; ++q) s += sums[q][k];
+  const int64_t at = I * kW + k;
+  if (at < n * NRHS) out[at] = s;
+}
+
+// flags[I * nt + J] = 1 for the lower tiles with an image within the cutoff, else 0
+__global__ __launch_bounds__(256) void eeq_store_meet_kernel(EeqCell C, const double* __restrict__ tiles,
+                                                             int64_t nt, double cutoff,
+                                                             int32_t* __restrict__ flags) {
+  const int64_t k = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (k >= nt * nt) return;
+  const int64_t I = k / nt, J = k % nt;
+  flags[k] = J <= I && (tiles == nullptr || eeq_tiles_meet(C, tiles, I, J, cutoff)) ? 1 : 0;
+}
+
+// One tile: which columns of each row have an image within the cutoff (FILL = false: the
+// bits, each half row's place and the number of values), and their entries of
+// eeq_real_matrix_kernel (FILL). A wave takes 32 rows, a lane the columns l and l + 64.
+template <bool FILL>
+__global__ __launch_bounds__(256) void eeq_store_kernel(
+    const double* __restrict__ pos, int64_t n, EeqCell C, const double* __restrict__ rad,
+    double alpha, double cut2, const int32_t* __restrict__ tile_ij, uint64_t* __restrict__ mask,
+    uint32_t* __restrict__ off, int64_t* __restrict__ count, const int64_t* __restrict__ base,
+    double* __restrict__ values) {
+  __shared__ double sp[3][kStoreTile], sa[kStoreTile];
+  __shared__ uint32_t place[kStoreTile * 2], wave_total[4];
+  const int64_t id = blockIdx.x, i0 = (int64_t)tile_ij[2 * id] * kStoreTile;
+  const int64_t j0 = (int64_t)tile_ij[2 * id + 1] * kStoreTile;
+  const int lane = threadIdx.x % kWave, w = wave_in_block();
+  if (threadIdx.x < kStoreTile) {
+    const int c = threadIdx.x;
+    const int64_t i = i0 + c < n ? i0 + c : 0;
+    double p[3] = {pos[3 * i], pos[3 * i + 1], pos[3 * i + 2]};
+    if (C.periodic) to_frac(C, pos[3 * i], pos[3 * i + 1], pos[3 * i + 2], p);
+#pragma unroll
+    for (int q = 0; q < 3; ++q) sp[q][c] = p[q];
+    sa[c] = FILL ? rad[i] * rad[i] : 0.0;
+  }
+  double pj[2][3], aj2[2];
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int64_t j = j0 + lane + 64 * h, jc = j < n ? j : 0;
+#pragma unroll
+    for (int q = 0; q < 3; ++q) pj[h][q] = pos[3 * jc + q];
+    if (C.periodic) to_frac(C, pos[3 * jc], pos[3 * jc + 1], pos[3 * jc + 2], pj[h]);
+    aj2[h] = FILL ? rad[jc] * rad[jc] : 0.0;
+  }
+  __syncthreads();
+  uint32_t total = 0;
+  for (int q = w * 32; q < w * 32 + 32; ++q)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t j = j0 + lane + 64 * h, row = (id * kStoreTile + q) * 2 + h;
+      const double d0 = pj[h][0] - sp[0][q], d1 = pj[h][1] - sp[1][q], d2 = pj[h][2] - sp[2][q];
+      const bool pair = j < n && i0 + q < n;
+      double k = 0.0;
+      bool near = false;
+      const double gam = FILL ? rsq_nr(sa[q] + aj2[h]) : 0.0;
+      const auto add = [&](double dx, double dy, double dz, int, int, int) {
+        near = true;
+        if constexpr (FILL) {
+          const double r2 = dx * dx + dy * dy + dz * dz;
+          k += screened_inv(r2, rsq_nr(r2), gam, alpha);
+        }
+      };
+      if (pair && C.periodic) {
+        for_images_frac(C, C.reach, d0, d1, d2, cut2, add);
+      } else if (pair && i0 + q != j && d0 * d0 + d1 * d1 + d2 * d2 <= cut2) {
+        add(d0, d1, d2, 0, 0, 0);
+      }
+      if constexpr (FILL) {
+        const uint64_t m = mask[row];
+        if ((m >> lane) & 1) values[base[id] + off[row] + lanes_below(m)] = k;
+      } else {
+        const uint64_t m = __ballot(near);
+        if (lane == 0) {
+          mask[row] = m;
+          place[q * 2 + h] = total;
+        }
+        total += __popcll(m);
+      }
+    }
+  if constexpr (!FILL) {
+    if (lane == 0) wave_total[w] = total;
+    __syncthreads();
+    const int k = threadIdx.x;                      // one half row a thread
+    uint32_t before = 0;
+    for (int x = 0; x < k / 64; ++x) before += wave_total[x];
+    off[id * (2 * kStoreTile) + k] = before + place[k];
+    if (k == 0) count[id] = (int64_t)wave_total[0] + wave_total[1] + wave_total[2] + wave_total[3];
+  }
+}
+
 static int64_t eeq_apply_splits(int64_t n) {
   const int64_t tiles = (n + kApplyTile - 1) / kApplyTile;
   if (tiles == 0) return 1;
@@ -769,6 +1024,83 @@ int xnn_eeq_real_apply(const double* pos, int64_t n_nodes, const double* cell, c
   const int64_t m = n_nodes * nrhs;
   hipLaunchKernelGGL(eeq_sum_splits_kernel, dim3((unsigned)grid_1d(m, 256)), dim3(256), 0, s, part,
                      splits, m, out);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_eeq_store_meet(const double* tiles, int64_t n_nodes, const double* cell, double cutoff,
+                       int32_t* flags, xnn_stream_t stream) {
+  XNN_REQUIRE(n_nodes >= 0, "negative size");
+  if (n_nodes == 0) return XNN_OK;
+  XNN_REQUIRE(flags != nullptr && cutoff > 0.0, "NULL flags or a cutoff that is not positive");
+  XNN_REQUIRE(n_nodes <= (int64_t(1) << 21), "at most 2^21 atoms");
+  EeqCell C;
+  XNN_REQUIRE(eeq_cell(cell, cutoff, C), "singular cell");
+  XNN_REQUIRE(eeq_reach_ok(C, cutoff), "the real-space range spans more than %g cells",
+              kMaxReach);
+  const int64_t nt = (n_nodes + kStoreTile - 1) / kStoreTile;
+  hipLaunchKernelGGL(eeq_store_meet_kernel, dim3((unsigned)grid_1d(nt * nt, 256)), dim3(256), 0,
+                     as_hip(stream), C, tiles, nt, cutoff, flags);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_eeq_store_tiles(const double* pos, int64_t n_nodes, const double* cell, const double* rad,
+                        double alpha, double cutoff, const xnn_eeq_tiles* tiles, int64_t* counts,
+                        double* values, xnn_stream_t stream) {
+  XNN_REQUIRE(n_nodes >= 0 && tiles != nullptr && tiles->n_tiles >= 0, "negative size or NULL tiles");
+  if (n_nodes == 0 || tiles->n_tiles == 0) return XNN_OK;
+  XNN_REQUIRE(pos && rad && tiles->tile_ij && tiles->mask && tiles->off, "NULL input or output");
+  XNN_REQUIRE((values == nullptr) != (counts == nullptr), "either counts or values");
+  XNN_REQUIRE(values == nullptr || tiles->base, "NULL tile bases");
+  XNN_REQUIRE(n_nodes <= (int64_t(1) << 21) && tiles->n_tiles < (int64_t(1) << 31), "too many tiles");
+  XNN_REQUIRE(cutoff > 0.0 && alpha >= 0.0, "cutoff must be positive, alpha non-negative");
+  XNN_REQUIRE(cell != nullptr || alpha == 0.0, "a molecule takes alpha = 0");
+  EeqCell C;
+  XNN_REQUIRE(eeq_cell(cell, cutoff, C), "singular cell");
+  XNN_REQUIRE(eeq_reach_ok(C, cutoff), "the real-space range spans more than %g cells",
+              kMaxReach);
+  const auto k = values != nullptr ? eeq_store_kernel<true> : eeq_store_kernel<false>;
+  hipLaunchKernelGGL(k, dim3((unsigned)tiles->n_tiles), dim3(256), 0, as_hip(stream), pos, n_nodes,
+                     C, rad, alpha, cutoff * cutoff, tiles->tile_ij, tiles->mask, tiles->off, counts,
+                     tiles->base, values);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_eeq_store_apply_work_size(int64_t n_tiles, int32_t nrhs, size_t* bytes) {
+  XNN_REQUIRE(n_tiles >= 0 && bytes != nullptr, "negative size or NULL output");
+  XNN_REQUIRE(nrhs == 1 || nrhs == 2, "one or two right-hand sides (got %d)", (int)nrhs);
+  *bytes = sizeof(double) * (size_t)(std::max<int64_t>(n_tiles, 1) * 2 * kStoreTile * nrhs);
+  return XNN_OK;
+}
+
+int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_t n_nodes,
+                        const double* v, int32_t nrhs, double* out, void* work, size_t work_bytes,
+                        xnn_stream_t stream) {
+  XNN_REQUIRE(n_nodes >= 0 && tiles != nullptr, "negative size or NULL tiles");
+  size_t need = 0;
+  const int rc = xnn_eeq_store_apply_work_size(tiles->n_tiles, nrhs, &need);
+  if (rc != XNN_OK) return rc;
+  if (n_nodes == 0) return XNN_OK;
+  XNN_REQUIRE(values && v && out && work, "NULL input, output or workspace");
+  XNN_REQUIRE(tiles->n_tiles > 0 && tiles->tile_ij && tiles->index && tiles->mask && tiles->off &&
+                  tiles->base,
+              "empty or NULL tile list");
+  XNN_REQUIRE(n_nodes <= (int64_t(1) << 21) && tiles->n_tiles < (int64_t(1) << 31),
+              "too many tiles");
+  XNN_REQUIRE(work_bytes >= need, "workspace too small: %zu < %zu", work_bytes, need);
+  hipStream_t s = as_hip(stream);
+  const int64_t nt = (n_nodes + kStoreTile - 1) / kStoreTile;
+  double* part = static_cast<double*>(work);
+  const auto go = [&](auto apply, auto sum) {
+    hipLaunchKernelGGL(apply, dim3((unsigned)tiles->n_tiles), dim3(256), 0, s, values,
+                       tiles->tile_ij, tiles->mask, tiles->off, tiles->base, n_nodes, v, part);
+    hipLaunchKernelGGL(sum, dim3((unsigned)nt), dim3(1024), 0, s, part, tiles->index, n_nodes, nt,
+                       out);
+  };
+  if (nrhs == 1) go(eeq_tiles_apply_kernel<1>, eeq_tiles_sum_kernel<1>);
+  else go(eeq_tiles_apply_kernel<2>, eeq_tiles_sum_kernel<2>);
   XNN_LAUNCH_CHECK();
   return XNN_OK;
 }

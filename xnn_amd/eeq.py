@@ -48,6 +48,11 @@ TABLE_BUDGET = 1 << 28
 #: (N, G) entries per block of the differentiable reciprocal sum (recomputed in the
 #: backward)
 LIVE_BUDGET = 1 << 23
+#: bytes of real-space values the conjugate-gradient regime keeps (8.2 B per unordered pair
+#: in reach: 1.3 GB at 24,000 atoms and 60 bohr); beyond it, or when the device has not that
+#: much left, every product evaluates its pairs again
+STORE_BYTES = 32 << 30
+STORE_TILE = 128
 #: reciprocal vectors (smallest |G|, largest weights) in the low-rank part of the
 #: conjugate-gradient preconditioner (dispersion_fast/eeq.py:60-66); 0 for plain Jacobi
 LOW_K_VECTORS = 256
@@ -173,6 +178,70 @@ def real_apply(pos: Tensor, cell, rad: Tensor, alpha: float, cutoff_au: float,
               float(alpha), float(cutoff_au), _lib.ptr(tiles), _lib.ptr(vv), r, _lib.ptr(out),
               _lib.ptr(work), int(work.numel()), _lib.stream(pos.device))
     return out
+
+
+class RealTiles:
+    """The real-space matrix of ``N`` spatially ordered atoms, evaluated once: of the lower
+    128 x 128 tiles the pairs with an image within the cutoff (``xnn_eeq_store_tiles``)."""
+
+    def __init__(self, keep: Tuple[Tensor, ...], tiles: "_lib.EeqTiles", values: Tensor):
+        self._keep, self.tiles, self.values = keep, tiles, values
+
+    @classmethod
+    def build(cls, pos: Tensor, host_cell, rad: Tensor, alpha: float,
+              cutoff_au: float) -> Optional["RealTiles"]:
+        """None where the values exceed :data:`STORE_BYTES` or do not fit the device."""
+        n, dev = int(pos.shape[0]), pos.device
+        nt = -(-n // STORE_TILE)
+        if n == 0 or nt * nt > 1 << 26:
+            return None
+        stream = _lib.stream(dev)
+        bounds = None if host_cell is None else tile_bounds(pos, STORE_TILE)
+        flags = torch.empty(nt * nt, dtype=torch.int32, device=dev)
+        _lib.call("xnn_eeq_store_meet", _lib.ptr(bounds), n, host_cell, float(cutoff_au),
+                  _lib.ptr(flags), stream)
+        at = flags.nonzero()[:, 0]
+        m = int(at.shape[0])
+        if m == 0:
+            return None
+        try:
+            ij = torch.stack([at // nt, at % nt], 1).to(torch.int32).contiguous()
+            index = torch.full((nt * nt,), -1, dtype=torch.int32, device=dev)
+            index[at] = torch.arange(m, dtype=torch.int32, device=dev)
+            mask = torch.empty(m * 2 * STORE_TILE, dtype=torch.int64, device=dev)
+            off = torch.empty(m * 2 * STORE_TILE, dtype=torch.int32, device=dev)
+            counts = torch.empty(m, dtype=torch.int64, device=dev)
+            tiles = _lib.EeqTiles(m, _lib.ptr(ij), _lib.ptr(index), _lib.ptr(mask), _lib.ptr(off), None)
+
+            def step(c, v):
+                _lib.call("xnn_eeq_store_tiles", _lib.ptr(pos), n, host_cell, _lib.ptr(rad),
+                          float(alpha), float(cutoff_au), ctypes.byref(tiles), _lib.ptr(c),
+                          _lib.ptr(v), stream)
+
+            step(counts, None)
+            end = torch.cumsum(counts, 0)
+            base = end - counts
+            total = int(end[-1])
+            if total * 8 > STORE_BYTES:
+                return None
+            values = torch.empty(max(total, 1), dtype=torch.float64, device=dev)
+        except torch.cuda.OutOfMemoryError:
+            return None
+        tiles.base = _lib.ptr(base)
+        step(None, values)
+        return cls((ij, index, mask, off, base), tiles, values)
+
+    def apply(self, v: Tensor) -> Tensor:
+        """``R v`` for ``v`` (N, 1 or 2)."""
+        n, r = int(v.shape[0]), int(v.shape[1])
+        out = torch.empty((n, r), dtype=torch.float64, device=v.device)
+        need = ctypes.c_size_t(0)
+        _lib.call("xnn_eeq_store_apply_work_size", self.tiles.n_tiles, r, ctypes.byref(need))
+        work = torch.empty(need.value, dtype=torch.uint8, device=v.device)
+        _lib.call("xnn_eeq_store_apply", _lib.ptr(self.values), ctypes.byref(self.tiles), n,
+                  _lib.ptr(v.contiguous()), r, _lib.ptr(out), _lib.ptr(work), int(work.numel()),
+                  _lib.stream(v.device))
+        return out
 
 
 @torch.library.custom_op(f"{_NS}::eeq_real_apply", mutates_args=())
@@ -431,13 +500,14 @@ class FactorizedReciprocal:
 
 
 class IterativeEEQSystem:
-    """The EEQ operator of one structure at fixed (detached) geometry, never assembled: the
+    """The EEQ operator of one structure at fixed (detached) geometry: the
     conjugate-gradient regime above :data:`LU_MAX_ATOMS` (eeq.py:226, 325-360;
-    dispersion_fast/eeq.py:1-33). A product is ``diag v`` plus the matrix-free real-space
-    product (``xnn_eeq_real_apply``, HIP, atoms ordered along a Morton curve of the wrapped
-    fractional coordinates so that 256-atom tiles are compact and far tiles are skipped)
-    plus the factorized reciprocal product (:class:`FactorizedReciprocal`). Memory O(N) in
-    the real-space part and O(N C) in the reciprocal tables. Solves: preconditioned
+    dispersion_fast/eeq.py:1-33). A product is ``diag v`` plus the real-space
+    product (atoms ordered along a Morton curve of the wrapped fractional coordinates, so
+    that tiles are compact and far tiles are left out) plus the factorized reciprocal
+    product (:class:`FactorizedReciprocal`). The real-space pairs are evaluated once into
+    tiles (:class:`RealTiles`) up to :data:`STORE_BYTES`; beyond that at every product
+    (``xnn_eeq_real_apply``, memory O(N)). Solves: preconditioned
     conjugate gradients, the preconditioner the full diagonal (``J + sqrt(2/pi)/a - 2
     alpha/sqrt(pi)``, the own images and ``sum_G w_G``) with the long-range modes of the
     smallest reciprocal vectors as a low-rank part (:meth:`_low_rank`; Jacobi for a
@@ -480,6 +550,8 @@ class IterativeEEQSystem:
             self.inv_d = (1.0 / full[self.order]).contiguous()
         self.y_ones = None
         self.iterations = []                   # per conjugate-gradient solve
+        self.store = (RealTiles.build(self.pos_s, self.cell_host, self.rad_s, self.alpha, self.cutoff)
+                      if self.pos_s.is_cuda else None)
         self._work = None
 
     def _low_rank(self, full_s: Tensor) -> None:
@@ -512,12 +584,15 @@ class IterativeEEQSystem:
 
     def _matvec(self, v: Tensor) -> Tensor:
         """``A v`` in the spatial order, ``v`` (N, 1 or 2)."""
-        need = ctypes.c_size_t(0)
-        _lib.call("xnn_eeq_real_apply_work_size", self.n, int(v.shape[1]), ctypes.byref(need))
-        if self._work is None or self._work.numel() < need.value:
-            self._work = torch.empty(need.value, dtype=torch.uint8, device=v.device)
-        out = real_apply(self.pos_s, self.cell_host, self.rad_s, self.alpha, self.cutoff, v,
-                         self.tiles, self._work)
+        if self.store is not None:
+            out = self.store.apply(v)
+        else:
+            need = ctypes.c_size_t(0)
+            _lib.call("xnn_eeq_real_apply_work_size", self.n, int(v.shape[1]), ctypes.byref(need))
+            if self._work is None or self._work.numel() < need.value:
+                self._work = torch.empty(need.value, dtype=torch.uint8, device=v.device)
+            out = real_apply(self.pos_s, self.cell_host, self.rad_s, self.alpha, self.cutoff, v,
+                             self.tiles, self._work)
         out += self.diag_s[:, None] * v
         if self.recip is not None:
             out += self.recip.apply(v)
