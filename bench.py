@@ -679,11 +679,11 @@ def cpu_baseline_d3(s, tables, w: np.ndarray, model, k: int = 200,
                       f"PyTorch-CPU float64, torch threads={torch.get_num_threads()}"}
 
 
-# D3 (BJ) algorithmic float64 flops per launch: per pair-image term as D4 (60 energy, +35
-# for the backward); per atom pair C6 = W_i . C6ref . W_j (56 FMA = 112) and, backward,
-# both atoms' dC6/dW (2 x 112)
-D3_FLOPS = {"xnn_d3_two_body": lambda M, P: 60 * M + 112 * P,
-            "xnn_d3_two_body_backward": lambda M, P: 95 * M + 336 * P}
+# D3 (BJ) algorithmic float64 flops per launch over the unordered sums (M directed pair-image
+# terms, P atom pairs), per term as D4; per atom pair C6 = W_i . v_j (14) with the damping
+# radius and the sums (16), backward the forces and cell moment (51) and both atoms' dE/dW (31)
+D3_FLOPS = {"xnn_d3_two_body_tiles": lambda M, P: 29 * M // 2 + 30 * P,
+            "xnn_d3_two_body_tiles_backward": lambda M, P: 57 * M // 2 + 96 * P}
 
 
 def bench_d3(steps: int, warmup: int, cpu: bool = True) -> dict:
@@ -717,7 +717,8 @@ def bench_d3(steps: int, warmup: int, cpu: bool = True) -> dict:
         out, gp, gc = step()
     torch.cuda.synchronize()
     ms = (time.perf_counter() - t0) / steps * 1e3
-    kernels = list(D3_FLOPS) + ["xnn_d3_coordination", "xnn_d3_coordination_backward"]
+    kernels = list(D3_FLOPS) + ["xnn_d3_coordination_planned",
+                                "xnn_d3_coordination_backward_planned"]
     _lib.timed.clear()
     _lib.time_launches(*kernels)
     for _ in range(steps):

@@ -724,6 +724,21 @@ int xnn_d3_coordination_backward(const double* pos, int64_t n_nodes, const int32
                                  const double* g_cn, double* grad_pos, double* cell_partial,
                                  void* workspace, size_t workspace_bytes, xnn_stream_t stream);
 
+/* The same with a tile plan of xnn_d4_plan for these positions (NULL: built in the call,
+ * as the two entry points above do). */
+int xnn_d3_coordination_planned(const double* pos, int64_t n_nodes, const int32_t* species,
+                                const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                                int64_t max_atoms, const double* cell, const int32_t* images,
+                                const int32_t* plan, const double* rcov, double cutoff_cn,
+                                double kcn, double* cn, void* workspace, size_t workspace_bytes,
+                                xnn_stream_t stream);
+int xnn_d3_coordination_backward_planned(
+    const double* pos, int64_t n_nodes, const int32_t* species, const int32_t* batch,
+    const int64_t* node_ptr, int64_t n_graphs, int64_t max_atoms, const double* cell,
+    const int32_t* images, const int32_t* plan, const double* rcov, double cutoff_cn, double kcn,
+    const double* g_cn, double* grad_pos, double* cell_partial, void* workspace,
+    size_t workspace_bytes, xnn_stream_t stream);
+
 typedef struct {
   double s6, s8, a1, a2;   /* scalings; rational-damping radius a1 sqrt(C8/C6) + a2   */
   double rs6, rs8, alp;    /* zero damping: radii scalings and exponent              */
@@ -754,6 +769,25 @@ int xnn_d3_two_body_backward(const double* pos, int64_t n_nodes, const int32_t* 
                              const xnn_d3_pair_params* prm, const double* g_e2, double* grad_pos,
                              double* cell_partial, double* grad_weights, void* workspace,
                              size_t workspace_bytes, xnn_stream_t stream);
+
+/* xnn_d3_two_body(_backward) with the rational damping over the tiles of xnn_d4_plan (plan
+ * nullable), every unordered pair once: for at most 16 species and a c6ref symmetric under
+ * the exchange of its atoms, c6ref[s][t][a][b] = c6ref[t][s][b][a] (the caller's to check).
+ * Workspace: xnn_d4_workspace_bytes. */
+int xnn_d3_two_body_tiles(const double* pos, int64_t n_nodes, const int32_t* species,
+                          const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                          int64_t max_atoms, const double* cell, const int32_t* images,
+                          const int32_t* plan, const double* r4r2, const double* c6ref,
+                          int32_t n_species, const double* weights, const xnn_d3_pair_params* prm,
+                          double* e2, void* workspace, size_t workspace_bytes,
+                          xnn_stream_t stream);
+int xnn_d3_two_body_tiles_backward(
+    const double* pos, int64_t n_nodes, const int32_t* species, const int32_t* batch,
+    const int64_t* node_ptr, int64_t n_graphs, int64_t max_atoms, const double* cell,
+    const int32_t* images, const int32_t* plan, const double* r4r2, const double* c6ref,
+    int32_t n_species, const double* weights, const xnn_d3_pair_params* prm, const double* g_e2,
+    double* grad_pos, double* cell_partial, double* grad_weights, void* workspace,
+    size_t workspace_bytes, xnn_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Cell-list radius graph. Replaces build_neighbor_list (neighborlist.py:411-506):

@@ -186,6 +186,14 @@ _SIGNATURES = {
                                          vp, vp],
     "xnn_d4_two_body_backward": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, vp,
                                  ctypes.POINTER(D4PairParams), vp, vp, vp, vp, vp, sz, vp],
+    "xnn_d3_coordination_planned": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, dbl, dbl, vp, vp,
+                                    sz, vp],
+    "xnn_d3_coordination_backward_planned": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, dbl, dbl,
+                                             vp, vp, vp, vp, sz, vp],
+    "xnn_d3_two_body_tiles": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, vp, i32, vp,
+                              ctypes.POINTER(D3PairParams), vp, vp, sz, vp],
+    "xnn_d3_two_body_tiles_backward": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, vp, vp, i32, vp,
+                                       ctypes.POINTER(D3PairParams), vp, vp, vp, vp, vp, sz, vp],
     "xnn_d3_coordination": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, dbl, dbl, vp, vp, sz, vp],
     "xnn_d3_coordination_backward": [vp, i64, vp, vp, vp, i64, i64, vp, vp, vp, dbl, dbl, vp, vp,
                                      vp, vp, sz, vp],

@@ -1,9 +1,7 @@
-// D3 dispersion pair terms on lattice images and the D4 polarizabilities (gfx950, wave64,
-// float64). The D4 coordination numbers and two-body term walk spatially ordered tiles
-// (d4_tiles.hip).
+// D3 two-body term on lattice images in its general form and the D4 polarizabilities
+// (gfx950, wave64, float64). The coordination numbers, the D4 two-body term and the D3 one
+// with the rational damping walk spatially ordered tiles (d4_tiles.hip).
 //
-// xnn_d3_coordination(_backward)  DFTD3.coordination_numbers (d3.py:632-642), the
-//                                 exponential count
 // xnn_d3_two_body(_backward)      DFTD3.pair_c6 / two_body_energy (d3.py:651-722): C6
 //                                 from per-atom reference weights and the species-pair
 //                                 reference block, bj / zero / mzero / op damping
@@ -62,104 +60,6 @@ struct D4Stage {
   int sp[kD4Sub];         // species
   int b[kD4Sub];          // structure
 };
-
-// ---------------------------------------------------------------- D3 coordination numbers
-// The exponential count 1 / (1 + exp(-k1 (rc / r - 1))) within cut_cn (d3.py:632-642).
-// BACKWARD = false: partial[cy][0][i] = the count of this chunk (np = 2, component 1 unused).
-// BACKWARD = true:  partial[cy][0..11][i] = grad_pos (3), cell gradient n (x) g (9).
-template <bool BACKWARD>
-__global__ __launch_bounds__(64, 3) void d3_cn_kernel(
-    const double* __restrict__ pos, int64_t n_nodes, const int32_t* __restrict__ species,
-    const int32_t* __restrict__ batch, const int64_t* __restrict__ node_ptr,
-    const double* __restrict__ cell, const int32_t* __restrict__ images,
-    const double* __restrict__ rcov, CnParams prm, const double* __restrict__ g_cn,
-    int64_t chunk, int64_t n_cy, double* __restrict__ partial) {
-  __shared__ D4Stage st;
-  const int lane = threadIdx.x;
-  const int64_t t = blockIdx.x, cy = blockIdx.y;
-  const int64_t i = t * kD4Tile + lane;
-  const bool live = i < n_nodes;
-  // source range of the tile's structures, in chunks
-  const int64_t i_first = t * kD4Tile, i_last = std::min<int64_t>(i_first + kD4Tile, n_nodes) - 1;
-  const int64_t s_lo = node_ptr[batch[i_first]], s_hi = node_ptr[batch[i_last] + 1];
-  const int64_t c = s_lo / chunk + cy;
-  const int64_t j0 = std::max<int64_t>(c * chunk, s_lo), j1 = std::min<int64_t>((c + 1) * chunk, s_hi);
-  constexpr int NP = BACKWARD ? 12 : 2;
-  double acc[NP];
-#pragma unroll
-  for (int k = 0; k < NP; ++k) acc[k] = 0.0;
-  double xi = 0, yi = 0, zi = 0, rci = 0, gi = 0;
-  int bi = -1;
-  Lattice L;
-  if (live) {
-    xi = pos[3 * i];
-    yi = pos[3 * i + 1];
-    zi = pos[3 * i + 2];
-    rci = rcov[species[i]];
-    bi = batch[i];
-    if (BACKWARD) gi = g_cn[i];
-    load_lattice(cell, images, bi, L);
-  } else {
-    load_lattice(nullptr, nullptr, 0, L);
-  }
-  const double cmax = prm.cut_cn;
-  for (int64_t base = j0; base < j1; base += kD4Sub) {
-    const int cnt = (int)std::min<int64_t>(kD4Sub, j1 - base);
-    __syncthreads();
-    if (lane < cnt) {
-      const int64_t j = base + lane;
-      st.x[lane] = pos[3 * j];
-      st.y[lane] = pos[3 * j + 1];
-      st.z[lane] = pos[3 * j + 2];
-      st.b[lane] = batch[j];
-      st.p[lane] = rcov[species[j]];
-      if (BACKWARD) st.w[lane] = g_cn[j];
-    }
-    __syncthreads();
-    if (!live) continue;
-    for (int jj = 0; jj < cnt; ++jj) {
-      if (st.b[jj] != bi) continue;
-      const double rc = rci + st.p[jj];
-      const double dx = xi - st.x[jj], dy = yi - st.y[jj], dz = zi - st.z[jj];
-      const double bx = dx * kInvBohr, by = dy * kInvBohr, bz = dz * kInvBohr;
-      const double wsum = BACKWARD ? gi + st.w[jj] : 0.0;
-      const ImageRange win = image_window(L, dx, dy, dz, cmax * kBohr);
-      for (int n0 = win.lo0; n0 <= win.hi0; ++n0)
-        for (int n1 = win.lo1; n1 <= win.hi1; ++n1) {
-          // the image's vector in bohr, d + n @ cell
-          const double px = bx + n0 * L.ab[0] + n1 * L.ab[3];
-          const double py = by + n0 * L.ab[1] + n1 * L.ab[4];
-          const double pz = bz + n0 * L.ab[2] + n1 * L.ab[5];
-          for (int n2 = win.lo2; n2 <= win.hi2; ++n2) {
-            const double vx = px + n2 * L.ab[6], vy = py + n2 * L.ab[7], vz = pz + n2 * L.ab[8];
-            const double r2 = vx * vx + vy * vy + vz * vz;
-            if (r2 <= 0.0 || r2 > cmax * cmax) continue;
-            const double rinv = rsq_nr(r2);
-            // d/dr of the count = -s (1 - s) k1 rc / r^2
-            const double sg = rcp_nr(1.0 + exp(-prm.kcn * (rc * rinv - 1.0)));
-            if (!BACKWARD) {
-              acc[0] += sg;
-            } else {
-              const double dcount = -sg * (1.0 - sg) * prm.kcn * rc * rinv * rinv;
-              // per Angstrom of the edge vector: d r_bohr / d v = v_bohr / (r bohr)
-              const double s = dcount * rinv * kInvBohr;
-              acc[0] += wsum * s * vx;
-              acc[1] += wsum * s * vy;
-              acc[2] += wsum * s * vz;
-              const double ox = gi * s * vx, oy = gi * s * vy, oz = gi * s * vz;
-              acc[3] += n0 * ox; acc[4] += n0 * oy; acc[5] += n0 * oz;
-              acc[6] += n1 * ox; acc[7] += n1 * oy; acc[8] += n1 * oz;
-              acc[9] += n2 * ox; acc[10] += n2 * oy; acc[11] += n2 * oz;
-            }
-          }
-        }
-    }
-  }
-  if (live) {
-#pragma unroll
-    for (int k = 0; k < NP; ++k) partial[((int64_t)cy * NP + k) * n_nodes + i] = acc[k];
-  }
-}
 
 // ---------------------------------------------------------------- D3 two-body term
 constexpr int kNR = 7;  // D3 reference systems per element
@@ -677,60 +577,6 @@ size_t xnn_d4_workspace_bytes(int64_t n_nodes, int64_t n_graphs, int64_t max_ato
   // slot; the D4 tile kernels: their own layout
   const size_t d3 = (size_t)(w.n_cy * (12 + kNR) * n_nodes) * sizeof(double);
   return std::max(d3, d4_tiles_workspace_bytes(n_nodes, n_graphs, max_atoms));
-}
-
-int xnn_d3_coordination(const double* pos, int64_t n_nodes, const int32_t* species,
-                        const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
-                        int64_t max_atoms, const double* cell, const int32_t* images,
-                        const double* rcov, double cutoff_cn, double kcn, double* cn,
-                        void* workspace, size_t workspace_bytes, xnn_stream_t stream) {
-  const int st = d4_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images, max_atoms);
-  if (st != XNN_OK) return st;
-  XNN_REQUIRE(rcov != nullptr, "NULL rcov");
-  XNN_REQUIRE(n_nodes == 0 || cn, "NULL output");
-  if (n_nodes == 0) return XNN_OK;
-  const D4Work w = d4_work(n_nodes, n_graphs, max_atoms);
-  const size_t need = (size_t)(w.n_cy * 2 * n_nodes) * sizeof(double);
-  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need, "workspace too small (%zu < %zu)",
-              workspace_bytes, need);
-  const CnParams p{cutoff_cn, 0.0, kcn, 0.0, 0.0, 1.0};
-  hipStream_t s = as_hip(stream);
-  double* part = static_cast<double*>(workspace);
-  hipLaunchKernelGGL(d3_cn_kernel<false>, dim3((unsigned)w.n_tiles, (unsigned)w.n_cy),
-                     dim3(kD4Tile), 0, s, pos, n_nodes, species, batch, node_ptr, cell, images,
-                     rcov, p, nullptr, w.chunk, w.n_cy, part);
-  XNN_LAUNCH_CHECK();
-  reduce_into(part, n_nodes, 2, 0, 1, w.n_cy, cn, s);
-  XNN_LAUNCH_CHECK();
-  return XNN_OK;
-}
-
-int xnn_d3_coordination_backward(const double* pos, int64_t n_nodes, const int32_t* species,
-                                 const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
-                                 int64_t max_atoms, const double* cell, const int32_t* images,
-                                 const double* rcov, double cutoff_cn, double kcn,
-                                 const double* g_cn, double* grad_pos, double* cell_partial,
-                                 void* workspace, size_t workspace_bytes, xnn_stream_t stream) {
-  const int st = d4_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images, max_atoms);
-  if (st != XNN_OK) return st;
-  XNN_REQUIRE(rcov != nullptr, "NULL rcov");
-  XNN_REQUIRE(n_nodes == 0 || (grad_pos && g_cn), "NULL g_cn or grad_pos");
-  if (n_nodes == 0) return XNN_OK;
-  const D4Work w = d4_work(n_nodes, n_graphs, max_atoms);
-  const size_t need = (size_t)(w.n_cy * 12 * n_nodes) * sizeof(double);
-  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need, "workspace too small (%zu < %zu)",
-              workspace_bytes, need);
-  const CnParams p{cutoff_cn, 0.0, kcn, 0.0, 0.0, 1.0};
-  hipStream_t s = as_hip(stream);
-  double* part = static_cast<double*>(workspace);
-  hipLaunchKernelGGL(d3_cn_kernel<true>, dim3((unsigned)w.n_tiles, (unsigned)w.n_cy),
-                     dim3(kD4Tile), 0, s, pos, n_nodes, species, batch, node_ptr, cell, images,
-                     rcov, p, g_cn, w.chunk, w.n_cy, part);
-  XNN_LAUNCH_CHECK();
-  reduce_into(part, n_nodes, 12, 0, 3, w.n_cy, grad_pos, s);
-  reduce_into(part, n_nodes, 12, 3, 9, w.n_cy, cell_partial, s);
-  XNN_LAUNCH_CHECK();
-  return XNN_OK;
 }
 
 static int d3_pair_check(const xnn_d3_pair_params* prm, const double* r4r2, const double* rvdw,

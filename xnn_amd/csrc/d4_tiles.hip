@@ -10,6 +10,10 @@
 //                                 pair image; the backward gives grad_pos, the cell gradient
 //                                 and dE/d alpha, the quantities of the reference's native
 //                                 kernel run_d4 (dispersion_fast/cpu.py:834-935)
+// xnn_d3_coordination(_backward), xnn_d3_two_body_tiles(_backward)
+//                                 DFTD3.coordination_numbers (d3.py:632-642) and, with the
+//                                 rational damping, pair_c6 / two_body_energy (d3.py:651-722)
+//                                 on the same tiles
 //
 // Layout. A call first orders the atoms of every structure along a Morton curve of a bin
 // grid over their coordinates (fractional ones for a periodic structure), so that 64
@@ -48,6 +52,17 @@ constexpr int kOrderThreads = 1024;    // one workgroup orders one structure
 constexpr int kOrderBits = 4;          // at most 16 bins per axis
 constexpr int kOrderBins = 1 << (3 * kOrderBits);
 constexpr int kRedWaves = 8;           // waves of a slot-reduction block
+constexpr int kNR = 7;                 // D3 reference systems per element
+constexpr int kD3MaxSpecies = 16;      // species of the D3 tiles' source rows
+
+// what the D3 pair tiles read in place of the polarizabilities: the reference weights (N, 7)
+// and each atom's rows v_j[s][a] = sum_b C6ref[s][s_j][a][b] W_j[b] (N, S, 7), so that
+// C6_ij = sum_a W_i[a] v_j[s_i][a] (d3.py:651-674)
+struct D3Rows {
+  const double* weights;
+  const double* rows;
+  int n_species;
+};
 
 __constant__ double c_cp3[kNW] = {
     cp3_weight(0),  cp3_weight(1),  cp3_weight(2),  cp3_weight(3),  cp3_weight(4),
@@ -561,6 +576,44 @@ __device__ __forceinline__ void pair_alpha_products(
   }
 }
 
+// D3: dE/dW of both atoms from the same sums, dE/dW_i[a] = sum_j K_ij v_j[s_i][a] (C6ref is
+// symmetric under the exchange of its atoms): seven values an atom against rows picked by
+// the atom's species, so a lane per output atom on the vector ALU; the waves take a side
+// each.
+template <bool DIAG, int W>
+__device__ __forceinline__ void pair_weight_sums(
+    const PairStage<true, W>& st, const TileItem& it, const D3Rows& D,
+    const int32_t* __restrict__ species, int64_t n_nodes, const double* __restrict__ fb,
+    double* __restrict__ partial_w) {
+  __syncthreads();  // the block's rows, written by every lane, read across lanes and waves
+  const int lane = threadIdx.x % kT, wv = wave_in_block();
+  for (int side = wv; side < (DIAG ? 1 : 2); side += W) {
+    const int out_cnt = side == 0 ? it.rcnt : it.scnt;
+    const int b_cnt = side == 0 ? it.scnt : it.rcnt;
+    const int so = species[st.id[side][lane]];
+    const double g_out = side == 0 ? st.gr[lane] : st.w[lane];
+    double dw[kNR];
+#pragma unroll
+    for (int a = 0; a < kNR; ++a) dw[a] = 0.0;
+#pragma unroll 4
+    for (int kk = 0; kk < b_cnt; ++kk) {
+      const int j = __builtin_amdgcn_readfirstlane(st.id[1 - side][kk]);
+      const double g = g_out + (side == 0 ? st.w[kk] : st.gr[kk]);
+      const double K = -0.5 * g * fb[side == 0 ? kk * kT + lane : lane * kT + kk];
+      const double* __restrict__ row = D.rows + ((int64_t)j * D.n_species + so) * kNR;
+#pragma unroll
+      for (int a = 0; a < kNR; ++a) dw[a] += K * row[a];
+    }
+    const int slot = side == 0 ? it.ls : it.lt;
+    double* __restrict__ pw =
+        partial_w + (int64_t)slot * kNR * n_nodes + (side == 0 ? it.r0 : it.s0);
+    if (lane < out_cnt) {
+#pragma unroll
+      for (int a = 0; a < kNR; ++a) pw[(int64_t)a * n_nodes + lane] = dw[a];
+    }
+  }
+}
+
 // BACKWARD = false: partial[slot][0][p] = the atom's sum of -1/2 C6 f(r).
 // BACKWARD = true:  partial[slot][0..2][p] = grad_pos, [3..11] the cell gradient (CELL),
 //                   partial_alpha[slot][w][p] = dE/d alpha(i w); fsum_out[jj][lane] (this
@@ -571,13 +624,14 @@ __device__ __forceinline__ void pair_alpha_products(
 //                   and reads back one source at a time, just before that source's row takes
 //                   the image sum: no alpha table in LDS and no 23 alpha registers in the
 //                   loop, so three waves fit on a SIMD.
-template <bool BACKWARD, bool CELL, bool DIAG, int W>
+// D3: C6 from the reference weights (D), dE/dW in partial_alpha (7 components).
+template <bool BACKWARD, bool CELL, bool DIAG, int W, bool D3>
 __device__ __forceinline__ void pair_tile(
     PairStage<BACKWARD, W>& st, const TileItem& it, const TileGeo& G, const PairParams& prm,
     const double* __restrict__ pos, const int32_t* __restrict__ species,
     const double* __restrict__ r4r2, const double* __restrict__ alpha,
-    const double* __restrict__ g_e2, const int32_t* __restrict__ order, int64_t n_nodes,
-    double* __restrict__ partial, double* __restrict__ fsum_out,
+    const D3Rows& D, const double* __restrict__ g_e2, const int32_t* __restrict__ order,
+    int64_t n_nodes, double* __restrict__ partial, double* __restrict__ fsum_out,
     double* __restrict__ partial_alpha) {
   constexpr int NV = BACKWARD ? 3 : 1;
   constexpr int NP = BACKWARD ? (CELL ? 12 : 3) : 1;
@@ -590,12 +644,25 @@ __device__ __forceinline__ void pair_tile(
   const int i = order[pi];
   const double xa = pos[3 * (int64_t)i], ya = pos[3 * (int64_t)i + 1], za = pos[3 * (int64_t)i + 2];
   const double xb = xa * kInvBohr, yb = ya * kInvBohr, zb = za * kInvBohr;
-  const double qi = r4r2[species[i]], sq3qi = sqrt(3.0 * qi);
+  const int si = species[i];
+  const double qi = r4r2[si], sq3qi = sqrt(3.0 * qi);
   const double gi = BACKWARD ? g_e2[i] : 0.0;
-  double ai[kNW];
+  constexpr int NA = D3 ? kNR : kNW;  // the receiver's weights or polarizabilities
+  double ai[NA];
 #pragma unroll
-  for (int w = 0; w < kNW; ++w) ai[w] = alpha[(int64_t)kNW * i + w];
-  if constexpr (BACKWARD) {
+  for (int w = 0; w < NA; ++w) ai[w] = (D3 ? D.weights : alpha)[(int64_t)NA * i + w];
+  const auto d3_c6 = [&](int j) {
+    const double* __restrict__ row = D.rows + ((int64_t)j * D.n_species + si) * kNR;
+    double c = 0.0;
+#pragma unroll
+    for (int a = 0; a < kNR; ++a) c += ai[a] * row[a];
+    return c;
+  };
+  if constexpr (BACKWARD && D3) {
+#pragma unroll 4
+    for (int jj = j_lo; jj < j_end; ++jj)
+      fsum_out[jj * kT + lane] = d3_c6(__builtin_amdgcn_readfirstlane(order[it.s0 + jj]));
+  } else if constexpr (BACKWARD) {
     // C6 of this lane's pair with each of the wave's sources, into the block's rows; the
     // source's alpha is wave-uniform (scalar loads)
     for (int jj = j_lo; jj < j_end; ++jj) {
@@ -622,6 +689,8 @@ __device__ __forceinline__ void pair_tile(
     if constexpr (BACKWARD) {
       st.w[lane] = g_e2[j];
       st.id[1][lane] = j;
+    } else if constexpr (D3) {
+      st.id[0][lane] = j;
     } else {
 #pragma unroll
       for (int w = 0; w < kNW; ++w) st.sa[lane][w] = alpha[(int64_t)kNW * j + w] * c_cp3[w];
@@ -670,6 +739,8 @@ __device__ __forceinline__ void pair_tile(
       double c6;
       if constexpr (BACKWARD) {
         c6 = fsum_out[jj * kT + lane];
+      } else if constexpr (D3) {
+        c6 = d3_c6(__builtin_amdgcn_readfirstlane(st.id[0][jj]));
       } else {
         // four partial sums: four short dependency chains instead of one of 23
         double c6p[4] = {0.0, 0.0, 0.0, 0.0};
@@ -807,18 +878,20 @@ __device__ __forceinline__ void pair_tile(
         }
     }
   }
-  if constexpr (BACKWARD) pair_alpha_products<DIAG, W>(st, it, alpha, n_nodes, fsum_out,
-                                                        partial_alpha);
+  if constexpr (BACKWARD && D3)
+    pair_weight_sums<DIAG, W>(st, it, D, species, n_nodes, fsum_out, partial_alpha);
+  else if constexpr (BACKWARD)
+    pair_alpha_products<DIAG, W>(st, it, alpha, n_nodes, fsum_out, partial_alpha);
 }
 
 // The energy kernel (64, 2): at most 256 registers, two waves per SIMD (18 KB of LDS). The
 // backward (64 W, 3): at most 168 registers, three waves per SIMD.
-template <bool BACKWARD, bool CELL, int W>
+template <bool BACKWARD, bool CELL, int W, bool D3>
 __global__ __launch_bounds__(kT * W, BACKWARD ? 3 : 2) void d4_pair_tiles_kernel(
     const double* __restrict__ pos, const int32_t* __restrict__ species,
     const int64_t* __restrict__ node_ptr, int64_t n_graphs, const double* __restrict__ cell,
     const int32_t* __restrict__ images, const double* __restrict__ r4r2,
-    const double* __restrict__ alpha, PairParams prm, const double* __restrict__ g_e2,
+    const double* __restrict__ alpha, D3Rows D, PairParams prm, const double* __restrict__ g_e2,
     const int32_t* __restrict__ order, const int32_t* __restrict__ tile_ptr, int64_t n_nodes,
     int max_nt, double* __restrict__ partial, double* __restrict__ fsum,
     double* __restrict__ partial_alpha) {
@@ -829,11 +902,11 @@ __global__ __launch_bounds__(kT * W, BACKWARD ? 3 : 2) void d4_pair_tiles_kernel
   tile_geo(cell, images, it.b, prm.cutoff * kBohr, G);
   double* fb = BACKWARD ? fsum + ((int64_t)blockIdx.x * max_nt + blockIdx.y) * (kT * kT) : nullptr;
   if (it.ls == it.lt)
-    pair_tile<BACKWARD, CELL, true, W>(st, it, G, prm, pos, species, r4r2, alpha, g_e2, order,
-                                       n_nodes, partial, fb, partial_alpha);
+    pair_tile<BACKWARD, CELL, true, W, D3>(st, it, G, prm, pos, species, r4r2, alpha, D, g_e2,
+                                           order, n_nodes, partial, fb, partial_alpha);
   else
-    pair_tile<BACKWARD, CELL, false, W>(st, it, G, prm, pos, species, r4r2, alpha, g_e2, order,
-                                        n_nodes, partial, fb, partial_alpha);
+    pair_tile<BACKWARD, CELL, false, W, D3>(st, it, G, prm, pos, species, r4r2, alpha, D, g_e2,
+                                            order, n_nodes, partial, fb, partial_alpha);
 }
 
 // ---------------------------------------------------------------- coordination numbers
@@ -855,15 +928,21 @@ struct CnStage {
 
 // BACKWARD = false: partial[slot][0/1][p] = (cn_d4, cn_raw) sums.
 // BACKWARD = true:  partial[slot][0..2][p] = grad_pos, [3..11] the cell gradient (CELL).
-template <bool BACKWARD, bool CELL, bool DIAG, int W>
+// D3: the exponential count 1 / (1 + exp(-k1 (rc / r - 1))) within cut_cn in cn_d4's place (one
+// component), no electronegativities; it does not vanish before the cutoff. Bound by the
+// float64 vector ALU; 5,000 atoms at 40 bohr: 325 -> 123 us, backward 412 -> 167 us against
+// walking the directed pairs (each pair image evaluated once instead of twice, images no
+// receiver of the tile reaches left out by the whole wave).
+template <bool BACKWARD, bool CELL, bool DIAG, int W, bool D3>
 __device__ __forceinline__ void cn_tile(
     CnStage<W>& st, const TileItem& it, const TileGeo& G, const CnParams& prm,
     const double* __restrict__ pos, const int32_t* __restrict__ species,
     const double* __restrict__ rcov, const double* __restrict__ en,
     const double* __restrict__ g_cn, const double* __restrict__ g_raw,
     const int32_t* __restrict__ order, int64_t n_nodes, double* __restrict__ partial) {
-  constexpr int NV = BACKWARD ? 3 : 2;
-  constexpr int NP = BACKWARD ? (CELL ? 12 : 3) : 2;
+  constexpr int NF = D3 ? 1 : 2;  // counts of the forward
+  constexpr int NV = BACKWARD ? 3 : NF;
+  constexpr int NP = BACKWARD ? (CELL ? 12 : 3) : NF;
   constexpr int S = kT / W;  // sources of a wave
   static_assert(S % 8 == 0, "whole 8-source flushes per wave");
   const int lane = threadIdx.x % kT, wv = wave_in_block();
@@ -874,7 +953,7 @@ __device__ __forceinline__ void cn_tile(
   const double xa = pos[3 * (int64_t)i], ya = pos[3 * (int64_t)i + 1], za = pos[3 * (int64_t)i + 2];
   const double xb = xa * kInvBohr, yb = ya * kInvBohr, zb = za * kInvBohr;
   const int si = species[i];
-  const double rci = rcov[si], eni = en[si];
+  const double rci = rcov[si], eni = D3 ? 0.0 : en[si];
   const double gi = BACKWARD && g_cn ? g_cn[i] : 0.0;
   const double g2i = BACKWARD && g_raw ? g_raw[i] : 0.0;
   const double cmax = prm.cut_cn > prm.cut_eeq ? prm.cut_cn : prm.cut_eeq;
@@ -897,12 +976,12 @@ __device__ __forceinline__ void cn_tile(
       st.u.s.z[lane] = zs * kInvBohr;
       const int sj = species[j];
       st.u.s.rc[lane] = rcov[sj];
-      st.u.s.en[lane] = en[sj];
+      st.u.s.en[lane] = D3 ? 0.0 : en[sj];
       if (BACKWARD) {
         st.u.s.w[lane] = g_cn ? g_cn[j] : 0.0;
         st.u.s.w2[lane] = g_raw ? g_raw[j] : 0.0;
       }
-      const double r_src = fmin(cmax, (rc_tile + rcov[sj]) * zfac);
+      const double r_src = D3 ? cmax : fmin(cmax, (rc_tile + rcov[sj]) * zfac);
       int win[3];
       source_windows(G, xs, ys, zs, flo, fhi, win, r_src * kBohr);
 #pragma unroll
@@ -955,14 +1034,14 @@ __device__ __forceinline__ void cn_tile(
     if (lo0 <= hi0 && lo1 <= hi1 && lo2 <= hi2) {
       const double rc = rci + st.u.s.rc[jj];
       const double den = fabs(eni - st.u.s.en[jj]) + prm.k5;
-      const double enf = prm.k4 * exp(-den * den * inv_k6);
+      const double enf = D3 ? 1.0 : prm.k4 * exp(-den * den * inv_k6);
       // per pair: k0 / rc and the erf count's slope factor -k0 / (rc sqrt(pi))
-      const double k_rc = prm.kcn / rc;
+      const double k_rc = D3 ? prm.kcn * rc : prm.kcn / rc;
       const double dk = -k_rc * kInvSqrtPi;
       const double dx = xb - st.u.s.x[jj], dy = yb - st.u.s.y[jj], dz = zb - st.u.s.z[jj];
       const double wsum = BACKWARD ? gi + st.u.s.w[jj] : 0.0;
       const double w2sum = BACKWARD ? g2i + st.u.s.w2[jj] : 0.0;
-      const double reach2 = fmin(cmax2, rc * zfac * (rc * zfac));
+      const double reach2 = D3 ? cmax2 : fmin(cmax2, rc * zfac * (rc * zfac));
       double c_cn = 0.0, c_eeq = 0.0;          // counts within the two cutoffs
       double sv[3] = {0.0, 0.0, 0.0};          // sum of the weighted gradients
       double sc[3] = {0.0, 0.0, 0.0};          // the same with the cell's weights (own tile)
@@ -980,15 +1059,19 @@ __device__ __forceinline__ void cn_tile(
             // every lane evaluates the term and the ones outside the cutoffs discard it
             const double rinv = rsq_nr(fmax(r2, 1e-300));
             const double r = r2 * rinv;
-            const bool in_cn = in && r <= prm.cut_cn, in_eeq = in && r <= prm.cut_eeq;
-            // (1 + erf(-k0 (r - rc) / rc)) / 2; d/dr = -k0 exp(-x^2) / (rc sqrt(pi))
+            const bool in_cn = in && (D3 || r <= prm.cut_cn), in_eeq = !D3 && in && r <= prm.cut_eeq;
+            // D4: (1 + erf(-k0 (r - rc) / rc)) / 2; d/dr = -k0 exp(-x^2) / (rc sqrt(pi))
+            // D3: s = 1 / (1 + exp(-k1 (rc / r - 1))); d/dr = -s (1 - s) k1 rc / r^2
             const double x = k_rc * (rc - r);
-            if (!BACKWARD) {
+            const double sg = D3 ? rcp_nr(1.0 + exp(prm.kcn - k_rc * rinv)) : 0.0;
+            if (D3 && !BACKWARD) {
+              c_cn += in_cn ? sg : 0.0;
+            } else if (!BACKWARD) {
               const double count = 0.5 * (1.0 + erf(x));
               c_cn += in_cn ? count : 0.0;
               c_eeq += in_eeq ? count : 0.0;
             } else {
-              const double dcount = dk * exp(-x * x);
+              const double dcount = D3 ? -sg * (1.0 - sg) * k_rc * rinv * rinv : dk * exp(-x * x);
               // per Angstrom of the vector: d r_bohr / d v = v_bohr / (r bohr)
               const double s = dcount * rinv * kInvBohr;
               const double bs = ((in_cn ? wsum * enf : 0.0) + (in_eeq ? w2sum : 0.0)) * s;
@@ -1019,7 +1102,7 @@ __device__ __forceinline__ void cn_tile(
         acc[0] += enf * c_cn;
         acc[1] += c_eeq;
         vs[0] = enf * c_cn;
-        vs[1] = c_eeq;
+        if constexpr (!D3) vs[1] = c_eeq;
       } else {
 #pragma unroll
         for (int k = 0; k < 3; ++k) {
@@ -1055,7 +1138,7 @@ __device__ __forceinline__ void cn_tile(
   double v[NP];
   if constexpr (!BACKWARD) {
     v[0] = acc[0];
-    v[1] = acc[1];
+    if constexpr (!D3) v[1] = acc[1];
   } else {
 #pragma unroll
     for (int k = 0; k < 3; ++k) v[k] = g3[k];
@@ -1067,7 +1150,7 @@ __device__ __forceinline__ void cn_tile(
   if (waves_combine<W>(st.u.comb, v, wv, lane) && live) {
     double* po = partial + (int64_t)it.ls * NP * n_nodes + pi;
 #pragma unroll
-    for (int k = 0; k < (BACKWARD ? 3 : 2); ++k) po[(int64_t)k * n_nodes] = v[k];
+    for (int k = 0; k < (BACKWARD ? 3 : NF); ++k) po[(int64_t)k * n_nodes] = v[k];
     if constexpr (BACKWARD && CELL) {
 #pragma unroll
       for (int c = 0; c < 3; ++c)
@@ -1080,7 +1163,7 @@ __device__ __forceinline__ void cn_tile(
   }
 }
 
-template <bool BACKWARD, bool CELL, int W>
+template <bool BACKWARD, bool CELL, int W, bool D3>
 __global__ __launch_bounds__(kT * W, 3) void d4_cn_tiles_kernel(
     const double* __restrict__ pos, const int32_t* __restrict__ species,
     const int64_t* __restrict__ node_ptr, int64_t n_graphs, const double* __restrict__ cell,
@@ -1096,11 +1179,34 @@ __global__ __launch_bounds__(kT * W, 3) void d4_cn_tiles_kernel(
   const double cmax = prm.cut_cn > prm.cut_eeq ? prm.cut_cn : prm.cut_eeq;
   tile_geo(cell, images, it.b, cmax * kBohr, G);
   if (it.ls == it.lt)
-    cn_tile<BACKWARD, CELL, true, W>(st, it, G, prm, pos, species, rcov, en, g_cn, g_raw, order,
-                                     n_nodes, partial);
+    cn_tile<BACKWARD, CELL, true, W, D3>(st, it, G, prm, pos, species, rcov, en, g_cn, g_raw,
+                                         order, n_nodes, partial);
   else
-    cn_tile<BACKWARD, CELL, false, W>(st, it, G, prm, pos, species, rcov, en, g_cn, g_raw, order,
-                                      n_nodes, partial);
+    cn_tile<BACKWARD, CELL, false, W, D3>(st, it, G, prm, pos, species, rcov, en, g_cn, g_raw,
+                                          order, n_nodes, partial);
+}
+
+// D3: rows[i][s][a] = sum_b C6ref[s][s_i][a][b] W_i[b], a thread per (atom, species)
+__global__ __launch_bounds__(256) void d3_rows_kernel(const double* __restrict__ weights,
+                                                      const int32_t* __restrict__ species,
+                                                      const double* __restrict__ c6ref,
+                                                      int n_species, int64_t n_nodes,
+                                                      double* __restrict__ rows) {
+  const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (t >= n_nodes * n_species) return;
+  const int64_t i = t / n_species;
+  const int s = (int)(t % n_species);
+  const double* __restrict__ blk = c6ref + ((int64_t)s * n_species + species[i]) * (kNR * kNR);
+  double w[kNR];
+#pragma unroll
+  for (int b = 0; b < kNR; ++b) w[b] = weights[kNR * i + b];
+#pragma unroll
+  for (int a = 0; a < kNR; ++a) {
+    double v = 0.0;
+#pragma unroll
+    for (int b = 0; b < kNR; ++b) v += blk[a * kNR + b] * w[b];
+    rows[t * kNR + a] = v;
+  }
 }
 
 // ---------------------------------------------------------------- image counts
@@ -1200,6 +1306,7 @@ struct TilesWs {
   double* partial;
   double* partial_alpha;
   double* fsum;       // pair sums of the two-body backward, kT x kT per work item
+  double* rows;       // D3: the atoms' C6 rows
   int max_nt;
   int64_t grid_tiles;
   size_t need;
@@ -1209,7 +1316,7 @@ size_t ws_align(size_t x) { return (x + 255) & ~size_t(255); }
 
 // workspace layout for components np (+ 23 alpha components when alpha is set)
 TilesWs tiles_layout(void* ws, int64_t n_nodes, int64_t n_graphs, int64_t max_atoms, int np,
-                     bool alpha) {
+                     bool alpha, int d3_species = 0) {
   TilesWs w{};
   w.max_nt = (int)((std::max<int64_t>(max_atoms, 1) + kT - 1) / kT);
   // tiles of all structures: sum of ceil(n_b / 64) <= (n_nodes + 63 n_graphs) / 64
@@ -1226,6 +1333,8 @@ TilesWs tiles_layout(void* ws, int64_t n_nodes, int64_t n_graphs, int64_t max_at
   if (alpha) o += ws_align((size_t)w.max_nt * kNW * n_nodes * sizeof(double));
   const size_t o_fsum = o;
   if (alpha) o += ws_align((size_t)w.grid_tiles * w.max_nt * kT * kT * sizeof(double));
+  const size_t o_rows = o;
+  o += ws_align((size_t)d3_species * kNR * n_nodes * sizeof(double));
   w.need = o;
   if (base) {
     w.order = reinterpret_cast<int32_t*>(base + o_order);
@@ -1233,6 +1342,7 @@ TilesWs tiles_layout(void* ws, int64_t n_nodes, int64_t n_graphs, int64_t max_at
     w.partial = reinterpret_cast<double*>(base + o_part);
     w.partial_alpha = alpha ? reinterpret_cast<double*>(base + o_alpha) : nullptr;
     w.fsum = alpha ? reinterpret_cast<double*>(base + o_fsum) : nullptr;
+    w.rows = d3_species ? reinterpret_cast<double*>(base + o_rows) : nullptr;
   }
   return w;
 }
@@ -1305,19 +1415,19 @@ void launch_pair_backward(bool with_cell, dim3 grid, hipStream_t s, const double
                           const double* alpha, const PairParams& p, const double* g_e2,
                           const int32_t* order, const int32_t* tile_ptr, int64_t n_nodes,
                           int max_nt, double* partial, double* fsum, double* partial_alpha) {
-  auto k = with_cell ? d4_pair_tiles_kernel<true, true, kPairWaves>
-                     : d4_pair_tiles_kernel<true, false, kPairWaves>;
+  auto k = with_cell ? d4_pair_tiles_kernel<true, true, kPairWaves, false>
+                     : d4_pair_tiles_kernel<true, false, kPairWaves, false>;
   hipLaunchKernelGGL(k, grid, dim3(kT * kPairWaves), 0, s, pos, species, node_ptr, n_graphs, cell,
-                     images, r4r2, alpha, p, g_e2, order, tile_ptr, n_nodes, max_nt, partial, fsum,
-                     partial_alpha);
+                     images, r4r2, alpha, D3Rows{}, p, g_e2, order, tile_ptr, n_nodes, max_nt,
+                     partial, fsum, partial_alpha);
 }
 
 }  // namespace
 
 size_t d4_tiles_workspace_bytes(int64_t n_nodes, int64_t n_graphs, int64_t max_atoms) {
   if (n_nodes <= 0) return 0;
-  // the largest user: the pair backward with the cell, 12 + 23 components
-  return tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, 12, true).need;
+  // the largest user: the pair backward with the cell, 12 + 23 components, and D3's rows
+  return tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, 12, true, kD3MaxSpecies).need;
 }
 
 }  // namespace xnn
@@ -1346,7 +1456,7 @@ int xnn_d4_coordination(const double* pos, int64_t n_nodes, const int32_t* speci
   const CnParams p{prm->cutoff_cn, prm->cutoff_eeq_cn, prm->kcn, prm->k4, prm->k5, prm->k6};
   hipStream_t s = as_hip(stream);
   launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
-  hipLaunchKernelGGL((d4_cn_tiles_kernel<false, false, kCnWaves>), tiles_grid(w),
+  hipLaunchKernelGGL((d4_cn_tiles_kernel<false, false, kCnWaves, false>), tiles_grid(w),
                      dim3(kT * kCnWaves), 0, s, pos,
                      species, node_ptr, n_graphs, cell, images, rcov, en, p, nullptr, nullptr,
                      w.order, w.tile_ptr, n_nodes, w.max_nt, w.partial);
@@ -1380,8 +1490,8 @@ int xnn_d4_coordination_backward(const double* pos, int64_t n_nodes, const int32
   const CnParams p{prm->cutoff_cn, prm->cutoff_eeq_cn, prm->kcn, prm->k4, prm->k5, prm->k6};
   hipStream_t s = as_hip(stream);
   launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
-  auto k = with_cell ? d4_cn_tiles_kernel<true, true, kCnWaves>
-                     : d4_cn_tiles_kernel<true, false, kCnWaves>;
+  auto k = with_cell ? d4_cn_tiles_kernel<true, true, kCnWaves, false>
+                     : d4_cn_tiles_kernel<true, false, kCnWaves, false>;
   hipLaunchKernelGGL(k, tiles_grid(w), dim3(kT * kCnWaves), 0, s, pos, species, node_ptr, n_graphs,
                      cell,
                      images, rcov, en, p, g_cn_d4, g_cn_raw, w.order, w.tile_ptr, n_nodes,
@@ -1412,9 +1522,9 @@ int xnn_d4_two_body(const double* pos, int64_t n_nodes, const int32_t* species,
   const PairParams p{prm->s6, prm->s8, prm->a1, prm->a2, prm->cutoff, prm->width};
   hipStream_t s = as_hip(stream);
   launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
-  hipLaunchKernelGGL((d4_pair_tiles_kernel<false, false, 1>), tiles_grid(w), dim3(kT), 0, s, pos,
-                     species, node_ptr, n_graphs, cell, images, r4r2, alpha, p, nullptr, w.order,
-                     w.tile_ptr, n_nodes, w.max_nt, w.partial, nullptr, nullptr);
+  hipLaunchKernelGGL((d4_pair_tiles_kernel<false, false, 1, false>), tiles_grid(w), dim3(kT), 0, s,
+                     pos, species, node_ptr, n_graphs, cell, images, r4r2, alpha, D3Rows{}, p,
+                     nullptr, w.order, w.tile_ptr, n_nodes, w.max_nt, w.partial, nullptr, nullptr);
   launch_reduce({{w.partial, e2, 1, 0, 1}}, n_nodes, w, batch, node_ptr, s);
   XNN_LAUNCH_CHECK();
   return XNN_OK;
@@ -1450,6 +1560,162 @@ int xnn_d4_two_body_backward(const double* pos, int64_t n_nodes, const int32_t* 
                        w.fsum, w.partial_alpha);
   launch_reduce({{w.partial, grad_pos, np, 0, 3}, {w.partial, cell_partial, np, 3, 9},
                  {w.partial_alpha, grad_alpha, kNW, 0, kNW}},
+                n_nodes, w, batch, node_ptr, s);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_d3_coordination_planned(const double* pos, int64_t n_nodes, const int32_t* species,
+                                const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                                int64_t max_atoms, const double* cell, const int32_t* images,
+                                const int32_t* plan, const double* rcov, double cutoff_cn,
+                                double kcn, double* cn, void* workspace, size_t workspace_bytes,
+                                xnn_stream_t stream) {
+  const int st = tiles_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images,
+                             max_atoms);
+  if (st != XNN_OK) return st;
+  XNN_REQUIRE(rcov != nullptr, "NULL rcov");
+  XNN_REQUIRE(n_nodes == 0 || cn, "NULL output");
+  if (n_nodes == 0) return XNN_OK;
+  const TilesWs need = tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, 1, false);
+  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need.need,
+              "workspace too small (%zu < %zu)", workspace_bytes, need.need);
+  TilesWs w = tiles_layout(workspace, n_nodes, n_graphs, max_atoms, 1, false);
+  const CnParams p{cutoff_cn, 0.0, kcn, 0.0, 0.0, 1.0};
+  hipStream_t s = as_hip(stream);
+  launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
+  hipLaunchKernelGGL((d4_cn_tiles_kernel<false, false, kCnWaves, true>), tiles_grid(w),
+                     dim3(kT * kCnWaves), 0, s, pos, species, node_ptr, n_graphs, cell, images, rcov,
+                     nullptr, p, nullptr, nullptr, w.order, w.tile_ptr, n_nodes, w.max_nt, w.partial);
+  launch_reduce({{w.partial, cn, 1, 0, 1}}, n_nodes, w, batch, node_ptr, s);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_d3_coordination_backward_planned(
+    const double* pos, int64_t n_nodes, const int32_t* species, const int32_t* batch,
+    const int64_t* node_ptr, int64_t n_graphs, int64_t max_atoms, const double* cell,
+    const int32_t* images, const int32_t* plan, const double* rcov, double cutoff_cn, double kcn,
+    const double* g_cn, double* grad_pos, double* cell_partial, void* workspace,
+    size_t workspace_bytes, xnn_stream_t stream) {
+  const int st = tiles_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images,
+                             max_atoms);
+  if (st != XNN_OK) return st;
+  XNN_REQUIRE(rcov != nullptr, "NULL rcov");
+  XNN_REQUIRE(n_nodes == 0 || (grad_pos && g_cn), "NULL g_cn or grad_pos");
+  if (n_nodes == 0) return XNN_OK;
+  const bool with_cell = cell_partial != nullptr;
+  const int np = with_cell ? 12 : 3;
+  const TilesWs need = tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, np, false);
+  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need.need,
+              "workspace too small (%zu < %zu)", workspace_bytes, need.need);
+  TilesWs w = tiles_layout(workspace, n_nodes, n_graphs, max_atoms, np, false);
+  const CnParams p{cutoff_cn, 0.0, kcn, 0.0, 0.0, 1.0};
+  hipStream_t s = as_hip(stream);
+  launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
+  auto k = with_cell ? d4_cn_tiles_kernel<true, true, kCnWaves, true>
+                     : d4_cn_tiles_kernel<true, false, kCnWaves, true>;
+  hipLaunchKernelGGL(k, tiles_grid(w), dim3(kT * kCnWaves), 0, s, pos, species, node_ptr, n_graphs,
+                     cell, images, rcov, nullptr, p, g_cn, nullptr, w.order, w.tile_ptr, n_nodes,
+                     w.max_nt, w.partial);
+  launch_reduce({{w.partial, grad_pos, np, 0, 3}, {w.partial, cell_partial, np, 3, 9}}, n_nodes, w,
+                batch, node_ptr, s);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_d3_coordination(const double* pos, int64_t n_nodes, const int32_t* species,
+                        const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                        int64_t max_atoms, const double* cell, const int32_t* images,
+                        const double* rcov, double cutoff_cn, double kcn, double* cn,
+                        void* workspace, size_t workspace_bytes, xnn_stream_t stream) {
+  return xnn_d3_coordination_planned(pos, n_nodes, species, batch, node_ptr, n_graphs, max_atoms,
+                                     cell, images, nullptr, rcov, cutoff_cn, kcn, cn, workspace,
+                                     workspace_bytes, stream);
+}
+
+int xnn_d3_coordination_backward(const double* pos, int64_t n_nodes, const int32_t* species,
+                                 const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                                 int64_t max_atoms, const double* cell, const int32_t* images,
+                                 const double* rcov, double cutoff_cn, double kcn,
+                                 const double* g_cn, double* grad_pos, double* cell_partial,
+                                 void* workspace, size_t workspace_bytes, xnn_stream_t stream) {
+  return xnn_d3_coordination_backward_planned(pos, n_nodes, species, batch, node_ptr, n_graphs,
+                                              max_atoms, cell, images, nullptr, rcov, cutoff_cn,
+                                              kcn, g_cn, grad_pos, cell_partial, workspace,
+                                              workspace_bytes, stream);
+}
+
+static int d3_tiles_check(const xnn_d3_pair_params* prm, const double* r4r2, const double* c6ref,
+                          int n_species) {
+  XNN_REQUIRE(prm && r4r2 && c6ref, "NULL tables or params");
+  XNN_REQUIRE(n_species >= 1 && n_species <= kD3MaxSpecies, "1 to %d species (got %d)",
+              kD3MaxSpecies, n_species);
+  XNN_REQUIRE(prm->damping == 0, "the tiles take the rational damping only");
+  XNN_REQUIRE(prm->cutoff > 0.0, "pair cutoff must be positive");
+  return XNN_OK;
+}
+
+int xnn_d3_two_body_tiles(const double* pos, int64_t n_nodes, const int32_t* species,
+                          const int32_t* batch, const int64_t* node_ptr, int64_t n_graphs,
+                          int64_t max_atoms, const double* cell, const int32_t* images,
+                          const int32_t* plan, const double* r4r2, const double* c6ref,
+                          int32_t n_species, const double* weights, const xnn_d3_pair_params* prm,
+                          double* e2, void* workspace, size_t workspace_bytes,
+                          xnn_stream_t stream) {
+  int st = tiles_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images, max_atoms);
+  if (st == XNN_OK) st = d3_tiles_check(prm, r4r2, c6ref, n_species);
+  if (st != XNN_OK) return st;
+  XNN_REQUIRE(n_nodes == 0 || (weights && e2), "NULL weights or output");
+  if (n_nodes == 0) return XNN_OK;
+  const TilesWs need = tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, 1, false, n_species);
+  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need.need,
+              "workspace too small (%zu < %zu)", workspace_bytes, need.need);
+  TilesWs w = tiles_layout(workspace, n_nodes, n_graphs, max_atoms, 1, false, n_species);
+  const PairParams p{prm->s6, prm->s8, prm->a1, prm->a2, prm->cutoff, prm->width};
+  hipStream_t s = as_hip(stream);
+  launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
+  hipLaunchKernelGGL(d3_rows_kernel, dim3((unsigned)grid_1d(n_nodes * n_species, 256)), dim3(256), 0,
+                     s, weights, species, c6ref, n_species, n_nodes, w.rows);
+  hipLaunchKernelGGL((d4_pair_tiles_kernel<false, false, 1, true>), tiles_grid(w), dim3(kT), 0, s,
+                     pos, species, node_ptr, n_graphs, cell, images, r4r2, nullptr,
+                     D3Rows{weights, w.rows, n_species}, p, nullptr, w.order, w.tile_ptr, n_nodes,
+                     w.max_nt, w.partial, nullptr, nullptr);
+  launch_reduce({{w.partial, e2, 1, 0, 1}}, n_nodes, w, batch, node_ptr, s);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_d3_two_body_tiles_backward(
+    const double* pos, int64_t n_nodes, const int32_t* species, const int32_t* batch,
+    const int64_t* node_ptr, int64_t n_graphs, int64_t max_atoms, const double* cell,
+    const int32_t* images, const int32_t* plan, const double* r4r2, const double* c6ref,
+    int32_t n_species, const double* weights, const xnn_d3_pair_params* prm, const double* g_e2,
+    double* grad_pos, double* cell_partial, double* grad_weights, void* workspace,
+    size_t workspace_bytes, xnn_stream_t stream) {
+  int st = tiles_check(pos, n_nodes, species, batch, node_ptr, n_graphs, cell, images, max_atoms);
+  if (st == XNN_OK) st = d3_tiles_check(prm, r4r2, c6ref, n_species);
+  if (st != XNN_OK) return st;
+  XNN_REQUIRE(n_nodes == 0 || (weights && g_e2 && grad_pos), "NULL weights, g_e2 or grad_pos");
+  if (n_nodes == 0) return XNN_OK;
+  const bool with_cell = cell_partial != nullptr;
+  const int np = with_cell ? 12 : 3;
+  const TilesWs need = tiles_layout(nullptr, n_nodes, n_graphs, max_atoms, np, true, n_species);
+  XNN_REQUIRE(workspace != nullptr && workspace_bytes >= need.need,
+              "workspace too small (%zu < %zu)", workspace_bytes, need.need);
+  TilesWs w = tiles_layout(workspace, n_nodes, n_graphs, max_atoms, np, true, n_species);
+  const PairParams p{prm->s6, prm->s8, prm->a1, prm->a2, prm->cutoff, prm->width};
+  hipStream_t s = as_hip(stream);
+  launch_order(pos, n_nodes, node_ptr, n_graphs, cell, images, plan, w, s);
+  hipLaunchKernelGGL(d3_rows_kernel, dim3((unsigned)grid_1d(n_nodes * n_species, 256)), dim3(256), 0,
+                     s, weights, species, c6ref, n_species, n_nodes, w.rows);
+  auto k = with_cell ? d4_pair_tiles_kernel<true, true, kPairWaves, true>
+                     : d4_pair_tiles_kernel<true, false, kPairWaves, true>;
+  hipLaunchKernelGGL(k, tiles_grid(w), dim3(kT * kPairWaves), 0, s, pos, species, node_ptr, n_graphs,
+                     cell, images, r4r2, nullptr, D3Rows{weights, w.rows, n_species}, p, g_e2,
+                     w.order, w.tile_ptr, n_nodes, w.max_nt, w.partial, w.fsum, w.partial_alpha);
+  launch_reduce({{w.partial, grad_pos, np, 0, 3}, {w.partial, cell_partial, np, 3, 9},
+                 {w.partial_alpha, grad_weights, kNR, 0, kNR}},
                 n_nodes, w, batch, node_ptr, s);
   XNN_LAUNCH_CHECK();
   return XNN_OK;
