@@ -558,7 +558,7 @@ class IterativeEEQSystem:
         """The preconditioner ``M = D + U W U^T`` (dispersion_fast/eeq.py:72-86): ``U = [cos,
         sin]`` of the :data:`LOW_K_VECTORS` smallest reciprocal vectors at the (ordered)
         positions, ``W`` their weights, ``D`` the full diagonal of ``A`` less that part's
-        (``sum_l w_l``); ``M^-1`` through the Woodbury identity with the Cholesky factor of
+        (``sum_l w_l``); ``M^-1`` through the Woodbury identity with the inverse of
         ``W^-1 + U^T D^-1 U``. It changes how fast the iteration converges, not its limit."""
         g, w = reciprocal_weights(self.m, self.cell, self.alpha)
         L = min(LOW_K_VECTORS, int(g.shape[0]))
@@ -572,14 +572,16 @@ class IterativeEEQSystem:
         wl = torch.cat([w[idx], w[idx]])
         self.inv_d = (1.0 / (full_s - w[idx].sum())).contiguous()
         core = torch.diag(1.0 / wl) + self.U.t() @ (self.inv_d[:, None] * self.U)
-        self.core = torch.linalg.cholesky(core)
+        # its inverse, once: two triangular solves of 512 rows are some twenty small launches
+        # an iteration, a product with the inverse is one
+        self.core_inv = torch.cholesky_inverse(torch.linalg.cholesky(core))
 
     def precondition(self, r: Tensor) -> Tensor:
         """``M^-1 r`` for the columns of ``r``."""
         z = self.inv_d[:, None] * r
         if self.U is None:
             return z
-        t = torch.cholesky_solve(_tn_product(self.U, z), self.core)
+        t = self.core_inv @ _tn_product(self.U, z)
         return z - self.inv_d[:, None] * (self.U @ t)
 
     def _matvec(self, v: Tensor) -> Tensor:
