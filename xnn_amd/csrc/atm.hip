@@ -31,8 +31,8 @@
 // lane pair holding one of up to 32 sums) and added atomically as reproducible sums: a
 // head and a tail of fixed quanta whose float64 sums are exact in any order (atm_acc), so
 // the results do not depend on the order of the atomics. Items run heaviest tile first.
-// Repeated-atom triangles: one wave per flagged center, lanes over its edges, each lane
-// walking the few later edges that share an atom with its own.
+// Repeated-atom triangles: waves over tiles of a flagged center's edges, an edge per lane,
+// against the center's few self edges in lockstep and the lane's own run of equal neighbors.
 //
 // Pair C6 = <fa[x], fb[y]> over K <= 32 components (held per lane for j); the damping
 // radius is the product of three species-pair factors. Energies in hartree, lengths in
@@ -140,7 +140,7 @@ static AtmPlanLayout atm_plan_layout(int64_t E, int64_t N) {
 }
 
 struct AtmWorkLayout {
-  size_t rec, rec_up, fa, fb, gs, skey, sval, skey_out, sperm, cub, cub_bytes, tail,
+  size_t rec, rec_up, fa, fb, gs, rep, skey, sval, skey_out, sperm, cub, cub_bytes, tail,
       tail_count, total;
 };
 
@@ -172,6 +172,9 @@ static AtmWorkLayout atm_work_layout(int64_t E, int64_t N, int kp, bool backward
   L.fb = at; at += atm_align(sizeof(double) * kp * std::max<int64_t>(N, 1));
   L.gs = at;
   if (backward) at += atm_align(sizeof(double) * 4 * std::max<int64_t>(E, 1));
+  // the repeated triangles' g1 and gt of every edge
+  L.rep = at;
+  if (backward) at += atm_align(sizeof(double) * 2 * std::max<int64_t>(E, 1));
   // the tails of the reproducible sums: energies (forward); or gs, gfa and gfb (backward)
   L.tail = at;
   L.tail_count = backward ? 4 * E + 2 * N * (int64_t)kp : N;
@@ -710,103 +713,144 @@ __global__ __launch_bounds__(kAtmWaves * kWave) void atm_upper_kernel(
 // Triangles with a repeated atom, at every visit of a flagged center c, a third to c:
 // the pairs of c's edges where one edge goes to an image of c itself (any partner) or
 // both go to images of one neighbor. Edges of c are sorted by neighbor, so the partners
-// of an edge are its run of equal neighbors and the run of self-image edges, which ends
-// the lower range [lo[c], lo1[c]).
-template <int KP, bool SWITCH, bool BWD>
+// of an edge are its run of equal neighbors and the run of self-image edges [s0, lo1[c]),
+// which ends the lower range. A wave takes a center and every `splits`-th tile of 64 of its
+// edges, an edge per lane: the few self edges are walked in lockstep (wave-uniform, their
+// sums folded over the wave), and each lane walks its own run. The backward walks the run
+// in both directions and keeps its own edge's gradients only, so the partners need no
+// atomics. The factor gradients need none either: with the first edge of a pair the one
+// earlier in c's row, C6_jk is <fa[j], fb[c]> for an edge before the self edges (its dE/dC6
+// summed to g1), <fa[c], fb[j]> = the edge's own C6_cj after them (added to that) and
+// <fa[j], fb[j]> within a run (gt); the center-side kernel multiplies them by the factors,
+// a wave per atom. A lane that walked a self edge's partners by itself, each with 56
+// atomics, took 42.5 ms for the 2.2 million edges of a 700-atom cell; this takes
+// 0.6 ms.
+template <int KP, bool SWITCH, bool BWD, bool P16>
 __global__ __launch_bounds__(kAtmWaves * kWave) void atm_repeat_kernel(
     const AtmEdge* __restrict__ rec, const int32_t* __restrict__ lo,
     const int32_t* __restrict__ lo1, const int32_t* __restrict__ flag, int64_t N,
     const double* __restrict__ fa, const double* __restrict__ fb,
     const double* __restrict__ table, int S, AtmConst kc, double* __restrict__ energy,
-    const double* __restrict__ go, double* __restrict__ gs, double* __restrict__ gfa,
-    double* __restrict__ gfb, int K, AtmTail tail) {
+    const double* __restrict__ go, double* __restrict__ gs, AtmTail tail,
+    double* __restrict__ g1_out, double* __restrict__ gt_out) {
   __shared__ double sTab[kAtmMaxSpecies * kAtmMaxSpecies];
   atm_stage_table(table, S, sTab);
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t c = (int64_t)blockIdx.x * kAtmWaves + wave_in_block();
-  if (c >= N || flag[c] == 0) return;
+  if (c >= N) return;
   const int32_t l0 = lo[c], u0 = lo1[c], hi = lo[c + 1];
+  const int32_t a_first = l0 + (int32_t)blockIdx.y * kAtmTile;
+  const int32_t a_step = (int32_t)gridDim.y * kAtmTile;
+  if (flag[c] == 0) {                               // uniform
+    if (BWD)
+      for (int32_t a = a_first + lane; a < hi; a += a_step) g1_out[a] = gt_out[a] = 0.0;
+    return;
+  }
+  const AtmLanes L = atm_lanes(lane);
   int32_t s0 = u0;                                  // self-image edges: [s0, u0)
   while (s0 > l0 && atm_nb(rec[s0 - 1]) == (int32_t)c) --s0;
-  const double go_c = BWD ? go[c] : 0.0;
+  const double weight = BWD ? go[c] : 1.0;
+  const double* __restrict__ fac = fa + c * KP;
+  const double* __restrict__ fbc = fb + c * KP;
   double e_acc = 0.0;
-  for (int32_t a0 = l0; a0 < hi; a0 += kAtmTile) {
+  for (int32_t a0 = a_first; a0 < hi; a0 += a_step) {
     const int32_t a = a0 + lane;
-    if (a >= hi) break;
-    const AtmEdge ea = rec[a];
+    const bool va = a < hi;
+    const AtmEdge ea = rec[va ? a : a0];
     const double ax = ea.vx, ay = ea.vy, az = ea.vz;
     const double x = ax * ax + ay * ay + az * az;
     const double ix = BWD ? rcp_nr(x) : 0.0;
+    const double hc6a = BWD ? 0.5 / (ea.c6 != 0.0 ? ea.c6 : 1.0) : 0.0;
     const int32_t j = atm_nb(ea);
-    double fj[KP];
+    const int sj = atm_snb(ea);
+    double before = 0.0, own = 0.0;                 // <fa[j], fb[c]>, <fa[j], fb[j]>
 #pragma unroll
-    for (int w = 0; w < KP; ++w) fj[w] = fa[(int64_t)j * KP + w];
-    double gax = 0.0, gay = 0.0, gaz = 0.0, gc6a = 0.0;
-    double gfj[BWD ? KP : 1];
-#pragma unroll
-    for (int w = 0; w < (BWD ? KP : 1); ++w) gfj[w] = 0.0;
-    // partner ranges: a self edge pairs with every later edge; another edge with its
-    // run of equal neighbors and with the later self edges
-    const bool self = j == (int32_t)c;
-    int32_t run_end = a + 1;
-    if (!self)
-      while (run_end < hi && atm_nb(rec[run_end]) == j) ++run_end;
-    const int32_t r1_end = self ? hi : run_end;
+    for (int w = 0; w < KP; ++w) {
+      const double f = fa[(int64_t)j * KP + w];
+      before = fma(f, fbc[w], before);
+      own = fma(f, fb[(int64_t)j * KP + w], own);
+    }
+    double gax = 0.0, gay = 0.0, gaz = 0.0, gc6a = 0.0, g1 = 0.0, g2 = 0.0, gt = 0.0;
     bool any = false;                               // a triangle was kept for this edge
-    const int32_t r2_beg = self ? hi : (s0 > a + 1 ? s0 : a + 1);
-    const int32_t r2_end = self ? hi : u0;
-    for (int pass = 0; pass < 2; ++pass) {
-      const int32_t b_beg = pass == 0 ? a + 1 : r2_beg;
-      const int32_t b_end = pass == 0 ? r1_end : r2_end;
-      for (int32_t b = b_beg; b < b_end; ++b) {
+    for (int32_t q = s0; q < u0; ++q) {
+      const AtmEdge es = rec[q];                    // wave-uniform
+      const double dx = ax - es.vx, dy = ay - es.vy, dz = az - es.vz;
+      const double w2 = dx * dx + dy * dy + dz * dz;
+      // another edge pairs with every self edge, a self edge with the earlier ones
+      const bool keep = va && (a < s0 || a >= u0 || q < a) && w2 <= kc.cut2 && w2 > kAtmEps;
+      if (__ballot(keep) == 0) continue;
+      double e = 0.0, gx = 0.0, gy = 0.0, gw = 0.0;
+      const double c6jk = a < s0 ? before : ea.c6;
+      if (keep) {
+        any = true;
+        const double y = es.vx * es.vx + es.vy * es.vy + es.vz * es.vz;
+        const int sc = atm_snb(es);
+        const double r0 = ea.p * es.p * sTab[a < s0 ? sj * S + sc : sc * S + sj];
+        atm_triangle<SWITCH, BWD, P16>(kc, x, y, w2, ix, BWD ? rcp_nr(y) : 0.0,
+                                       fabs(ea.c6 * es.c6 * c6jk), r0, ea.sw, es.sw, ea.dsw,
+                                       es.dsw, weight, e, gx, gy, gw);
+      }
+      if (!BWD) {
+        e_acc += e;
+      } else {
+        const double g3 = 0.5 * e * rcp_nr(c6jk != 0.0 ? c6jk : 1.0);
+        g1 += a < s0 ? g3 : 0.0;
+        g2 += a < s0 ? 0.0 : g3;
+        gax = fma(2.0, fma(gx, ax, gw * dx), gax);
+        gay = fma(2.0, fma(gx, ay, gw * dy), gay);
+        gaz = fma(2.0, fma(gx, az, gw * dz), gaz);
+        gc6a = fma(e, hc6a, gc6a);
+        const double vs = atm_fold4(2.0 * fma(gy, es.vx, -gw * dx), 2.0 * fma(gy, es.vy, -gw * dy),
+                                    2.0 * fma(gy, es.vz, -gw * dz),
+                                    0.5 * e / (es.c6 != 0.0 ? es.c6 : 1.0), lane, L);
+        if ((lane & 15) == 0) atm_acc(gs, tail.gs, (int64_t)q * 4 + (lane >> 4), vs);
+      }
+    }
+    // the edges of the lane's own run: the later ones, in the backward the earlier ones too
+    if (va && (a < s0 || a >= u0)) {
+      const double r0p = sTab[sj * S + sj];
+      const auto pair = [&](int32_t b) {
         const AtmEdge eb = rec[b];
+        if (atm_nb(eb) != j) return false;
         const double dx = ax - eb.vx, dy = ay - eb.vy, dz = az - eb.vz;
         const double w2 = dx * dx + dy * dy + dz * dz;
-        if (!(w2 <= kc.cut2 && w2 > kAtmEps)) continue;
+        if (!(w2 <= kc.cut2 && w2 > kAtmEps)) return true;
         any = true;
-        const int32_t k = atm_nb(eb);
         const double y = eb.vx * eb.vx + eb.vy * eb.vy + eb.vz * eb.vz;
-        const double* __restrict__ fk = fb + (int64_t)k * KP;
-        double c6jk = 0.0;
-#pragma unroll
-        for (int w = 0; w < KP; ++w) c6jk = fma(fj[w], fk[w], c6jk);
-        const double r0 = ea.p * eb.p * sTab[atm_snb(ea) * S + atm_snb(eb)];
         double e, gx = 0.0, gy = 0.0, gw = 0.0;
-        atm_triangle<SWITCH, BWD, false>(kc, x, y, w2, ix, BWD ? rcp_nr(y) : 0.0,
-                                  fabs(ea.c6 * eb.c6 * c6jk), r0, ea.sw, eb.sw, ea.dsw, eb.dsw,
-                                  BWD ? go_c : 1.0, e, gx, gy, gw);
+        atm_triangle<SWITCH, BWD, P16>(kc, x, y, w2, ix, BWD ? rcp_nr(y) : 0.0,
+                                       fabs(ea.c6 * eb.c6 * own), ea.p * eb.p * r0p, ea.sw, eb.sw,
+                                       ea.dsw, eb.dsw, weight, e, gx, gy, gw);
         if (!BWD) {
           e_acc += e;
         } else {
-          const double g3 = 0.5 * e / (c6jk != 0.0 ? c6jk : 1.0);
           gax = fma(2.0, fma(gx, ax, gw * dx), gax);
           gay = fma(2.0, fma(gx, ay, gw * dy), gay);
           gaz = fma(2.0, fma(gx, az, gw * dz), gaz);
-          gc6a += 0.5 * e / (ea.c6 != 0.0 ? ea.c6 : 1.0);
-#pragma unroll
-          for (int w = 0; w < KP; ++w) gfj[w] = fma(g3, fk[w], gfj[w]);
-          atm_acc(gs, tail.gs, (int64_t)b * 4 + 0, 2.0 * fma(gy, eb.vx, -gw * dx));
-          atm_acc(gs, tail.gs, (int64_t)b * 4 + 1, 2.0 * fma(gy, eb.vy, -gw * dy));
-          atm_acc(gs, tail.gs, (int64_t)b * 4 + 2, 2.0 * fma(gy, eb.vz, -gw * dz));
-          atm_acc(gs, tail.gs, (int64_t)b * 4 + 3, 0.5 * e / (eb.c6 != 0.0 ? eb.c6 : 1.0));
-#pragma unroll
-          for (int w = 0; w < KP; ++w)
-            if (w < K) atm_acc(gfb, tail.gfb, (int64_t)k * K + w, g3 * fj[w]);
+          gc6a = fma(e, hc6a, gc6a);
+          if (b > a) gt += 0.5 * e * rcp_nr(own != 0.0 ? own : 1.0);
         }
+        return true;
+      };
+      for (int32_t b = a + 1; b < hi && pair(b); ++b) {
       }
+      if (BWD)
+        for (int32_t b = a - 1; b >= l0 && pair(b); --b) {
+        }
     }
-    if (BWD && any) {
-      atm_acc(gs, tail.gs, (int64_t)a * 4 + 0, gax);
-      atm_acc(gs, tail.gs, (int64_t)a * 4 + 1, gay);
-      atm_acc(gs, tail.gs, (int64_t)a * 4 + 2, gaz);
-      atm_acc(gs, tail.gs, (int64_t)a * 4 + 3, gc6a);
-#pragma unroll
-      for (int w = 0; w < KP; ++w)
-        if (w < K) atm_acc(gfa, tail.gfa, (int64_t)j * K + w, gfj[w]);
+    if (BWD && va) {
+      g1_out[a] = g1;
+      gt_out[a] = gt;
+      if (any) {
+        atm_acc(gs, tail.gs, (int64_t)a * 4 + 0, gax);
+        atm_acc(gs, tail.gs, (int64_t)a * 4 + 1, gay);
+        atm_acc(gs, tail.gs, (int64_t)a * 4 + 2, gaz);
+        atm_acc(gs, tail.gs, (int64_t)a * 4 + 3, gc6a + g2);
+      }
     }
   }
   if (!BWD) {
-    const double ec = atm_wave_sum(e_acc, atm_lanes(lane));
+    const double ec = atm_wave_sum(e_acc, L);
     if (lane == 0) atm_acc(energy, tail.energy, c, ec);
   }
 }
@@ -825,14 +869,17 @@ __global__ __launch_bounds__(256) void atm_vec_grad_kernel(const int32_t* __rest
 
 // The center sides C6_cj = <fa[c], fb[j]> of every edge, one wave per atom x, no atomics:
 // gfa[x] += sum over x's row (x the center) of dE/dC6 fb[j], gfb[x] += sum over the edges
-// whose neighbor is x (the plan's by-source order) of dE/dC6 fa[c].
-template <int KP>
+// whose neighbor is x (the plan's by-source order) of dE/dC6 fa[c]. REP: the repeated
+// triangles' sums of atm_repeat_kernel too, gfb[x] += sum over x's row of g1 fa[j], gfa[x] +=
+// sum over the by-source edges of g1 fb[c], and sum gt times the other factor of x.
+template <int KP, bool REP>
 __global__ __launch_bounds__(kAtmWaves * kWave) void atm_center_side_kernel(
     const int32_t* __restrict__ lo, const int32_t* __restrict__ nbr,
     const int32_t* __restrict__ lo_src, const int32_t* __restrict__ by_src,
     const int32_t* __restrict__ ctr, const double* __restrict__ gs,
     const double* __restrict__ fa, const double* __restrict__ fb, int64_t N, int K,
-    double* __restrict__ gfa, double* __restrict__ gfb) {
+    const double* __restrict__ g1, const double* __restrict__ gt, double* __restrict__ gfa,
+    double* __restrict__ gfb) {
   const int lane = threadIdx.x & (kWave - 1);
   const int64_t x = (int64_t)blockIdx.x * kAtmWaves + wave_in_block();
   if (x >= N) return;
@@ -841,20 +888,37 @@ __global__ __launch_bounds__(kAtmWaves * kWave) void atm_center_side_kernel(
     const int32_t p0 = side == 0 ? lo[x] : lo_src[x];
     const int32_t p1 = side == 0 ? lo[x + 1] : lo_src[x + 1];
     if (p0 == p1) continue;                         // uniform
-    double acc[KP];
+    double acc[KP], rep[REP ? KP : 1], own = 0.0;
 #pragma unroll
     for (int w = 0; w < KP; ++w) acc[w] = 0.0;
+#pragma unroll
+    for (int w = 0; w < (REP ? KP : 1); ++w) rep[w] = 0.0;
     for (int32_t q = p0 + lane; q < p1; q += kWave) {
       const int64_t p = side == 0 ? q : by_src[q];
       const double g = gs[4 * p + 3];
-      const double* __restrict__ f = side == 0 ? fb + (int64_t)nbr[p] * KP : fa + (int64_t)ctr[p] * KP;
+      const int64_t other = side == 0 ? nbr[p] : ctr[p];
+      const double* __restrict__ f = (side == 0 ? fb : fa) + other * KP;
 #pragma unroll
       for (int w = 0; w < KP; ++w) acc[w] = fma(g, f[w], acc[w]);
+      if constexpr (REP) {
+        const double h = g1[p];
+        const double* __restrict__ f2 = (side == 0 ? fa : fb) + other * KP;
+#pragma unroll
+        for (int w = 0; w < KP; ++w) rep[w] = fma(h, f2[w], rep[w]);
+        if (side == 1) own += gt[p];
+      }
     }
     double* __restrict__ out = side == 0 ? gfa : gfb;
+    double* __restrict__ out2 = side == 0 ? gfb : gfa;
+    if constexpr (REP) own = atm_wave_sum(own, L);
 #pragma unroll
     for (int w = 0; w < KP; ++w) {
-      const double v = atm_wave_sum(acc[w], L);
+      double v = atm_wave_sum(acc[w], L);
+      if constexpr (REP) {
+        const double v2 = atm_wave_sum(rep[w], L);
+        v = fma(own, fa[x * KP + w], v);             // out is gfb where own is not zero
+        if (lane == 0 && w < K) out2[x * K + w] += fma(own, fb[x * KP + w], v2);
+      }
       if (lane == 0 && w < K) out[x * K + w] += v;
     }
   }
@@ -1364,6 +1428,8 @@ static int atm_run(const AtmArgs& A) {
   double* faP = at_off<double>(A.work, W.fa);
   double* fbP = at_off<double>(A.work, W.fb);
   double* gs = BWD ? at_off<double>(A.work, W.gs) : nullptr;
+  double* g1 = BWD ? at_off<double>(A.work, W.rep) : nullptr;
+  double* gt = BWD ? g1 + A.E : nullptr;
   const int64_t nk = A.N * (int64_t)A.K;
   double* tails = at_off<double>(A.work, W.tail);
   AtmTail tail{nullptr, nullptr, nullptr, nullptr};
@@ -1407,9 +1473,11 @@ static int atm_run(const AtmArgs& A) {
     XNN_LAUNCH_CHECK();
   }
   if (A.has_repeats) {
-    hipLaunchKernelGGL((atm_repeat_kernel<KP, SWITCH, BWD>), dim3((unsigned)n_groups),
+    // as many waves a center as its mean row has tiles
+    const unsigned splits = (unsigned)std::min<int64_t>(64, A.E / (A.N * kAtmTile) + 1);
+    hipLaunchKernelGGL((atm_repeat_kernel<KP, SWITCH, BWD, P16>), dim3((unsigned)n_groups, splits),
                        dim3(kAtmWaves * kWave), 0, A.s, rec, lo, lo1, flag, A.N, faP, fbP,
-                       A.table, A.S, A.kc, A.energy, A.go, gs, A.gfa, A.gfb, A.K, tail);
+                       A.table, A.S, A.kc, A.energy, A.go, gs, tail, g1, gt);
     XNN_LAUNCH_CHECK();
   }
   if (!BWD) {
@@ -1422,10 +1490,11 @@ static int atm_run(const AtmArgs& A) {
   if (BWD) {
     hipLaunchKernelGGL(atm_vec_grad_kernel, dim3(grid_1d(A.E, 256)), dim3(256), 0, A.s, perm, gs,
                        A.E, A.gvec);
-    hipLaunchKernelGGL((atm_center_side_kernel<KP>), dim3((unsigned)n_groups),
-                       dim3(kAtmWaves * kWave), 0, A.s, lo, nbr,
+    const auto side = A.has_repeats ? atm_center_side_kernel<KP, true>
+                                    : atm_center_side_kernel<KP, false>;
+    hipLaunchKernelGGL(side, dim3((unsigned)n_groups), dim3(kAtmWaves * kWave), 0, A.s, lo, nbr,
                        at_off<int32_t>(A.plan, P.lo_src), at_off<int32_t>(A.plan, P.by_src),
-                       at_off<int32_t>(A.plan, P.ctr), gs, faP, fbP, A.N, A.K, A.gfa, A.gfb);
+                       at_off<int32_t>(A.plan, P.ctr), gs, faP, fbP, A.N, A.K, g1, gt, A.gfa, A.gfb);
     XNN_LAUNCH_CHECK();
   }
   return XNN_OK;
@@ -1561,12 +1630,12 @@ static int atm_tangent_run(const AtmArgs& A, const AtmTanArgs& D) {
   // the factors, then their gradients with the factors' directions
   const int64_t n_groups = (A.N + kAtmWaves - 1) / kAtmWaves;
   for (int pass = 0; pass < 2; ++pass)
-    hipLaunchKernelGGL((atm_center_side_kernel<KP>), dim3((unsigned)n_groups),
+    hipLaunchKernelGGL((atm_center_side_kernel<KP, false>), dim3((unsigned)n_groups),
                        dim3(kAtmWaves * kWave), 0, A.s, lo, nbr,
                        at_off<int32_t>(A.plan, P.lo_src), at_off<int32_t>(A.plan, P.by_src),
                        at_off<int32_t>(A.plan, P.ctr), pass == 0 ? out.gs_t : out.gs,
-                       pass == 0 ? faP : fatP, pass == 0 ? fbP : fbtP, A.N, A.K, D.gfa_t,
-                       D.gfb_t);
+                       pass == 0 ? faP : fatP, pass == 0 ? fbP : fbtP, A.N, A.K, nullptr, nullptr,
+                       D.gfa_t, D.gfb_t);
   XNN_LAUNCH_CHECK();
   return XNN_OK;
 }
