@@ -619,6 +619,23 @@ int xnn_eeq_real_apply(const double* pos, int64_t n_nodes, const double* cell, c
                        int32_t nrhs, double* out, void* work, size_t work_bytes,
                        xnn_stream_t stream);
 
+/* Dense EEQ charges of molecules of at most 128 atoms (d4.py:593-606, 682-723), float64,
+ * bohr: [A 1; 1^T 0] [q; mu] = [x; Q], A_ij = erf(gamma_ij r_ij) / r_ij, gamma_ij =
+ * (rad_i^2 + rad_j^2)^(-1/2), A_ii = diag_i, for the structures ids (n_ids, nullable:
+ * 0 .. n_ids - 1) of node_ptr; max_atoms bounds their sizes; total (B, nullable: 0) their
+ * charges Q. q (N) of other structures is not written. *info (device, set to 0 by the
+ * caller) gets bit 0 for a pivot that is exactly zero. */
+int xnn_eeq_molecules(const double* pos, int64_t n_nodes, const int64_t* node_ptr,
+                      const int32_t* ids, int64_t n_ids, int64_t max_atoms, const double* rad,
+                      const double* diag, const double* x, const double* total, double* q,
+                      int32_t* info, xnn_stream_t stream);
+/* Gradients of sum_i g_q[i] q[i] in the positions (N,3) and x (N). */
+int xnn_eeq_molecules_backward(const double* pos, int64_t n_nodes, const int64_t* node_ptr,
+                               const int32_t* ids, int64_t n_ids, int64_t max_atoms,
+                               const double* rad, const double* diag, const double* q,
+                               const double* g_q, double* grad_pos, double* grad_x, int32_t* info,
+                               xnn_stream_t stream);
+
 /* The real-space matrix of the conjugate-gradient regime kept packed in 128 x 128 tiles,
  * for sizes whose pairs in reach fit the memory (8.2 bytes each, an unordered pair once).
  * All device memory, nt = ceil(N / 128). */

@@ -212,6 +212,8 @@ _SIGNATURES = {
     "xnn_eeq_real_grad": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp],
     "xnn_eeq_cholesky_block": [vp, i64, i64, i64, vp, vp, vp],
     "xnn_eeq_cholesky_solve": [vp, i64, vp, vp, i32, vp, vp],
+    "xnn_eeq_molecules": [vp, i64, vp, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp],
+    "xnn_eeq_molecules_backward": [vp, i64, vp, vp, i64, i64, vp, vp, vp, vp, vp, vp, vp, vp],
     "xnn_eeq_store_meet": [vp, i64, vp, dbl, vp, vp],
     "xnn_eeq_store_tiles": [vp, i64, vp, vp, dbl, dbl, ctypes.POINTER(EeqTiles), vp, vp, vp],
     "xnn_eeq_store_apply_work_size": [i64, i32, ctypes.POINTER(ctypes.c_size_t)],

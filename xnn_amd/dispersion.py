@@ -835,6 +835,48 @@ class DFTD4(nn.Module):
                                        device=pos_au.device)])
         return torch.linalg.solve(M, rhs[:, None])[:n, 0]
 
+    def _batch_charges(self, zc: Tensor, pos: Tensor, cell64: Optional[Tensor], cn_eeq: Tensor,
+                       counts: List[int], periodic: List[bool], total_charge: Optional[Tensor],
+                       node_ptr: Tensor) -> Tensor:
+        """EEQ charges (N,) of a batch: the dense regime's molecules that fit the batched kernel
+        in one launch (:func:`~xnn_amd.eeq.molecule_charges_op`), every other structure by
+        :meth:`charges`."""
+        from .eeq import MOLECULE_MAX_ATOMS, molecule_charges_op
+        B, dev = len(counts), pos.device
+        totals = [0.0] * B if total_charge is None else \
+            [float(v) for v in total_charge.reshape(-1).tolist()]
+        if len(totals) < B:
+            raise IndexError(f"{len(totals)} total charges for {B} structures")
+        small = [b for b, n in enumerate(counts)
+                 if 0 < n <= MOLECULE_MAX_ATOMS and not periodic[b]
+                 and self.select_regime(n, False) == "dense"
+                 and not (self.eeq_rad.requires_grad or self.eeq_eta.requires_grad)]
+        q_small = None
+        if small:
+            rad = self.eeq_rad[zc]
+            x = -self.eeq_chi[zc] + self.eeq_kcnchi[zc] * cn_eeq / torch.sqrt(cn_eeq + EEQ_CN_REG)
+            whole = len(small) == B
+            ids = None if whole else torch.tensor(small, dtype=torch.int32, device=dev)
+            total = (pos.new_zeros(B) if total_charge is None
+                     else torch.tensor(totals[:B], dtype=torch.float64, device=dev))
+            q_small, info = molecule_charges_op(
+                (pos / BOHR).contiguous(), x.contiguous(), rad, self.eeq_eta[zc] + math.sqrt(2.0 / math.pi) / rad,
+                total, node_ptr, ids, len(small), max(counts[b] for b in small))
+            if not torch.cuda.is_current_stream_capturing() and int(info):
+                raise torch.linalg.LinAlgError("the EEQ matrix of a molecule is singular")
+            if whole:
+                return q_small
+        qs, s0, batched = [], 0, set(small)
+        for b, n in enumerate(counts):
+            if b in batched:
+                qs.append(q_small[s0:s0 + n])
+            else:
+                cell_b = cell64[b] / BOHR if (cell64 is not None and periodic[b]) else None
+                qs.append(self.charges(zc[s0:s0 + n], pos[s0:s0 + n] / BOHR, cn_eeq[s0:s0 + n],
+                                       totals[b], cell_b))
+            s0 += n
+        return torch.cat(qs) if qs else pos.new_zeros(0)
+
     def _coulomb_molecular(self, z, pos):
         n = pos.shape[0]
         rad = self.eeq_rad[z]
@@ -953,15 +995,11 @@ class DFTD4(nn.Module):
                                      self.rcov, self.en, [cut_cn, cut_eeq], max_atoms)
         periodic = None  # host flags per structure, read only where needed (a synchronization)
         if charges is None:
-            periodic = [bool(x) for x in (images != 0).any(1).cpu()]
+            periodic = ([False] * B if cell64 is None
+                        else [bool(x) for x in (images != 0).any(1).cpu()])
             cn_eeq = math.log(1.0 + math.exp(EEQ_CN_MAX)) - torch.log(1.0 + torch.exp(EEQ_CN_MAX - raw))
-            qs = []
-            for b in range(B):
-                s0, s1 = sum(n_atoms_h[:b]), sum(n_atoms_h[:b + 1])
-                qt = 0.0 if total_charge is None else float(total_charge.reshape(-1)[b])
-                cell_b = cell64[b] / BOHR if (cell64 is not None and periodic[b]) else None
-                qs.append(self.charges(zc[s0:s1], pos[s0:s1] / BOHR, cn_eeq[s0:s1], qt, cell_b))
-            q = torch.cat(qs) if qs else pos.new_zeros(0)
+            q = self._batch_charges(zc, pos, cell64, cn_eeq, n_atoms_h, periodic, total_charge,
+                                    node_ptr)
         else:
             q = charges.to(dev, torch.float64)
         alpha = self.polarizabilities(zc, cn, q).contiguous()

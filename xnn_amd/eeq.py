@@ -289,6 +289,58 @@ def _real_apply_backward(ctx, grad):
 real_apply_op.register_autograd(_real_apply_backward, setup_context=_real_apply_setup)
 
 
+# --------------------------------------------------------------------------- molecules (HIP)
+#: atoms of a molecule up to which the dense charges of a batch are solved in one launch: its
+#: bordered matrix fits a compute unit's LDS. 32 molecules of 21 atoms, energy and forces: 2.3 ms
+#: against 24 ms with a library solve per molecule
+MOLECULE_MAX_ATOMS = 128
+
+
+@torch.library.custom_op(f"{_NS}::eeq_molecules", mutates_args=())
+def molecule_charges_op(pos: Tensor, x: Tensor, rad: Tensor, diag: Tensor, total: Tensor,
+                        node_ptr: Tensor, ids: Optional[Tensor], n_ids: int,
+                        max_atoms: int) -> Tuple[Tensor, Tensor]:
+    """Dense EEQ charges (N,) of the molecules ``ids`` (int32; None: the first ``n_ids``) of a
+    batch, zero elsewhere, and a flag (1,) that is not zero where a pivot was (d4.py:593-606,
+    682-723): positions in bohr, ``diag = J + sqrt(2/pi) / a``, ``total`` (B,) the charges;
+    differentiable once in ``pos`` and ``x``."""
+    q = torch.zeros_like(x)
+    info = torch.zeros(1, dtype=torch.int32, device=x.device)
+    _lib.call("xnn_eeq_molecules", _lib.ptr(pos), int(x.shape[0]), _lib.ptr(node_ptr), _lib.ptr(ids),
+              n_ids, max_atoms, _lib.ptr(rad), _lib.ptr(diag), _lib.ptr(x), _lib.ptr(total),
+              _lib.ptr(q), _lib.ptr(info), _lib.stream(x.device))
+    return q, info
+
+
+@molecule_charges_op.register_fake
+def _(pos, x, rad, diag, total, node_ptr, ids, n_ids, max_atoms):
+    return x.new_empty(x.shape), x.new_empty(1, dtype=torch.int32)
+
+
+def _molecules_setup(ctx, inputs, output):
+    pos, x, rad, diag, total, node_ptr, ids, n_ids, max_atoms = inputs
+    ctx.save_for_backward(pos, rad, diag, node_ptr, ids, output[0])
+    ctx.n_ids, ctx.max_atoms = n_ids, max_atoms
+
+
+def _molecules_backward(ctx, g_q, _g_info):
+    if torch.is_grad_enabled():
+        raise RuntimeError("the batched EEQ charges are differentiable once")
+    pos, rad, diag, node_ptr, ids, q = ctx.saved_tensors
+    if any(ctx.needs_input_grad[2:5]):
+        raise NotImplementedError("eeq_molecules differentiates positions and x only")
+    grad_pos, grad_x = torch.zeros_like(pos), torch.zeros_like(q)
+    info = torch.zeros(1, dtype=torch.int32, device=q.device)
+    _lib.call("xnn_eeq_molecules_backward", _lib.ptr(pos), int(q.shape[0]), _lib.ptr(node_ptr),
+              _lib.ptr(ids), ctx.n_ids, ctx.max_atoms, _lib.ptr(rad), _lib.ptr(diag), _lib.ptr(q),
+              _lib.ptr(g_q.contiguous()), _lib.ptr(grad_pos), _lib.ptr(grad_x), _lib.ptr(info),
+              _lib.stream(q.device))
+    return grad_pos, grad_x, None, None, None, None, None, None, None
+
+
+molecule_charges_op.register_autograd(_molecules_backward, setup_context=_molecules_setup)
+
+
 # --------------------------------------------------------------------------- the system
 class LargeEEQSystem:
     """The EEQ operator of one structure at fixed (detached) geometry, assembled densely and
