@@ -679,6 +679,13 @@ int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_
 int xnn_eeq_cholesky_block(double* matrix, int64_t n, int64_t k0, int64_t b, double* inv,
                            int* info, xnn_stream_t stream);
 
+/* The whole factorization: every diagonal block as above, each followed by its panel and
+ * the trailing matrix's lower part. matrix: the lower triangle in place (above the diagonal
+ * the entries are unspecified); inv_blocks: 128 * 128 * ceil(n / 128) doubles, as
+ * xnn_eeq_cholesky_solve takes them; *info (device) is 0 on entry. */
+int xnn_eeq_cholesky(double* matrix, int64_t n, double* inv_blocks, int* info,
+                     xnn_stream_t stream);
+
 /* (L L^T) X = B in place: X (n, nrhs) row-major float64 on entry B, nrhs 1 or 2; L the
  * factor that xnn_eeq_cholesky_block left in the matrix (row-major, lower), inv_blocks the
  * inverses of its diagonal blocks (block j of rows [128 j, 128 j + b_j) at inv_blocks +

@@ -745,12 +745,9 @@ def _add_gram(A: Tensor, X: Tensor, parts: int = GRAM_PARTS) -> None:
 
 def _cholesky(A: Tensor, keep_inverses: bool = False):
     """The Cholesky factor of the float64 operator and LAPACK's ``info`` (0, or the 1-based
-    column of the first pivot that is not positive). On the device: right-looking blocked
-    factorization, 128 columns at a time: ``xnn_eeq_cholesky_block`` factors the diagonal
-    block in LDS and forms its inverse, the panel below it is ``A21 L11^-T`` and the
-    trailing matrix takes ``- L21 L21^T`` (library GEMMs; a large trailing update is split
-    at half height into the top rows' left square and the bottom rows, 3/4 of the square,
-    and the upper triangle is discarded at the end). ``keep_inverses``: also return the
+    column of the first pivot that is not positive). On the device ``xnn_eeq_cholesky``: the
+    right-looking blocked factorization, 128 columns at a time, on the float64 matrix cores
+    (the upper triangle is discarded at the end). ``keep_inverses``: also return the
     diagonal blocks' inverses (block j at ``128 * 128 j``, row stride its size; None off
     the device) for :func:`_cholesky_solve`."""
     if not A.is_cuda:
@@ -761,25 +758,8 @@ def _cholesky(A: Tensor, keep_inverses: bool = False):
     info = torch.zeros(1, dtype=torch.int32, device=A.device)
     inv_all = torch.empty(max((n + nb - 1) // nb, 1) * nb * nb, dtype=torch.float64,
                           device=A.device)
-    panel = torch.empty((max(n - nb, 0), nb), dtype=torch.float64, device=A.device)
-    stream = _lib.stream(A.device)
-    for k in range(0, n, nb):
-        b = min(nb, n - k)
-        inv = inv_all[(k // nb) * nb * nb:]
-        _lib.call("xnn_eeq_cholesky_block", _lib.ptr(L), n, k, b, _lib.ptr(inv),
-                  _lib.ptr(info), stream)
-        r = k + b
-        if r < n:
-            p = panel[:n - r, :b]
-            torch.matmul(L[r:, k:r], inv[:b * b].view(b, b).t(), out=p)
-            L[r:, k:r].copy_(p)
-            m = n - r
-            if m >= 4 * nb:                # the lower part only: 3/4 of the square
-                h = (m // 2 + nb - 1) // nb * nb
-                L[r:r + h, r:r + h].addmm_(p[:h], p[:h].t(), alpha=-1.0)
-                L[r + h:, r:].addmm_(p[h:], p.t(), alpha=-1.0)
-            else:
-                L[r:, r:].addmm_(p, p.t(), alpha=-1.0)
+    _lib.call("xnn_eeq_cholesky", _lib.ptr(L), n, _lib.ptr(inv_all), _lib.ptr(info),
+              _lib.stream(A.device))
     return (L.tril_(), info[0], inv_all) if keep_inverses else (L.tril_(), info[0])
 
 
