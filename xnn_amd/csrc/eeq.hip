@@ -1113,14 +1113,23 @@ static int launch_cholesky_block(double* matrix, int64_t n, int64_t k0, int b, d
 // rows with the block's inverse (forward y = inv r, backward x = inv^T r; a 128 x 128
 // product, repeated per workgroup rather than waiting for one), workgroup 0 stores it,
 // and every row still to come takes away the block's contribution (forward: r_i -= L[i,
-// k0:k0 + b_k] y_k, a wave per row over its contiguous entries, 8 rows' loads in flight at
-// once; backward: r_i -= L[k0:k0 + b_k, i]^T x_k for i < k0, a thread per row, the block
-// row read across threads). The solution goes to another array than the residual rows
+// k0:k0 + b_k] y_k, 32 rows a workgroup; backward: r_i -= L[k0:k0 + b_k, i]^T x_k for i <
+// k0, 64 rows a workgroup). Everything a launch reads is loaded first, unconditionally (past
+// an edge the last valid entry, dropped by a select), so the chain of a launch is one memory
+// latency and the two products. The solution goes to another array than the residual rows
 // the launch reads (forward: residual in X, solution in the work array; backward the
 // reverse), so no workgroup reads a row another one rewrites. Sums in a fixed order.
+// 40 blocks of 5,000 rows: 7.5 us a forward and 6.4 us a backward launch of one column (8.5
+// and 6.4 of two), where loads behind bounds tests, one latency each, took 11.4 and 13.8.
 constexpr int kTrsvBlock = kCholBlock;
-constexpr int kTrsvFwdRows = 32;      // rows per workgroup (forward)
-constexpr int kTrsvBwdRows = 256;     // rows per workgroup (backward)
+constexpr int kTrsvThreads = 512;
+constexpr int kTrsvGroups = kTrsvThreads / kTrsvBlock;    // 4 threads per row or column of a block
+constexpr int kTrsvPer = kTrsvBlock / kTrsvGroups;        // entries each of them takes
+constexpr int kTrsvFwdRows = 32;      // rows per workgroup (forward): four a wave
+constexpr int kTrsvBwdRows = 64;      // rows per workgroup (backward)
+constexpr int kTrsvWaves = kTrsvThreads / kWave;
+constexpr int kTrsvFwdBatch = kTrsvFwdRows / kTrsvWaves;  // rows of L a wave takes (forward)
+constexpr int kTrsvBwdBatch = kTrsvBlock / kTrsvWaves;    // and rows of the block (backward)
 
 __device__ __forceinline__ double wave_sum_xor(double v) {
 #pragma unroll
@@ -1128,105 +1137,170 @@ __device__ __forceinline__ double wave_sum_xor(double v) {
   return v;
 }
 
-// out = inv rb (TRANS: inv^T rb) over one block of size b <= 128 with its lower-triangular
-// inverse (row stride b), rb and out in LDS: two threads per entry, each over half of the
-// columns (the loads independent of the sums, so they are in flight together), the halves
-// added by one exchange.
-template <int NRHS, bool TRANS>
-__device__ __forceinline__ void trsv_block_inverse(const double* __restrict__ ib, int b,
-                                                   const double (*rb)[NRHS],
-                                                   double (*out)[NRHS]) {
-  const int t = threadIdx.x, i = t >> 1, h = t & 1;
-  const int ii = i < b ? i : 0;
-  double s[NRHS];
-#pragma unroll
-  for (int r = 0; r < NRHS; ++r) s[r] = 0.0;
-#pragma unroll 16
-  for (int q = 0; q < kTrsvBlock / 2; ++q) {
-    const int c = h * (kTrsvBlock / 2) + q;
-    // forward: inv[i][c], c <= i; backward: inv[c][i], c >= i
-    const bool use = c < b && (TRANS ? c >= ii : c <= ii);
-    const double l = use ? (TRANS ? ib[(int64_t)c * b + ii] : ib[(int64_t)ii * b + c]) : 0.0;
-#pragma unroll
-    for (int r = 0; r < NRHS; ++r) s[r] = fma(l, rb[use ? c : 0][r], s[r]);
-  }
-#pragma unroll
-  for (int r = 0; r < NRHS; ++r) s[r] += __shfl_xor(s[r], 1, kWave);
-  if (h == 0 && i < b) {
-#pragma unroll
-    for (int r = 0; r < NRHS; ++r) out[i][r] = s[r];
-  }
-}
-
-template <int NRHS, bool TRANS>
-__global__ __launch_bounds__(256) void eeq_trsv_step_kernel(const double* __restrict__ L,
-                                                            int64_t n,
-                                                            const double* __restrict__ inv,
-                                                            int k, double* __restrict__ res,
-                                                            double* __restrict__ sol) {
-  __shared__ double rs[kTrsvBlock][NRHS];     // block k's residual
-  __shared__ double xs[kTrsvBlock][NRHS];     // its solution
+template <int NRHS>
+__global__ __launch_bounds__(kTrsvThreads) void eeq_trsv_forward_kernel(
+    const double* __restrict__ L, int64_t n, const double* __restrict__ inv, int k,
+    double* __restrict__ res, double* __restrict__ sol) {
+  extern __shared__ double trsv_lds[];                    // the inverse, rows of 129
+  __shared__ double rs[kTrsvBlock][NRHS];                 // block k's residual
+  __shared__ double xs[kTrsvBlock][NRHS];                 // its solution
+  constexpr int kLd = kTrsvBlock + 1;
   const int t = threadIdx.x, lane = t & (kWave - 1), wv = t >> 6;
   const int64_t k0 = (int64_t)k * kTrsvBlock;
   const int bk = (int)(n - k0 < kTrsvBlock ? n - k0 : kTrsvBlock);
-  for (int i = t; i < bk * NRHS; i += blockDim.x) (&rs[0][0])[i] = res[k0 * NRHS + i];
+  const double* ib = inv + (int64_t)k * kTrsvBlock * kTrsvBlock;
+  const int g = t / kTrsvBlock, c = t % kTrsvBlock;
+  double m[kTrsvPer], v0[kTrsvFwdBatch], v1[kTrsvFwdBatch], old[kTrsvFwdBatch][NRHS], r0[NRHS];
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) r0[r] = res[(k0 + min(c, bk - 1)) * NRHS + r];
+#pragma unroll
+  for (int q = 0; q < kTrsvPer; ++q)
+    m[q] = ib[min(kTrsvGroups * q + g, bk - 1) * bk + min(c, bk - 1)];
+  const int64_t i0 = k0 + bk + (int64_t)blockIdx.x * kTrsvFwdRows + wv * kTrsvFwdBatch;
+#pragma unroll
+  for (int q = 0; q < kTrsvFwdBatch; ++q) {
+    const int64_t i = min(i0 + q, n - 1);
+    v0[q] = L[i * n + k0 + min(lane, bk - 1)];
+    v1[q] = L[i * n + k0 + min(lane + kWave, bk - 1)];
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) old[q][r] = res[i * NRHS + r];
+  }
+  if (g == 0) {
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) rs[c][r] = c < bk ? r0[r] : 0.0;
+  }
+#pragma unroll
+  for (int q = 0; q < kTrsvPer; ++q) trsv_lds[(kTrsvGroups * q + g) * kLd + c] = m[q];
   __syncthreads();
-  trsv_block_inverse<NRHS, TRANS>(inv + (int64_t)k * kTrsvBlock * kTrsvBlock, bk, rs, xs);
-  __syncthreads();
-  if (blockIdx.x == 0)
-    for (int i = t; i < bk * NRHS; i += blockDim.x) sol[k0 * NRHS + i] = (&xs[0][0])[i];
-  if (!TRANS) {
-    // rows after the block, kTrsvFwdRows per workgroup; a wave takes 8 rows at a time
-    constexpr int kBatch = 8;
-    const int64_t r0 = k0 + bk + (int64_t)blockIdx.x * kTrsvFwdRows;
-    const int64_t r1 = r0 + kTrsvFwdRows < n ? r0 + kTrsvFwdRows : n;
-    const int ca = lane < bk ? lane : 0, cb = lane + kWave < bk ? lane + kWave : 0;
-    for (int64_t base = r0 + (int64_t)wv * kBatch; base < r1;
-         base += (int64_t)(blockDim.x / kWave) * kBatch) {
-      double v0[kBatch], v1[kBatch], old[kBatch][NRHS];
+  {  // four threads an entry, over entries h, h + 4, ...
+    const int i = t / kTrsvGroups, h = t % kTrsvGroups;
+    double s[NRHS];
 #pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int64_t i = base + q;
-        const bool ok = i < r1;
-        const double* row = L + (ok ? i : k0) * n + k0;
-        v0[q] = ok && lane < bk ? row[lane] : 0.0;
-        v1[q] = ok && lane + kWave < bk ? row[lane + kWave] : 0.0;
+    for (int r = 0; r < NRHS; ++r) s[r] = 0.0;
 #pragma unroll
-        for (int r = 0; r < NRHS; ++r) old[q][r] = ok ? res[i * NRHS + r] : 0.0;
-      }
+    for (int q = 0; q < kTrsvPer; ++q) {
+      const int cc = kTrsvGroups * q + h;
+      const double l = cc <= i ? trsv_lds[i * kLd + cc] : 0.0;
 #pragma unroll
-      for (int q = 0; q < kBatch; ++q) {
-        const int64_t i = base + q;
-        if (i >= r1) break;                       // uniform in the wave
-#pragma unroll
-        for (int r = 0; r < NRHS; ++r) {
-          const double sr = wave_sum_xor(fma(v0[q], xs[ca][r], v1[q] * xs[cb][r]));
-          if (lane == 0) res[i * NRHS + r] = old[q][r] - sr;
-        }
-      }
+      for (int r = 0; r < NRHS; ++r) s[r] = fma(l, rs[cc][r], s[r]);
     }
-  } else {
-    // rows before the block, kTrsvBwdRows per workgroup, a thread per row
-    const int64_t r0 = (int64_t)blockIdx.x * kTrsvBwdRows;
-    const int64_t r1 = r0 + kTrsvBwdRows < k0 ? r0 + kTrsvBwdRows : k0;
-    for (int64_t i = r0 + t; i < r1; i += blockDim.x) {
-      double s[NRHS], old[NRHS];
 #pragma unroll
-      for (int r = 0; r < NRHS; ++r) {
-        s[r] = 0.0;
-        old[r] = res[i * NRHS + r];
-      }
-#pragma unroll 16
-      for (int c = 0; c < kTrsvBlock; ++c) {
-        const bool use = c < bk;
-        const double l = use ? L[(k0 + c) * n + i] : 0.0;
-#pragma unroll
-        for (int r = 0; r < NRHS; ++r) s[r] = fma(l, xs[use ? c : 0][r], s[r]);
-      }
-#pragma unroll
-      for (int r = 0; r < NRHS; ++r) res[i * NRHS + r] = old[r] - s[r];
+    for (int r = 0; r < NRHS; ++r) {
+      s[r] += __shfl_xor(s[r], 1, kWave);
+      s[r] += __shfl_xor(s[r], 2, kWave);
+      if (h == 0) xs[i][r] = i < bk ? s[r] : 0.0;
     }
   }
+  __syncthreads();
+  if (blockIdx.x == 0)
+    for (int i = t; i < bk * NRHS; i += kTrsvThreads) sol[k0 * NRHS + i] = (&xs[0][0])[i];
+#pragma unroll
+  for (int q = 0; q < kTrsvFwdBatch; ++q) {
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) {
+      const double a = lane < bk ? v0[q] * xs[lane][r] : 0.0;
+      const double sr = wave_sum_xor(lane + kWave < bk ? fma(v1[q], xs[lane + kWave][r], a) : a);
+      if (lane == 0 && i0 + q < n) res[(i0 + q) * NRHS + r] = old[q][r] - sr;
+    }
+  }
+}
+
+template <int NRHS>
+__global__ __launch_bounds__(kTrsvThreads) void eeq_trsv_backward_kernel(
+    const double* __restrict__ L, int64_t n, const double* __restrict__ inv, int k,
+    double* __restrict__ res, double* __restrict__ sol) {
+  __shared__ double rs[kTrsvBlock][NRHS];                 // block k's residual
+  __shared__ double xs[kTrsvBlock][NRHS];                 // its solution
+  __shared__ double part[kTrsvGroups][kTrsvBlock][NRHS];
+  __shared__ double upd[kTrsvWaves][kTrsvBwdRows][NRHS];
+  const int t = threadIdx.x, lane = t & (kWave - 1), wv = t >> 6;
+  const int64_t k0 = (int64_t)k * kTrsvBlock;
+  const int bk = (int)(n - k0 < kTrsvBlock ? n - k0 : kTrsvBlock);
+  const double* ib = inv + (int64_t)k * kTrsvBlock * kTrsvBlock;
+  const int g = t / kTrsvBlock, c = t % kTrsvBlock;
+  double m[kTrsvPer], l[kTrsvBwdBatch], old[NRHS], r0[NRHS];
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) r0[r] = res[(k0 + min(c, bk - 1)) * NRHS + r];
+#pragma unroll
+  for (int q = 0; q < kTrsvPer; ++q)
+    m[q] = ib[min(kTrsvGroups * q + g, bk - 1) * bk + min(c, bk - 1)];
+  const int64_t i = (int64_t)blockIdx.x * kTrsvBwdRows + lane;   // < k0 or past the rows
+  const int64_t ic = min(i, n - 1);
+#pragma unroll
+  for (int q = 0; q < kTrsvBwdBatch; ++q)
+    l[q] = L[(k0 + min(wv * kTrsvBwdBatch + q, bk - 1)) * n + ic];
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) old[r] = res[ic * NRHS + r];
+  if (g == 0) {
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) rs[c][r] = c < bk ? r0[r] : 0.0;
+  }
+  __syncthreads();
+  double s[NRHS];
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) s[r] = 0.0;
+#pragma unroll
+  for (int q = 0; q < kTrsvPer; ++q) {                    // rows below or at the entry's own
+    const int row = kTrsvGroups * q + g;
+    const double e = row >= c && row < bk ? m[q] : 0.0;
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) s[r] = fma(e, rs[row][r], s[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) part[g][c][r] = s[r];
+  __syncthreads();
+  for (int e = t; e < kTrsvBlock * NRHS; e += kTrsvThreads) {
+    double x = 0.0;
+#pragma unroll
+    for (int h = 0; h < kTrsvGroups; ++h) x += (&part[h][0][0])[e];
+    (&xs[0][0])[e] = e < bk * NRHS ? x : 0.0;
+    if (blockIdx.x == 0 && e < bk * NRHS) sol[k0 * NRHS + e] = x;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) s[r] = 0.0;
+#pragma unroll
+  for (int q = 0; q < kTrsvBwdBatch; ++q) {
+    const int row = wv * kTrsvBwdBatch + q;
+    const double e = row < bk ? l[q] : 0.0;
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) s[r] = fma(e, xs[row][r], s[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < NRHS; ++r) upd[wv][lane][r] = s[r];
+  __syncthreads();
+  if (wv == 0 && i < k0) {
+#pragma unroll
+    for (int r = 0; r < NRHS; ++r) {
+      double x = 0.0;
+#pragma unroll
+      for (int h = 0; h < kTrsvWaves; ++h) x += upd[h][lane][r];
+      res[i * NRHS + r] = old[r] - x;
+    }
+  }
+}
+
+template <int NRHS>
+static int launch_trsv(const double* factor, int64_t n, const double* inv_blocks, double* x,
+                       double* work, hipStream_t s) {
+  const int nb = (int)((n + kTrsvBlock - 1) / kTrsvBlock);
+  constexpr size_t lds = sizeof(double) * kTrsvBlock * (kTrsvBlock + 1);
+  const auto fwd = eeq_trsv_forward_kernel<NRHS>;
+  XNN_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void*>(fwd),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  for (int k = 0; k < nb; ++k) {          // forward: residual in x, solution into work
+    const int64_t after = n - std::min<int64_t>(n, (int64_t)(k + 1) * kTrsvBlock);
+    const unsigned grid = (unsigned)std::max<int64_t>(1, (after + kTrsvFwdRows - 1) / kTrsvFwdRows);
+    hipLaunchKernelGGL(fwd, dim3(grid), dim3(kTrsvThreads), lds, s, factor, n, inv_blocks, k, x, work);
+  }
+  for (int k = nb - 1; k >= 0; --k) {     // backward: residual in work, solution into x
+    const int64_t before = (int64_t)k * kTrsvBlock;
+    const unsigned grid = (unsigned)std::max<int64_t>(1, (before + kTrsvBwdRows - 1) / kTrsvBwdRows);
+    hipLaunchKernelGGL(eeq_trsv_backward_kernel<NRHS>, dim3(grid), dim3(kTrsvThreads), 0, s, factor, n,
+                       inv_blocks, k, work, x);
+  }
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
 }
 
 }  // namespace xnn
@@ -1429,30 +1503,8 @@ int xnn_eeq_cholesky_solve(const double* factor, int64_t n, const double* inv_bl
   if (n == 0) return XNN_OK;
   XNN_REQUIRE(factor && inv_blocks && x && work, "NULL factor, inverses, right-hand side or work");
   XNN_REQUIRE(n <= (int64_t(1) << 20), "at most 2^20 rows");
-  const int nb = (int)((n + kTrsvBlock - 1) / kTrsvBlock);
-  hipStream_t s = as_hip(stream);
-  for (int k = 0; k < nb; ++k) {          // forward: residual in x, solution into work
-    const int64_t after = n - std::min<int64_t>(n, (int64_t)(k + 1) * kTrsvBlock);
-    const unsigned grid = (unsigned)std::max<int64_t>(1, (after + kTrsvFwdRows - 1) / kTrsvFwdRows);
-    if (nrhs == 1)
-      hipLaunchKernelGGL((eeq_trsv_step_kernel<1, false>), dim3(grid), dim3(256), 0, s, factor, n,
-                         inv_blocks, k, x, work);
-    else
-      hipLaunchKernelGGL((eeq_trsv_step_kernel<2, false>), dim3(grid), dim3(256), 0, s, factor, n,
-                         inv_blocks, k, x, work);
-  }
-  for (int k = nb - 1; k >= 0; --k) {     // backward: residual in work, solution into x
-    const int64_t before = (int64_t)k * kTrsvBlock;
-    const unsigned grid = (unsigned)std::max<int64_t>(1, (before + kTrsvBwdRows - 1) / kTrsvBwdRows);
-    if (nrhs == 1)
-      hipLaunchKernelGGL((eeq_trsv_step_kernel<1, true>), dim3(grid), dim3(256), 0, s, factor, n,
-                         inv_blocks, k, work, x);
-    else
-      hipLaunchKernelGGL((eeq_trsv_step_kernel<2, true>), dim3(grid), dim3(256), 0, s, factor, n,
-                         inv_blocks, k, work, x);
-  }
-  XNN_LAUNCH_CHECK();
-  return XNN_OK;
+  return nrhs == 1 ? launch_trsv<1>(factor, n, inv_blocks, x, work, as_hip(stream))
+                   : launch_trsv<2>(factor, n, inv_blocks, x, work, as_hip(stream));
 }
 
 int xnn_eeq_cholesky(double* matrix, int64_t n, double* inv_blocks, int* info,
