@@ -667,6 +667,23 @@ int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_
                         const double* v, int32_t nrhs, double* out, void* work, size_t work_bytes,
                         xnn_stream_t stream);
 
+/* The reciprocal part of the Ewald product at n_vectors half-set vectors g (M, 3) with
+ * weights w (M): out_i = sum_k w_k [cos(g_k r_i) Sc_k + sin(g_k r_i) Ss_k], the structure
+ * factors Sc_k, Ss_k = sum_j v_j (cos, sin)(g_k r_j) written to factors (2, M) for the
+ * backward (the torch sums of common/models/eeq.py:170-397, without their (N, M) phases).
+ * All device float64. The backward takes the output's gradient u (N) and writes grad_pos
+ * (N, 3) and, where not NULL, grad_g (M, 3) with grad_w (M), and grad_v (N). work: as many
+ * bytes as the size query gives. Nothing is written when n_nodes or n_vectors is 0. Sums in
+ * a fixed order. */
+int xnn_eeq_recip_work_size(int64_t n_nodes, int64_t n_vectors, int32_t backward, size_t* bytes);
+int xnn_eeq_recip(const double* pos, int64_t n_nodes, const double* g, const double* w,
+                  int64_t n_vectors, const double* v, double* factors, double* out, void* work,
+                  size_t work_bytes, xnn_stream_t stream);
+int xnn_eeq_recip_backward(const double* pos, int64_t n_nodes, const double* g, const double* w,
+                           int64_t n_vectors, const double* v, const double* factors,
+                           const double* u, double* grad_pos, double* grad_g, double* grad_w,
+                           double* grad_v, void* work, size_t work_bytes, xnn_stream_t stream);
+
 /* One diagonal block of the blocked Cholesky factorization of the assembled operator
  * (replaces the factorization of EEQSystem._solve_lu, common/models/eeq.py:312-323, which
  * LU-factors the augmented matrix; the operator is symmetric positive definite and the

@@ -210,6 +210,9 @@ _SIGNATURES = {
     "xnn_segment_reduce_noalloc_max_bytes": [],
     "xnn_eeq_real_matrix": [vp, i64, vp, vp, dbl, dbl, vp, vp],
     "xnn_eeq_real_grad": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp],
+    "xnn_eeq_recip_work_size": [i64, i64, i32, vp],
+    "xnn_eeq_recip": [vp, i64, vp, vp, i64, vp, vp, vp, vp, sz, vp],
+    "xnn_eeq_recip_backward": [vp, i64, vp, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp],
     "xnn_eeq_cholesky": [vp, i64, vp, vp, vp],
     "xnn_eeq_cholesky_block": [vp, i64, i64, i64, vp, vp, vp],
     "xnn_eeq_cholesky_solve": [vp, i64, vp, vp, i32, vp, vp],

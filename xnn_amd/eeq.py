@@ -115,7 +115,11 @@ def reciprocal_apply(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tensor:
     """``A_rec v = C diag(w) C^T v + S diag(w) S^T v`` with ``C, S = cos, sin(pos G^T)``,
     over blocks of reciprocal vectors of at most :data:`LIVE_BUDGET` phases each; a block
     that carries gradients is recomputed in the backward instead of kept (memory
-    ``O(LIVE_BUDGET)`` at any size)."""
+    ``O(LIVE_BUDGET)`` at any size). One vector ``v`` in float64 on the GPU goes through
+    :func:`reciprocal_op`, which keeps no phases: 5,000 atoms and their forces 0.15 ms
+    against 1.6 ms."""
+    if pos.is_cuda and v.dim() == 1 and all(t.dtype == torch.float64 for t in (pos, g, w, v)):
+        return reciprocal_op(pos.contiguous(), g.contiguous(), w.contiguous(), v.contiguous())[0]
     n = max(int(pos.shape[0]), 1)
     step = max(1, LIVE_BUDGET // n)
     if g.shape[0] <= step:
@@ -131,6 +135,58 @@ def reciprocal_apply(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tensor:
             part = _reciprocal_block(*args)
         out = part if out is None else out + part
     return out
+
+
+@torch.library.custom_op(f"{_NS}::eeq_reciprocal", mutates_args=())
+def reciprocal_op(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tuple[Tensor, Tensor]:
+    """:func:`reciprocal_apply` (N,) without its phases and the structure factors (2, M) of
+    ``v`` (``xnn_eeq_recip``, HIP)."""
+    n, m = int(pos.shape[0]), int(g.shape[0])
+    out = pos.new_zeros(n) if m == 0 else pos.new_empty(n)
+    factors = pos.new_zeros((2, m)) if n == 0 else pos.new_empty((2, m))
+    work = _recip_work(n, m, False, pos.device)
+    _lib.call("xnn_eeq_recip", _lib.ptr(pos), n, _lib.ptr(g), _lib.ptr(w), m, _lib.ptr(v),
+              _lib.ptr(factors), _lib.ptr(out), _lib.ptr(work), int(work.numel()),
+              _lib.stream(pos.device))
+    return out, factors
+
+
+def _recip_work(n: int, m: int, backward: bool, device) -> Tensor:
+    need = ctypes.c_size_t(0)
+    _lib.call("xnn_eeq_recip_work_size", n, m, int(backward), ctypes.byref(need))
+    return torch.empty(need.value, dtype=torch.uint8, device=device)
+
+
+@reciprocal_op.register_fake
+def _(pos, g, w, v):
+    return pos.new_empty(pos.shape[0]), pos.new_empty((2, g.shape[0]))
+
+
+def _reciprocal_setup(ctx, inputs, output):
+    ctx.save_for_backward(*inputs, output[1])
+    ctx.mark_non_differentiable(output[1])
+
+
+def _reciprocal_backward(ctx, u, _factors):
+    pos, g, w, v, factors = ctx.saved_tensors
+    if torch.is_grad_enabled():        # a gradient of the gradient: through the tensor form
+        out = _reciprocal_block(pos, g, w, v)
+        wanted = [t for t, need in zip((pos, g, w, v), ctx.needs_input_grad) if need]
+        grads = iter(torch.autograd.grad([out], wanted, [u], create_graph=True))
+        return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
+    n, m = int(pos.shape[0]), int(g.shape[0])
+    cell_side = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
+    grad_pos, grad_v = torch.zeros_like(pos), torch.zeros_like(v)
+    grad_g, grad_w = (torch.zeros_like(g), torch.zeros_like(w)) if cell_side else (None, None)
+    work = _recip_work(n, m, True, pos.device)
+    _lib.call("xnn_eeq_recip_backward", _lib.ptr(pos), n, _lib.ptr(g), _lib.ptr(w), m, _lib.ptr(v),
+              _lib.ptr(factors), _lib.ptr(u.contiguous()), _lib.ptr(grad_pos), _lib.ptr(grad_g),
+              _lib.ptr(grad_w), _lib.ptr(grad_v), _lib.ptr(work), int(work.numel()),
+              _lib.stream(pos.device))
+    return grad_pos, grad_g, grad_w, grad_v
+
+
+reciprocal_op.register_autograd(_reciprocal_backward, setup_context=_reciprocal_setup)
 
 
 # --------------------------------------------------------------------------- real space (HIP)
