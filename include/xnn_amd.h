@@ -206,6 +206,17 @@ int xnn_sh_linear_message_sum_backward(int geom_dtype, const float* vec_in, cons
                                        const float* d_out, float* d_h, float* g_vec,
                                        xnn_stream_t stream);
 
+/* The gradient of W (n_features, n_channels) of the same sum for the rows' cotangent d_out
+ * (N, C, L), 16-byte aligned, from given edge vectors: d_W = h^T d_phi without phi or d_phi
+ * (zeros without edges). work: the queried bytes. */
+int xnn_sh_linear_message_wgrad_work_size(int64_t n_nodes, int32_t n_features,
+                                          int32_t n_channels, size_t* bytes);
+int xnn_sh_linear_message_wgrad(const float* vec, int64_t n_nodes, int64_t n_edges,
+                                const int32_t* ptr_dst, const int32_t* perm_dst, int32_t l_max,
+                                int32_t sh_sign, int32_t n_features, int32_t n_channels,
+                                const float* h, const float* d_out, float* d_W, void* work,
+                                size_t work_bytes, xnn_stream_t stream);
+
 /* Featurizer, edge-weight linear layer and aggregation in one kernel: h is the
  * enveloped radial basis of the edge length, h[e,k] = rbf_k(|r_e|) envelope(|r_e|)
  * (SphericalHarmonicEdgeEmbedding.forward, gnn/featurizers/spherical.py:135-138, whose
@@ -1010,6 +1021,12 @@ int xnn_node_readout(int dtype, const void* rows, int64_t n_rows, int64_t n_feat
 int xnn_node_readout_backward(int dtype, const void* g, int64_t g_stride, int64_t n_rows,
                               int64_t n_features, const void* weights, void* d_rows,
                               xnn_stream_t stream);
+/* d_weights[f] = sum_i g[i * g_stride] rows[i, f], summed in float64 (zeros without rows);
+ * work: the queried bytes. */
+int xnn_node_readout_wgrad_work_size(int64_t n_rows, int64_t n_features, size_t* bytes);
+int xnn_node_readout_wgrad(int dtype, const void* rows, int64_t n_rows, int64_t n_features,
+                           const void* g, int64_t g_stride, void* d_weights, void* work,
+                           size_t work_bytes, xnn_stream_t stream);
 
 /* ------------------------------------------------------------------------ */
 /* Axilrod-Teller-Muto three-body dispersion (D4 and D3) over an edge list. Edges

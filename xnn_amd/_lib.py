@@ -126,6 +126,8 @@ _SIGNATURES = {
                                   i32, i32, vp, vp, vp, vp],
     "xnn_sh_linear_message_sum_backward": [c_int, vp, vp, i64, vp, i64, vp, vp, vp, i64, vp, vp,
                                            i32, i32, i32, i32, vp, vp, vp, vp, vp, vp],
+    "xnn_sh_linear_message_wgrad_work_size": [i64, i32, i32, vp],
+    "xnn_sh_linear_message_wgrad": [vp, i64, i64, vp, vp, i32, i32, i32, i32, vp, vp, vp, vp, sz, vp],
     "xnn_sh_radial_message_sum": [c_int, vp, vp, i64, vp, i64, vp, vp, vp, i64, vp, vp,
                                   ctypes.POINTER(FeaturizeParams), vp, i32, vp, vp, vp],
     "xnn_sh_radial_message_sum_backward": [c_int, vp, vp, i64, vp, i64, vp, vp, vp, i64, vp, vp,
@@ -181,6 +183,8 @@ _SIGNATURES = {
                                         ctypes.POINTER(AtmParams), vp, vp, vp, vp, vp, vp, vp,
                                         vp, vp, sz, vp],
     "xnn_node_readout_backward": [i32, vp, i64, i64, i64, vp, vp, vp],
+    "xnn_node_readout_wgrad_work_size": [i64, i64, vp],
+    "xnn_node_readout_wgrad": [i32, vp, i64, i64, vp, i64, vp, vp, sz, vp],
     "xnn_d4_polarizabilities": [i64, vp, vp, vp, ctypes.POINTER(D4AlphaTables), vp, vp],
     "xnn_d4_polarizabilities_backward": [i64, vp, vp, vp, ctypes.POINTER(D4AlphaTables), vp, vp,
                                          vp, vp],

@@ -41,6 +41,7 @@ differentiable once; a double backward through them (force training with
 """
 from __future__ import annotations
 
+import ctypes
 from typing import List, Optional, Tuple
 
 import torch
@@ -549,6 +550,13 @@ LINEAR_MESSAGE_CHANNELS = (32, 64, 128)
 LINEAR_MESSAGE_MAX_FEATURES = 8
 
 
+def _work(query: str, device, *sizes) -> Tensor:
+    """A workspace of the size that the library's ``query`` gives."""
+    need = ctypes.c_size_t(0)
+    _lib.call(query, *sizes, ctypes.byref(need))
+    return torch.empty(need.value, dtype=torch.uint8, device=device)
+
+
 @torch.library.custom_op(f"{_NS}::sh_linear_message_sum", mutates_args=())
 def sh_linear_message_sum_op(vec: Tensor, h: Tensor, W: Tensor, ptr_dst: Tensor,
                              perm_dst: Optional[Tensor], l_max: int, sh_sign: int) -> Tensor:
@@ -593,14 +601,12 @@ def _lin_msg_backward(ctx, d_out):
                   _lib.ptr(d_out), _lib.ptr(d_h), _lib.ptr(g_vec), _lib.stream(dev))
     d_W = None
     if need_W:
-        # d_W = h^T d_phi needs d_phi itself: one pass of the unfused backward forms it
-        phi = h @ W
-        d_phi = torch.empty_like(phi)
-        _lib.call("xnn_sh_message_sum_backward", _lib.XNN_F32, _lib.ptr(vec), None, n_nodes, None,
-                  0, None, None, None, vec.shape[0], _lib.ptr(ptr_dst), _lib.ptr(perm_dst),
-                  ctx.l_max, ctx.sh_sign, C, _lib.ptr(phi), _lib.ptr(d_out), _lib.ptr(d_phi),
-                  None, _lib.stream(dev))
-        d_W = h.t() @ d_phi
+        d_W = torch.empty_like(W)
+        work = _work("xnn_sh_linear_message_wgrad_work_size", dev, n_nodes, K, C)
+        _lib.call("xnn_sh_linear_message_wgrad", _lib.ptr(vec), n_nodes, vec.shape[0],
+                  _lib.ptr(ptr_dst), _lib.ptr(perm_dst), ctx.l_max, ctx.sh_sign, K, C, _lib.ptr(h),
+                  _lib.ptr(d_out), _lib.ptr(d_W), _lib.ptr(work), int(work.numel()),
+                  _lib.stream(dev))
     return g_vec, (d_h if need_h else None), d_W, None, None, None, None
 
 
@@ -969,6 +975,20 @@ def _readout_setup(ctx, inputs, output):
     ctx.n_bias, ctx.bias_dtype, ctx.weight_dtype = bias.shape[0], bias.dtype, weight.dtype
 
 
+def _readout_weight_grad(rows: Tensor, grad: Tensor) -> Tensor:
+    if rows.dtype != grad.dtype:
+        return rows.t() @ grad
+    F = rows.shape[1]
+    rows = rows.contiguous()
+    g = grad if (grad.dim() == 1 and grad.stride(0) == 0) else grad.contiguous()
+    out = torch.empty(F, dtype=rows.dtype, device=rows.device)
+    work = _work("xnn_node_readout_wgrad_work_size", rows.device, rows.shape[0], F)
+    _lib.call("xnn_node_readout_wgrad", _lib.dtype_code(rows.dtype), _lib.ptr(rows), rows.shape[0], F,
+              _lib.ptr(g), 0 if g.stride(0) == 0 else 1, _lib.ptr(out), _lib.ptr(work),
+              int(work.numel()), _lib.stream(rows.device))
+    return out
+
+
 def _readout_backward(ctx, grad):
     _once_differentiable()
     rows, weight, z = ctx.saved_tensors
@@ -984,7 +1004,7 @@ def _readout_backward(ctx, grad):
                   0 if g.stride(0) == 0 else 1, n, F, _lib.ptr(w), _lib.ptr(d_rows),
                   _lib.stream(grad.device))
     if ctx.needs_input_grad[1]:
-        d_weight = (rows.t() @ grad).to(ctx.weight_dtype)
+        d_weight = _readout_weight_grad(rows, grad).to(ctx.weight_dtype)
     if ctx.needs_input_grad[3]:
         d_bias = torch.zeros(ctx.n_bias, dtype=grad.dtype, device=grad.device).index_add_(
             0, z, grad).to(ctx.bias_dtype)
