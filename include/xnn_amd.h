@@ -678,6 +678,36 @@ int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_
                         const double* v, int32_t nrhs, double* out, void* work, size_t work_bytes,
                         xnn_stream_t stream);
 
+/* The vector work of the conjugate-gradient solves of the large EEQ regime (eeq.py:325-360),
+ * all device float64, nrhs 1 or 2 columns, row-major.
+ * spread: vp (n_rows, 2 K nrhs) = [pr v, pi v] of the phase tables pr, pi (N, K = n_phases)
+ * and v (N, nrhs), rows past n_nodes zero. fold: the partial products part (chunks, 2 C,
+ * 2 K nrhs) summed and weighted by weights (C, K) into out (2 C, 2 K nrhs) = [[gr, gi], [gi,
+ * -gr]]. gather: out (N, nrhs) += sum_k pr y_re + pi y_im + diag v with y (N, 2 K nrhs).
+ * step: a = rz / p.ap, x += a p, res -= a ap, z = inv_d res. project: t (n_low, nrhs) = U^T z,
+ * U (N, n_low <= 2048), work the queried bytes. search: z -= inv_d U t (U NULL: not), p = z + (res.z / rz) p (first: p = z), new_state = (res.z, |res| <= tol as 0 or 1); state and
+ * new_state are 2 nrhs doubles each, a column whose state says done takes a = 0 and p = z.
+ * sums: 512 nrhs doubles, the same for a step and the search after it. */
+int xnn_eeq_cg_spread(const double* pr, const double* pi, const double* v, int64_t n_nodes,
+                      int64_t n_rows, int32_t n_phases, int32_t nrhs, double* vp,
+                      xnn_stream_t stream);
+int xnn_eeq_cg_fold(const double* part, int64_t chunks, int64_t n_columns, int32_t n_phases,
+                    int32_t nrhs, const double* weights, double* out, xnn_stream_t stream);
+int xnn_eeq_cg_gather(const double* pr, const double* pi, const double* y, const double* diag,
+                      const double* v, int64_t n_nodes, int32_t n_phases, int32_t nrhs, double* out,
+                      xnn_stream_t stream);
+int xnn_eeq_cg_step(const double* p, const double* ap, const double* inv_d, const double* state,
+                    int64_t n_nodes, int32_t nrhs, double* x, double* res, double* z, double* sums,
+                    xnn_stream_t stream);
+int xnn_eeq_cg_project_work_size(int64_t n_nodes, int32_t n_low, int32_t nrhs, size_t* bytes);
+int xnn_eeq_cg_project(const double* U, const double* z, int64_t n_nodes, int32_t n_low,
+                       int32_t nrhs, double* t, void* work, size_t work_bytes,
+                       xnn_stream_t stream);
+int xnn_eeq_cg_search(const double* U, const double* t, int32_t n_low, const double* inv_d,
+                      const double* res, const double* tol, const double* state, int32_t first,
+                      int64_t n_nodes, int32_t nrhs, double* z, double* p, double* new_state,
+                      double* sums, xnn_stream_t stream);
+
 /* The reciprocal part of the Ewald product at n_vectors half-set vectors g (M, 3) with
  * weights w (M): out_i = sum_k w_k [cos(g_k r_i) Sc_k + sin(g_k r_i) Ss_k], the structure
  * factors Sc_k, Ss_k = sum_j v_j (cos, sin)(g_k r_j) written to factors (2, M) for the

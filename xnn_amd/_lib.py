@@ -214,6 +214,13 @@ _SIGNATURES = {
     "xnn_segment_reduce_noalloc_max_bytes": [],
     "xnn_eeq_real_matrix": [vp, i64, vp, vp, dbl, dbl, vp, vp],
     "xnn_eeq_real_grad": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp],
+    "xnn_eeq_cg_spread": [vp, vp, vp, i64, i64, i32, i32, vp, vp],
+    "xnn_eeq_cg_fold": [vp, i64, i64, i32, i32, vp, vp, vp],
+    "xnn_eeq_cg_gather": [vp, vp, vp, vp, vp, i64, i32, i32, vp, vp],
+    "xnn_eeq_cg_step": [vp, vp, vp, vp, i64, i32, vp, vp, vp, vp, vp],
+    "xnn_eeq_cg_project_work_size": [i64, i32, i32, vp],
+    "xnn_eeq_cg_project": [vp, vp, i64, i32, i32, vp, vp, sz, vp],
+    "xnn_eeq_cg_search": [vp, vp, i32, vp, vp, vp, vp, i32, i64, i32, vp, vp, vp, vp, vp],
     "xnn_eeq_recip_work_size": [i64, i64, i32, vp],
     "xnn_eeq_recip": [vp, i64, vp, vp, i64, vp, vp, vp, vp, sz, vp],
     "xnn_eeq_recip_backward": [vp, i64, vp, vp, i64, vp, vp, vp, vp, vp, vp, vp, vp, sz, vp],

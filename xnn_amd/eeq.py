@@ -526,7 +526,21 @@ def own_image_diagonal(cell: Tensor, rad: Tensor, alpha: float, cutoff_au: float
     return k.sum(1)
 
 
-def _tn_product(b: Tensor, v: Tensor, chunks: int = 32) -> Tensor:
+#: row chunks of :func:`_tn_product`
+TN_CHUNKS = 32
+
+
+def _tn_partials(b: Tensor, v: Tensor) -> Tensor:
+    """The partial products of ``b^T v`` over :data:`TN_CHUNKS` row chunks (one chunk for a
+    short reduction), for rows that they divide."""
+    n = int(b.shape[0])
+    if n < 256 * TN_CHUNKS:
+        return (b.t() @ v)[None]
+    m = n // TN_CHUNKS
+    return torch.bmm(b.view(TN_CHUNKS, m, -1).transpose(1, 2), v.view(TN_CHUNKS, m, -1))
+
+
+def _tn_product(b: Tensor, v: Tensor, chunks: int = TN_CHUNKS) -> Tensor:
     """``b^T v`` for tall ``b`` (N, P) and ``v`` (N, Q) with a long reduction over N: split
     into ``chunks`` batched products that are summed afterwards (one library GEMM of a small
     output would run on a handful of workgroups)."""
@@ -574,6 +588,8 @@ class FactorizedReciprocal:
         self.W = W
         self.n = int(f.shape[0])
         self.diagonal = float(w.sum())     # A_rec,ii = sum_G w_G
+        # on the device the products' row count is a multiple of the chunks (zero rows after)
+        self.rows = -(-self.n // TN_CHUNKS) * TN_CHUNKS if f.is_cuda else self.n
         self.block = max(1, TABLE_BUDGET // max(2 * self.n, 1))
         self.table = self._columns(0, self.C) if self.C <= self.block else None
 
@@ -581,7 +597,37 @@ class FactorizedReciprocal:
         (ar, ai), (br, bi) = self.tables[0], self.tables[1]
         ar, ai = ar[:, self.c1[c0:c1]], ai[:, self.c1[c0:c1]]
         br, bi = br[:, self.c2[c0:c1]], bi[:, self.c2[c0:c1]]
-        return torch.cat([ar * br - ai * bi, ar * bi + ai * br], 1)
+        if self.rows == self.n:
+            return torch.cat([ar * br - ai * bi, ar * bi + ai * br], 1)
+        out = ar.new_zeros((self.rows, 2 * (c1 - c0)))
+        out[:self.n, :c1 - c0] = ar * br - ai * bi
+        out[:self.n, c1 - c0:] = ar * bi + ai * br
+        return out
+
+    def add_to(self, out: Tensor, v: Tensor, diag: Tensor) -> Tensor:
+        """``out += A_rec v + diag v`` on the device, ``v`` (N, 1 or 2): per block of columns
+        two library products, and one launch before, between and after them."""
+        n, R = v.shape
+        v = v.contiguous()
+        K, stream = self.K, _lib.stream(v.device)
+        pr, pi = self.tables[2]
+        vp = v.new_empty((self.rows, 2 * K * R))
+        _lib.call("xnn_eeq_cg_spread", _lib.ptr(pr), _lib.ptr(pi), _lib.ptr(v), n, self.rows, K, R,
+                  _lib.ptr(vp), stream)
+        y = None
+        for c0 in range(0, self.C, self.block):
+            c1 = min(self.C, c0 + self.block)
+            b = self.table if self.table is not None else self._columns(c0, c1)
+            part = _tn_partials(b, vp)
+            g = v.new_empty((2 * (c1 - c0), 2 * K * R))
+            _lib.call("xnn_eeq_cg_fold", _lib.ptr(part), part.shape[0], c1 - c0, K, R,
+                      _lib.ptr(self.W[c0:c1]), _lib.ptr(g), stream)
+            y = b @ g if y is None else y.addmm_(b, g)
+        if y is None:                          # no reciprocal vector within the range
+            return out.addcmul_(diag[:, None], v)
+        _lib.call("xnn_eeq_cg_gather", _lib.ptr(pr), _lib.ptr(pi), _lib.ptr(y), _lib.ptr(diag),
+                  _lib.ptr(v), n, K, R, _lib.ptr(out), stream)
+        return out
 
     def apply(self, v: Tensor) -> Tensor:
         """``A_rec v`` for ``v`` (N, R)."""
@@ -703,34 +749,52 @@ class IterativeEEQSystem:
                 self._work = torch.empty(need.value, dtype=torch.uint8, device=v.device)
             out = real_apply(self.pos_s, self.cell_host, self.rad_s, self.alpha, self.cutoff, v,
                              self.tiles, self._work)
-        out += self.diag_s[:, None] * v
         if self.recip is not None:
-            out += self.recip.apply(v)
-        return out
+            return self.recip.add_to(out, v, self.diag_s)
+        return out.addcmul_(self.diag_s[:, None], v)
 
     def conjugate_gradient(self, b: Tensor, tol_abs: Tensor) -> Tensor:
         """``A^-1 b`` for the columns of ``b`` (N, 1 or 2) in the spatial order, each column
         to ``|r| <= tol_abs`` (a column that meets it is frozen while the other runs)."""
+        n, R = b.shape
+        stream = _lib.stream(b.device)
         x = self.precondition(b)
         r = b - self._matvec(x)
-        z = self.precondition(r)
-        p = z.clone()
-        rz = (r * z).sum(0)
+        z = self.inv_d[:, None] * r
+        p = torch.empty_like(r)
+        state, new_state = b.new_empty(2 * R), b.new_empty(2 * R)
+        sums = b.new_empty(512 * R)
+        tol_abs = tol_abs.to(torch.float64).contiguous()
+        low = 0 if self.U is None else int(self.U.shape[1])
+        if low:
+            need = ctypes.c_size_t(0)
+            _lib.call("xnn_eeq_cg_project_work_size", n, low, R, ctypes.byref(need))
+            work = torch.empty(need.value, dtype=torch.uint8, device=b.device)
+            t = b.new_empty((low, R))
+
+        def search(first: bool):
+            c = None
+            if low:
+                _lib.call("xnn_eeq_cg_project", _lib.ptr(self.U), _lib.ptr(z), n, low, R, _lib.ptr(t),
+                          _lib.ptr(work), int(work.numel()), stream)
+                c = self.core_inv @ t
+            _lib.call("xnn_eeq_cg_search", _lib.ptr(self.U), _lib.ptr(c), low, _lib.ptr(self.inv_d),
+                      _lib.ptr(r), _lib.ptr(tol_abs), _lib.ptr(state), int(first), n, R, _lib.ptr(z),
+                      _lib.ptr(p), _lib.ptr(new_state), _lib.ptr(sums), stream)
+
+        search(True)
         for it in range(self.maxiter + 1):
-            done = torch.linalg.vector_norm(r, dim=0) <= tol_abs
-            if bool(done.all()):
+            state, new_state = new_state, state
+            if all(state[R:].tolist()):
                 self.iterations.append(it)
                 return x
             if it == self.maxiter:
                 break
             ap = self._matvec(p)
-            a = torch.where(done, torch.zeros_like(rz), rz / (p * ap).sum(0))
-            x += a * p
-            r -= a * ap
-            z = self.precondition(r)
-            rz_new = (r * z).sum(0)
-            p = z + torch.where(done, torch.zeros_like(rz), rz_new / rz) * p
-            rz = rz_new
+            _lib.call("xnn_eeq_cg_step", _lib.ptr(p), _lib.ptr(ap), _lib.ptr(self.inv_d),
+                      _lib.ptr(state), n, R, _lib.ptr(x), _lib.ptr(r), _lib.ptr(z), _lib.ptr(sums),
+                      stream)
+            search(False)
         res = torch.linalg.vector_norm(r, dim=0) / torch.linalg.vector_norm(b, dim=0)
         raise RuntimeError(f"EEQ conjugate gradients did not converge in {self.maxiter} "
                            f"iterations (relative residuals {res.tolist()})")
