@@ -611,6 +611,15 @@ int xnn_eeq_real_grad(const double* pos, int64_t n_nodes, const double* cell, co
                       double alpha, double cutoff, const double* u, const double* w,
                       double* grad_pos, double* cell_partial, xnn_stream_t stream);
 
+/* The same derivatives over unordered pairs, every pair evaluated once, the cell's summed
+ * into grad_cell (9; NULL: not wanted). work: the queried bytes; the query gives 0 above
+ * 56,000 atoms, which xnn_eeq_real_grad takes. */
+int xnn_eeq_real_grad_pairs_work_size(int64_t n_nodes, size_t* bytes);
+int xnn_eeq_real_grad_pairs(const double* pos, int64_t n_nodes, const double* cell,
+                            const double* rad, double alpha, double cutoff, const double* u,
+                            const double* w, double* grad_pos, double* grad_cell, void* work,
+                            size_t work_bytes, xnn_stream_t stream);
+
 /* Bytes of the workspace of xnn_eeq_real_apply for n_nodes atoms and nrhs (1 or 2)
  * right-hand sides. */
 int xnn_eeq_real_apply_work_size(int64_t n_nodes, int32_t nrhs, size_t* bytes);

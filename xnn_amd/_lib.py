@@ -214,6 +214,8 @@ _SIGNATURES = {
     "xnn_segment_reduce_noalloc_max_bytes": [],
     "xnn_eeq_real_matrix": [vp, i64, vp, vp, dbl, dbl, vp, vp],
     "xnn_eeq_real_grad": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp],
+    "xnn_eeq_real_grad_pairs_work_size": [i64, vp],
+    "xnn_eeq_real_grad_pairs": [vp, i64, vp, vp, dbl, dbl, vp, vp, vp, vp, vp, sz, vp],
     "xnn_eeq_cg_spread": [vp, vp, vp, i64, i64, i32, i32, vp, vp],
     "xnn_eeq_cg_fold": [vp, i64, i64, i32, i32, vp, vp, vp],
     "xnn_eeq_cg_gather": [vp, vp, vp, vp, vp, i64, i32, i32, vp, vp],

@@ -202,6 +202,119 @@ __global__ __launch_bounds__(256) void eeq_real_grad_kernel(
   }
 }
 
+// The same derivatives over unordered pairs: the lower 64 x 64 tiles, a block a tile, four
+// waves of sixteen rows i each, lanes over the columns j. A pair's term goes to its column in
+// the lane's registers (the waves' shares added through LDS) and to its row by a butterfly over
+// the wave; both are written per tile, part[slot][atom], slots 0 .. T: an atom of tile I gets
+// its rows from tiles (I, J), slot J, its columns from (I', I), slot I', those of its own tile
+// in slot T; eeq_real_grad_sum_kernel adds the slots in order. The cell's sum is a row of nine
+// per block. For the far pairs (gamma r >= 7, where gamma's terms are below 1e-21) one error
+// function and one exponential remain, and 1/r is a refined estimate instead of three divisions.
+// 5,000 atoms, 2.7 images a pair: 0.93 ms, where the directed kernel takes 2.07.
+constexpr int kGradTile = 64;
+// part is (T + 1) x 3 N doubles, 1.2 GB at the most; beyond that the directed kernel
+constexpr int64_t kGradMaxAtoms = 56000;
+
+__global__ __launch_bounds__(256) void eeq_real_grad_tiles_kernel(
+    const double* __restrict__ pos, int64_t n, EeqCell C, const double* __restrict__ rad,
+    double alpha, double cut2, const double* __restrict__ u, const double* __restrict__ w,
+    int64_t n_tiles, bool want_cell, double* __restrict__ part, double* __restrict__ cell_rows) {
+  __shared__ double sg[4][3][kGradTile], sc[4][9];
+  const int lane = threadIdx.x & (kWave - 1), wv = threadIdx.x / kWave;
+  const int64_t b = blockIdx.x;
+  int64_t ti = (int64_t)((sqrt(8.0 * (double)b + 1.0) - 1.0) * 0.5);
+  while (ti * (ti + 1) / 2 > b) --ti;
+  while ((ti + 1) * (ti + 2) / 2 <= b) ++ti;
+  const int64_t tj = b - ti * (ti + 1) / 2;
+  const int64_t j = tj * kGradTile + lane, jc = min(j, n - 1);
+  const double xj = pos[3 * jc], yj = pos[3 * jc + 1], zj = pos[3 * jc + 2];
+  const double aj = rad[jc], uj = u[jc], wj = w[jc];
+  double g[3] = {0.0, 0.0, 0.0}, c[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  constexpr double two_over_sqrt_pi = 1.1283791670955126;
+  for (int q = 0; q < kGradTile / 4; ++q) {
+    const int64_t i = ti * kGradTile + wv * (kGradTile / 4) + q;
+    if (i >= n) break;                                    // uniform in the wave
+    double f[3] = {0.0, 0.0, 0.0};
+    if (j <= i && j < n) {
+      const double ai = rad[i], gam = rsq_nr(fma(ai, ai, aj * aj));
+      const double sym = j == i ? u[i] * w[i] : u[i] * wj + uj * w[i];
+      for_images(C, xj - pos[3 * i], yj - pos[3 * i + 1], zj - pos[3 * i + 2], cut2, j == i,
+                 [&](double dx, double dy, double dz, int n0, int n1, int n2) {
+                   const double r2 = dx * dx + dy * dy + dz * dz, ir = rsq_nr(r2);
+                   const double x = gam * (r2 * ir);
+                   double e = x < 7.0 ? gam * exp(-x * x) : 0.0;
+                   if (alpha > 0.0) e -= alpha * exp(-(alpha * alpha) * r2);
+                   const double K = screened_inv(r2, ir, gam, alpha);
+                   const double s = sym * ((two_over_sqrt_pi * e - K) * ir) * ir;
+                   const double px = s * dx, py = s * dy, pz = s * dz;
+                   f[0] += px;
+                   f[1] += py;
+                   f[2] += pz;
+                   if (want_cell) {
+                     c[0] = fma(n0, px, c[0]); c[1] = fma(n0, py, c[1]); c[2] = fma(n0, pz, c[2]);
+                     c[3] = fma(n1, px, c[3]); c[4] = fma(n1, py, c[4]); c[5] = fma(n1, pz, c[5]);
+                     c[6] = fma(n2, px, c[6]); c[7] = fma(n2, py, c[7]); c[8] = fma(n2, pz, c[8]);
+                   }
+                 });
+      if (j == i) f[0] = f[1] = f[2] = 0.0;               // an atom and its images: no force
+    }
+#pragma unroll
+    for (int a = 0; a < 3; ++a) g[a] += f[a];
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) f[a] += __shfl_xor(f[a], m, kWave);
+    if (lane == 0)
+#pragma unroll
+      for (int a = 0; a < 3; ++a) part[(tj * n + i) * 3 + a] = -f[a];
+  }
+#pragma unroll
+  for (int a = 0; a < 3; ++a) sg[wv][a][lane] = g[a];
+  if (want_cell) {
+#pragma unroll
+    for (int m = kWave / 2; m > 0; m >>= 1)
+#pragma unroll
+      for (int q = 0; q < 9; ++q) c[q] += __shfl_xor(c[q], m, kWave);
+    if (lane == 0)
+#pragma unroll
+      for (int q = 0; q < 9; ++q) sc[wv][q] = c[q];
+  }
+  __syncthreads();
+  if (wv < 3 && j < n)                                    // wave a: component a
+    part[((ti == tj ? n_tiles : ti) * n + j) * 3 + wv] =
+        (sg[0][wv][lane] + sg[1][wv][lane]) + (sg[2][wv][lane] + sg[3][wv][lane]);
+  if (want_cell && wv == 3 && lane < 9)
+    cell_rows[b * 9 + lane] = (sc[0][lane] + sc[1][lane]) + (sc[2][lane] + sc[3][lane]);
+}
+
+__global__ __launch_bounds__(256) void eeq_real_grad_sum_kernel(const double* __restrict__ part,
+                                                                int64_t slots, int64_t m,
+                                                                double* __restrict__ out) {
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e >= m) return;
+  double s = 0.0;
+#pragma unroll 8
+  for (int64_t q = 0; q < slots; ++q) s += part[q * m + e];
+  out[e] = s;
+}
+
+// out[q] = the sum of rows[b][q], a block per component, strided shares added in order
+__global__ __launch_bounds__(256) void eeq_cell_sum_kernel(const double* __restrict__ rows,
+                                                           int64_t n_rows, double* __restrict__ out) {
+  __shared__ double s[256];
+  double v = 0.0;
+#pragma unroll 4
+  for (int64_t b = threadIdx.x; b < n_rows; b += 256) v += rows[b * 9 + blockIdx.x];
+  s[threadIdx.x] = v;
+  for (int m = 128; m > 0; m >>= 1) {
+    __syncthreads();
+    if ((int)threadIdx.x < m) s[threadIdx.x] += s[threadIdx.x + m];
+  }
+  if (threadIdx.x == 0) out[blockIdx.x] = s[0];
+}
+
+static int64_t grad_tiles(int64_t n) { return (n + kGradTile - 1) / kGradTile; }
+
 // ------------------------------------------------------------------ matrix-free product
 // out = R v for one or two right-hand sides (the conjugate-gradient regime): R is never
 // stored. Atoms come in tiles of kApplyTile consecutive indices; block (i tile, split)
@@ -1345,6 +1458,44 @@ int xnn_eeq_real_grad(const double* pos, int64_t n_nodes, const double* cell, co
   hipLaunchKernelGGL(eeq_real_grad_kernel, dim3((unsigned)grid_1d(n_nodes, 4)), dim3(256), 0,
                      as_hip(stream), pos, n_nodes, C, rad, alpha, cutoff * cutoff, u, w, grad_pos,
                      cell_partial);
+  XNN_LAUNCH_CHECK();
+  return XNN_OK;
+}
+
+int xnn_eeq_real_grad_pairs_work_size(int64_t n_nodes, size_t* bytes) {
+  XNN_REQUIRE(n_nodes >= 0 && bytes != nullptr, "negative size or NULL result");
+  const int64_t t = grad_tiles(n_nodes);
+  *bytes = n_nodes > kGradMaxAtoms
+               ? 0 : sizeof(double) * (size_t)((t + 1) * 3 * n_nodes + 9 * (t * (t + 1) / 2));
+  return XNN_OK;
+}
+
+int xnn_eeq_real_grad_pairs(const double* pos, int64_t n_nodes, const double* cell,
+                            const double* rad, double alpha, double cutoff, const double* u,
+                            const double* w, double* grad_pos, double* grad_cell, void* work,
+                            size_t work_bytes, xnn_stream_t stream) {
+  XNN_REQUIRE(n_nodes >= 1 && n_nodes <= kGradMaxAtoms, "1 to %lld atoms", (long long)kGradMaxAtoms);
+  XNN_REQUIRE(pos && rad && u && w && grad_pos && work, "NULL input, output or work");
+  XNN_REQUIRE(cutoff > 0.0 && alpha >= 0.0, "cutoff must be positive, alpha non-negative");
+  XNN_REQUIRE(cell != nullptr || (alpha == 0.0 && grad_cell == nullptr),
+              "a molecule takes alpha = 0 and has no cell gradient");
+  EeqCell C;
+  XNN_REQUIRE(eeq_cell(cell, cutoff, C), "singular cell");
+  XNN_REQUIRE(eeq_reach_ok(C, cutoff), "the real-space range spans more than %g cells",
+              kMaxReach);
+  size_t need = 0;
+  (void)xnn_eeq_real_grad_pairs_work_size(n_nodes, &need);
+  XNN_REQUIRE(work_bytes >= need, "work too small");
+  const int64_t t = grad_tiles(n_nodes), blocks = t * (t + 1) / 2;
+  double* part = static_cast<double*>(work);
+  double* rows = part + (t + 1) * 3 * n_nodes;
+  hipStream_t s = as_hip(stream);
+  hipLaunchKernelGGL(eeq_real_grad_tiles_kernel, dim3((unsigned)blocks), dim3(256), 0, s, pos, n_nodes,
+                     C, rad, alpha, cutoff * cutoff, u, w, t, grad_cell != nullptr, part, rows);
+  hipLaunchKernelGGL(eeq_real_grad_sum_kernel, dim3((unsigned)grid_1d(3 * n_nodes, 256)), dim3(256), 0, s,
+                     part, t + 1, 3 * n_nodes, grad_pos);
+  if (grad_cell != nullptr)
+    hipLaunchKernelGGL(eeq_cell_sum_kernel, dim3(9), dim3(256), 0, s, rows, blocks, grad_cell);
   XNN_LAUNCH_CHECK();
   return XNN_OK;
 }

@@ -332,13 +332,23 @@ def _real_apply_backward(ctx, grad):
     dev = pos.device
     grad_pos = torch.empty((n, 3), dtype=torch.float64, device=dev)
     want_cell = cell is not None and ctx.needs_input_grad[1]
-    part = torch.empty((n, 9), dtype=torch.float64, device=dev) if want_cell else None
-    _lib.call("xnn_eeq_real_grad", _lib.ptr(pos.detach().to(torch.float64).contiguous()), n,
-              _host_cell(cell), _lib.ptr(rad.detach().to(torch.float64).contiguous()), float(ctx.alpha),
-              float(ctx.cutoff), _lib.ptr(grad.to(torch.float64).contiguous()),
-              _lib.ptr(v.detach().to(torch.float64).contiguous()), _lib.ptr(grad_pos),
-              _lib.ptr(part), _lib.stream(dev))
-    g_cell = part.sum(0).reshape(3, 3).to(cell.dtype) if want_cell else None
+    p, a, u, w = (t.detach().to(torch.float64).contiguous() for t in (pos, rad, grad, v))
+    args = (_lib.ptr(p), n, _host_cell(cell), _lib.ptr(a), float(ctx.alpha), float(ctx.cutoff),
+            _lib.ptr(u), _lib.ptr(w), _lib.ptr(grad_pos))
+    g_cell = None
+    need = ctypes.c_size_t(0)
+    _lib.call("xnn_eeq_real_grad_pairs_work_size", n, ctypes.byref(need))
+    if need.value:
+        work = torch.empty(need.value, dtype=torch.uint8, device=dev)
+        g_cell = torch.empty(9, dtype=torch.float64, device=dev) if want_cell else None
+        _lib.call("xnn_eeq_real_grad_pairs", *args, _lib.ptr(g_cell), _lib.ptr(work),
+                  int(work.numel()), _lib.stream(dev))
+    else:
+        part = torch.empty((n, 9), dtype=torch.float64, device=dev) if want_cell else None
+        _lib.call("xnn_eeq_real_grad", *args, _lib.ptr(part), _lib.stream(dev))
+        g_cell = part.sum(0) if want_cell else None
+    if want_cell:
+        g_cell = g_cell.reshape(3, 3).to(cell.dtype)
     return grad_pos.to(pos.dtype), g_cell, None, None, None, None, None
 
 
