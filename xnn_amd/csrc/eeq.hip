@@ -768,10 +768,10 @@ __global__ __launch_bounds__(kMolThreads) void eeq_molecule_kernel(
     }
     __syncthreads();
     const double* pk = A + row[k] * ld;
-    const double inv = 1.0 / pk[k];
+    const double pivot = pk[k];
     for (int i = k + 1 + ty; i < m; i += kMolThreads / 32) {
       double* pi = A + row[i] * ld;
-      const double f = pi[k] * inv;
+      const double f = pi[k] / pivot;
       for (int j = k + 1 + tx; j <= m; j += 32) pi[j] = fma(-f, pk[j], pi[j]);
     }
     __syncthreads();
