@@ -19,6 +19,7 @@
 //   dS/dpos_k = -sum_{j,n} (u_k w_j + u_j w_k) K'(r) d / r,
 //   dS/dcell = sum_k sum_{j,n} u_k w_j K'(r) n (x) d / r   (per-atom rows, summed by the caller),
 // one wave per atom k, lanes over j, a fixed butterfly: bitwise reproducible.
+// xnn_eeq_real_grad_pairs forms the same over unordered pairs (up to 56,000 atoms).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -305,7 +305,7 @@ def real_apply_op(pos: Tensor, cell: Optional[Tensor], rad: Tensor, v: Tensor,
                   matrix: Optional[Tensor], alpha: float, cutoff_au: float) -> Tensor:
     """``R(pos, cell) v`` with the matrix formed at these positions, or without a matrix
     (``matrix`` None: the matrix-free HIP product); differentiable in ``pos`` and ``cell``
-    through ``xnn_eeq_real_grad`` (``v`` is held constant)."""
+    through ``xnn_eeq_real_grad_pairs`` (``v`` is held constant)."""
     if matrix is not None:
         return matrix @ v
     return real_apply(pos, cell, rad, alpha, cutoff_au, v.reshape(-1, 1)).reshape(v.shape)
@@ -841,7 +841,7 @@ class IterativeEEQSystem:
 
     def apply_live(self, pos: Tensor, cell: Optional[Tensor], v: Tensor) -> Tensor:
         """``A(pos, cell) v`` with derivatives in ``pos`` and ``cell`` (``v`` constant): the
-        matrix-free real-space product and the reciprocal sum in recomputed blocks."""
+        matrix-free real-space product and the reciprocal sum (:func:`reciprocal_apply`)."""
         out = self.diag * v + real_apply_op(pos, cell, self.rad, v, None, self.alpha, self.cutoff)
         if cell is not None:
             g, w = reciprocal_weights(self.m, cell, self.alpha)
