@@ -39,6 +39,7 @@ def test_reciprocal_product(n, R):
     eps = torch.finfo(torch.float64).eps
     scale = float(w.sum() * v.abs().sum() + base.abs().max())     # every phase at one
     torch.testing.assert_close(fr.add_to(base.clone(), v, diag), want, rtol=0, atol=64 * eps * scale)
+    torch.testing.assert_close(fr.apply(v) + base + diag[:, None] * v, want, rtol=0, atol=64 * eps * scale)
     fr.table, fr.block = None, 3              # column blocks formed as they are needed
     torch.testing.assert_close(fr.add_to(base.clone(), v, diag), want, rtol=0, atol=64 * eps * scale)
 

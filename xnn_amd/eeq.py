@@ -120,6 +120,11 @@ def reciprocal_apply(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tensor:
     against 1.6 ms."""
     if pos.is_cuda and v.dim() == 1 and all(t.dtype == torch.float64 for t in (pos, g, w, v)):
         return reciprocal_op(pos.contiguous(), g.contiguous(), w.contiguous(), v.contiguous())[0]
+    return _reciprocal_blocks(pos, g, w, v)
+
+
+def _reciprocal_blocks(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tensor:
+    """The tensor form of :func:`reciprocal_apply`."""
     n = max(int(pos.shape[0]), 1)
     step = max(1, LIVE_BUDGET // n)
     if g.shape[0] <= step:
@@ -170,7 +175,7 @@ def _reciprocal_setup(ctx, inputs, output):
 def _reciprocal_backward(ctx, u, _factors):
     pos, g, w, v, factors = ctx.saved_tensors
     if torch.is_grad_enabled():        # a gradient of the gradient: through the tensor form
-        out = _reciprocal_block(pos, g, w, v)
+        out = _reciprocal_blocks(pos, g, w, v)
         wanted = [t for t, need in zip((pos, g, w, v), ctx.needs_input_grad) if need]
         grads = iter(torch.autograd.grad([out], wanted, [u], create_graph=True))
         return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
@@ -651,7 +656,7 @@ class FactorizedReciprocal:
         for c0 in range(0, self.C, self.block):
             c1 = min(self.C, c0 + self.block)
             b = self.table if self.table is not None else self._columns(c0, c1)
-            cb = c1 - c0
+            b, cb = b[:n], c1 - c0
             x = _tn_product(b, vp)                           # (2 cb, 2 KR)
             sr = x[:cb, :KR] - x[cb:, KR:]
             si = x[:cb, KR:] + x[cb:, :KR]
