@@ -665,7 +665,7 @@ typedef struct xnn_eeq_tiles {
   const int32_t* index;   /* (nt, nt): a tile's place in the list or -1 (I >= J read) */
   uint64_t* mask;         /* (n_tiles, 128, 2): the stored columns of each half row */
   uint32_t* off;          /* (n_tiles, 128, 2): its first value within the tile */
-  const int64_t* base;    /* (n_tiles): the tile's first value */
+  const int64_t* base;    /* (n_tiles): the tile's first value (not read without one) */
 } xnn_eeq_tiles;
 
 /* flags (nt, nt) int32: 1 for the tiles (I >= J) with a lattice image within the cutoff;

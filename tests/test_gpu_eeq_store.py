@@ -36,6 +36,21 @@ def test_stored_tiles_match_the_formed_matrix(n, periodic):
         assert torch.equal(store.apply(v[:, cols].contiguous()), got)
 
 
+@pytest.mark.parametrize("n,periodic", [(129, False), (257, False), (1, False), (129, True)])
+def test_every_tile_starts_within_the_values(n, periodic):
+    """Also the last one where it is a single atom without an own image, which has none; a
+    range of 10 bohr in a cell of 20 for the periodic case."""
+    from xnn_amd import eeq as E
+    pos, cell, rad, _ = _system(n)
+    cutoff = 10.0 if periodic else float("inf")
+    alpha = E.ewald_alpha(cutoff) if periodic else 0.0
+    store = E.RealTiles.build(pos, E._host_cell(cell) if periodic else None, rad, alpha, cutoff)
+    base = store._keep[-1]
+    masks = store._keep[2].view(len(base), -1)
+    assert bool((masks[-1] == 0).all())          # the case meant
+    assert int(base.max()) < store.values.numel()
+
+
 def test_far_tiles_are_left_out_and_the_fallback_agrees(monkeypatch):
     """Two clusters out of each other's reach: their tiles are not stored; without room for
     the tiles the regime evaluates its pairs at every product, to the same charges."""

@@ -511,6 +511,8 @@ __global__ __launch_bounds__(256) void eeq_tiles_apply_kernel(
   const int my_off = (int)off[half_row];
   const int mask_lo = (int)(uint32_t)my_mask, mask_hi = (int)(uint32_t)(my_mask >> 32);
   const double* vals = values + base[id];
+  // a wave without values loads none: a tile without any may start at the end of them all
+  const bool any = __ballot(my_mask != 0) != 0;    // uniform in the wave
   for (int k = threadIdx.x; k < kStoreTile * NRHS; k += 256) {
     const int64_t at = I * kStoreTile * NRHS + k;
     sv[k] = at < n * NRHS ? v[at] : 0.0;
@@ -526,7 +528,9 @@ __global__ __launch_bounds__(256) void eeq_tiles_apply_kernel(
     }
   __syncthreads();
   double* out = part + id * (2 * kStoreTile * NRHS);
-  for (int b = 0; b < 32; b += kRows) {
+  if (!any)
+    for (int k = lane; k < 32 * NRHS; k += kWave) out[32 * w * NRHS + k] = 0.0;
+  for (int b = 0; any && b < 32; b += kRows) {
     double a[kRows][2];
 #pragma unroll
     for (int q = 0; q < kRows; ++q)
@@ -536,8 +540,8 @@ __global__ __launch_bounds__(256) void eeq_tiles_apply_kernel(
         const uint64_t m = (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mask_lo, k) |
                            (uint64_t)(uint32_t)__builtin_amdgcn_readlane(mask_hi, k) << 32;
         const int at = __builtin_amdgcn_readlane(my_off, k) + (int)lanes_below(m);
-        // every lane loads (an unset column the next value of the tile or, past its last
-        // one, its first), so that no load waits for a branch
+        // every lane loads (an unset column the tile's first value), so that no load waits
+        // for a branch
         const double x = vals[(m >> lane) & 1 ? at : 0];
         a[q][h] = (m >> lane) & 1 ? x : 0.0;
       }

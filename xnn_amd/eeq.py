@@ -285,7 +285,8 @@ class RealTiles:
             total = int(end[-1])
             if total * 8 > STORE_BYTES:
                 return None
-            values = torch.empty(max(total, 1), dtype=torch.float64, device=dev)
+            # one more: a tile without values starts at their end
+            values = torch.empty(total + 1, dtype=torch.float64, device=dev)
         except torch.cuda.OutOfMemoryError:
             return None
         tiles.base = _lib.ptr(base)
