@@ -66,6 +66,30 @@ def test_tiles_match_the_general_kernel(counts, periodic):
         s0 += n
 
 
+@pytest.mark.parametrize("counts", [[70], [5, 130]])
+@pytest.mark.parametrize("periodic", [True, False])
+def test_a_shift_of_all_atoms_changes_nothing(counts, periodic):
+    """A pair vector is rounded to its own length, wherever the structure lies: positions on a
+    grid of 2^-20 Angstrom, so that a shift by 2^20 Angstrom changes no difference of two."""
+    import xnn_amd.dispersion as XD
+    tables = XD.load_d3_tables(os.path.join(GOLDEN, "d3_tables_hcnoar.npz"))
+    z, pos, cell = _inputs(counts, periodic)
+    pos = np.round(pos * 2.0 ** 20) / 2.0 ** 20
+    model = XD.DFTD3(tables, cutoff_pair=11.0, cutoff_cn=9.0, switch_width_pair=1.5, s9=0.0).to(DEV)
+    results = []
+    for shift in (0.0, 2.0 ** 20):
+        p = torch.tensor(pos + shift, device=DEV, requires_grad=True)
+        c = None if cell is None else torch.tensor(cell, device=DEV, requires_grad=True)
+        pbc = None if cell is None else torch.ones((len(counts), 3), dtype=torch.bool)
+        out = model.evaluate(torch.tensor(z, device=DEV), p, c, pbc, torch.tensor(counts))
+        grads = torch.autograd.grad(out["energy"].sum(), [p] if c is None else [p, c])
+        results.append([out["coordination_numbers"].detach(), out["node_energy"].detach(), *grads])
+    energy = float(results[0][1].abs().max())
+    for a, b in zip(*results):
+        # the same terms in another order: sums of a few thousand, as above
+        torch.testing.assert_close(b, a, rtol=0, atol=2e-13 * (float(a.abs().max()) + energy))
+
+
 def test_an_unsymmetric_table_takes_the_general_kernel():
     import xnn_amd.dispersion as XD
     tables = dict(XD.load_d3_tables(os.path.join(GOLDEN, "d3_tables_hcnoar.npz")))

@@ -643,7 +643,8 @@ __device__ __forceinline__ void pair_tile(
   const int64_t pi = it.r0 + (live ? lane : 0);
   const int i = order[pi];
   const double xa = pos[3 * (int64_t)i], ya = pos[3 * (int64_t)i + 1], za = pos[3 * (int64_t)i + 2];
-  const double xb = xa * kInvBohr, yb = ya * kInvBohr, zb = za * kInvBohr;
+  const double scale = D3 ? 1.0 : kInvBohr;  // of the positions; D3 scales their difference
+  const double xb = xa * scale, yb = ya * scale, zb = za * scale;
   const int si = species[i];
   const double qi = r4r2[si], sq3qi = sqrt(3.0 * qi);
   const double gi = BACKWARD ? g_e2[i] : 0.0;
@@ -680,9 +681,9 @@ __device__ __forceinline__ void pair_tile(
     if (lane < it.scnt) {
     const int j = order[it.s0 + lane];
     const double xs = pos[3 * (int64_t)j], ys = pos[3 * (int64_t)j + 1], zs = pos[3 * (int64_t)j + 2];
-    st.u.s.x[lane] = xs * kInvBohr;
-    st.u.s.y[lane] = ys * kInvBohr;
-    st.u.s.z[lane] = zs * kInvBohr;
+    st.u.s.x[lane] = xs * scale;
+    st.u.s.y[lane] = ys * scale;
+    st.u.s.z[lane] = zs * scale;
     const double pj = r4r2[species[j]];
     st.u.s.p[lane] = pj;
     st.u.s.q[lane] = sqrt(pj);
@@ -754,7 +755,8 @@ __device__ __forceinline__ void pair_tile(
       const double r0 = prm.a1 * (sq3qi * st.u.s.q[jj]) + prm.a2;
       const double r02 = r0 * r0;
       const double r06 = r02 * r02 * r02, r08 = r06 * r02;
-      const double dx = xb - st.u.s.x[jj], dy = yb - st.u.s.y[jj], dz = zb - st.u.s.z[jj];
+      double dx = xb - st.u.s.x[jj], dy = yb - st.u.s.y[jj], dz = zb - st.u.s.z[jj];
+      if constexpr (D3) dx *= kInvBohr, dy *= kInvBohr, dz *= kInvBohr;
       // E = sum_i g_i e_i: the pair's energy enters with (g_i + g_j) (-1/2 C6 f); the
       // vector's gradient per Angstrom carries d r_bohr / d v = v_bohr / (r_bohr bohr)
       const double wsum = BACKWARD ? gi + st.w[jj] : 0.0;
@@ -951,7 +953,8 @@ __device__ __forceinline__ void cn_tile(
   const int64_t pi = it.r0 + (live ? lane : 0);
   const int i = order[pi];
   const double xa = pos[3 * (int64_t)i], ya = pos[3 * (int64_t)i + 1], za = pos[3 * (int64_t)i + 2];
-  const double xb = xa * kInvBohr, yb = ya * kInvBohr, zb = za * kInvBohr;
+  const double scale = D3 ? 1.0 : kInvBohr;  // of the positions; D3 scales their difference
+  const double xb = xa * scale, yb = ya * scale, zb = za * scale;
   const int si = species[i];
   const double rci = rcov[si], eni = D3 ? 0.0 : en[si];
   const double gi = BACKWARD && g_cn ? g_cn[i] : 0.0;
@@ -971,9 +974,9 @@ __device__ __forceinline__ void cn_tile(
       const int j = order[it.s0 + lane];
       const double xs = pos[3 * (int64_t)j], ys = pos[3 * (int64_t)j + 1],
                    zs = pos[3 * (int64_t)j + 2];
-      st.u.s.x[lane] = xs * kInvBohr;
-      st.u.s.y[lane] = ys * kInvBohr;
-      st.u.s.z[lane] = zs * kInvBohr;
+      st.u.s.x[lane] = xs * scale;
+      st.u.s.y[lane] = ys * scale;
+      st.u.s.z[lane] = zs * scale;
       const int sj = species[j];
       st.u.s.rc[lane] = rcov[sj];
       st.u.s.en[lane] = D3 ? 0.0 : en[sj];
@@ -1038,7 +1041,8 @@ __device__ __forceinline__ void cn_tile(
       // per pair: k0 / rc and the erf count's slope factor -k0 / (rc sqrt(pi))
       const double k_rc = D3 ? prm.kcn * rc : prm.kcn / rc;
       const double dk = -k_rc * kInvSqrtPi;
-      const double dx = xb - st.u.s.x[jj], dy = yb - st.u.s.y[jj], dz = zb - st.u.s.z[jj];
+      double dx = xb - st.u.s.x[jj], dy = yb - st.u.s.y[jj], dz = zb - st.u.s.z[jj];
+      if constexpr (D3) dx *= kInvBohr, dy *= kInvBohr, dz *= kInvBohr;
       const double wsum = BACKWARD ? gi + st.u.s.w[jj] : 0.0;
       const double w2sum = BACKWARD ? g2i + st.u.s.w2[jj] : 0.0;
       const double reach2 = D3 ? cmax2 : fmin(cmax2, rc * zfac * (rc * zfac));
