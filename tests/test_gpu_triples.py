@@ -57,3 +57,17 @@ def test_triple_vectors_match_the_tensor_form(case):
     torch.testing.assert_close(vec, ref_v, rtol=0, atol=8 * tol)
     for a, b in zip(got, torch.autograd.grad([ref_v], ref_leaves, [ref_g])):
         torch.testing.assert_close(a, b, rtol=0, atol=1e-13 * float(b.abs().max()))
+
+
+@pytest.mark.parametrize("periodic", [False, True])
+def test_a_shift_of_all_atoms_changes_no_vector(periodic):
+    """Positions on a grid of 2^-20 Angstrom in a cell of 8: a shift by 2^20 Angstrom (whole
+    cells) changes no difference of two positions, so every bit stays."""
+    from xnn_amd import dispersion as XD
+    gen = torch.Generator().manual_seed(3)
+    counts = [20] if periodic else [12, 8]
+    pos = (torch.randint(0, 1 << 23, (20, 3), generator=gen).double() / 2.0 ** 20).to(DEV)
+    cell = 8.0 * torch.eye(3, dtype=torch.float64, device=DEV)[None] if periodic else None
+    pbc = torch.ones((1, 3), dtype=torch.bool) if periodic else None
+    (e0, v0), (e1, v1) = (XD.triple_graph(pos + s, cell, pbc, counts, 5.0) for s in (0.0, 2.0 ** 20))
+    assert e0.shape[1] > 20 and torch.equal(e0, e1) and torch.equal(v0, v1)

@@ -1179,7 +1179,8 @@ def triple_graph(pos: Tensor, cell64: Optional[Tensor], pbc: Optional[Tensor], c
             shs.append(h)
             s0 += n
         ei, sh = (eis[0], shs[0]) if len(eis) == 1 else (torch.cat(eis, 1), torch.cat(shs))
-    return ei, _triple_vectors(pos / BOHR, None if cell64 is None else cell64 / BOHR, ei, sh, counts)
+    # scaled after the subtraction: a vector is rounded to its own length, not to the positions'
+    return ei, _triple_vectors(pos, cell64, ei, sh, counts) / BOHR
 
 
 def _triple_vectors(pos: Tensor, cell: Optional[Tensor], ei: Tensor, sh: Tensor,
