@@ -71,3 +71,12 @@ def test_a_shift_of_all_atoms_changes_no_vector(periodic):
     pbc = torch.ones((1, 3), dtype=torch.bool) if periodic else None
     (e0, v0), (e1, v1) = (XD.triple_graph(pos + s, cell, pbc, counts, 5.0) for s in (0.0, 2.0 ** 20))
     assert e0.shape[1] > 20 and torch.equal(e0, e1) and torch.equal(v0, v1)
+
+
+def test_other_refusals_of_the_plan_are_not_hidden():
+    """Only shifts beyond the plan's 10 bits go on in the tensor form (``far`` above)."""
+    from xnn_amd import dispersion as XD
+    pos = torch.rand((5, 3), dtype=torch.float64, device=DEV)
+    ei = torch.tensor([[0, 1], [1, 0]], device=DEV)
+    with pytest.raises(ValueError, match="sums to 6"):
+        XD._triple_vectors(pos, None, ei, torch.zeros((2, 3), dtype=torch.long, device=DEV), [6])

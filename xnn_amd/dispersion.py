@@ -1190,18 +1190,19 @@ def _triple_vectors(pos: Tensor, cell: Optional[Tensor], ei: Tensor, sh: Tensor,
     by E by 3 runs on one workgroup (75.7 of the 163 ms of a 700-atom cell's evaluation with
     2.2 million edges), and the atoms' sums follow the orderings instead of an index sort."""
     from .ops import edge_vectors
-    from .plan import build_plan
+    from .plan import ShiftRangeError, build_plan
     node_ptr, batch32 = _batch_tensors(counts, pos.device)
-    try:
-        plan = build_plan(ei, sh if cell is not None else None, pos.shape[0], batch32,
-                          node_ptr[1:] - node_ptr[:-1])
-    except ValueError:
-        # shifts beyond the plan's 10 bits (positions hundreds of cells away)
-        v = pos[ei[1]] - pos[ei[0]]
-        if cell is None:
-            return v
-        return v + (sh.to(pos.dtype)[:, None, :] @ cell[batch32.long()[ei[0]]])[:, 0]
-    return edge_vectors(pos, cell, plan)
+    if pos.is_cuda:
+        try:
+            plan = build_plan(ei, sh if cell is not None else None, pos.shape[0], batch32,
+                              node_ptr[1:] - node_ptr[:-1])
+            return edge_vectors(pos, cell, plan)
+        except ShiftRangeError:
+            pass              # positions hundreds of cells away
+    v = pos[ei[1]] - pos[ei[0]]
+    if cell is None:
+        return v
+    return v + (sh.to(pos.dtype)[:, None, :] @ cell[batch32.long()[ei[0]]])[:, 0]
 
 
 # --------------------------------------------------------------------------- potentials

@@ -49,6 +49,10 @@ class EdgePlan:
         return self.ptr_dst.device
 
 
+class ShiftRangeError(ValueError):
+    """Image shifts that the packed int32 of a plan cannot hold (10 bits an axis)."""
+
+
 def _int64(t: Tensor, device) -> Tensor:
     return t.to(device=device, dtype=torch.int64).contiguous()
 
@@ -61,7 +65,7 @@ def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
     a space-filling curve (:attr:`EdgePlan.visit`; ``cell`` (B, 3, 3) or None).
 
     Raises ``ValueError`` for edge indices outside ``[0, n_nodes)``, image
-    shifts outside ``[-512, 511]`` or atoms not grouped by structure.
+    shifts outside ``[-512, 511]`` (:class:`ShiftRangeError`) or atoms not grouped by structure.
     """
     device = edge_index.device
     if device.type != "cuda":
@@ -104,8 +108,8 @@ def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
     if bits & 2:
         raise ValueError(f"edge_index holds atom indices outside [0, {n_nodes})")
     if bits & 1:
-        raise ValueError("cell_shifts outside [-512, 511]: the packed int32 shifts cannot hold "
-                         "them (wrap the positions into the cell first)")
+        raise ShiftRangeError("cell_shifts outside [-512, 511]: the packed int32 shifts cannot "
+                              "hold them (wrap the positions into the cell first)")
     if bits & 16:
         raise ValueError("batch holds structure indices outside [0, B)")
     if bits & 8:
