@@ -44,3 +44,27 @@ def test_gradient_of_the_gradient():
         res.append([t.detach().cpu() for t in second])
     for a, b in zip(*res):
         torch.testing.assert_close(a, b, rtol=1e-10, atol=1e-10 * float(b.abs().max()))
+
+
+def test_forward_mode_and_batched_gradients():
+    """A directional derivative (dual numbers and functional) is the gradient times the
+    direction, also over a batch of vectors; a batch of cotangents is one after another."""
+    from torch.autograd import forward_ad as fw
+    from xnn_amd.eeq import reciprocal_apply
+    gen = torch.Generator().manual_seed(4)
+    r = lambda *s: torch.randn(*s, dtype=torch.float64, generator=gen).to(DEV)
+    pos, g, w, v, u, t = r(20, 3), r(30, 3), r(30).abs(), r(20), r(3, 20), r(20, 3)
+    leaf = pos.clone().requires_grad_(True)
+    out = reciprocal_apply(leaf, g, w, v)
+    rows = torch.stack([torch.autograd.grad(out, leaf, k, retain_graph=True)[0] for k in u])
+    want = torch.einsum("bij,ij->b", rows, t)
+    tol = dict(rtol=0, atol=1e-12 * float(rows.abs().sum(0).max()) * 60)
+    with fw.dual_level():
+        tangent = fw.unpack_dual(reciprocal_apply(fw.make_dual(pos, t), g, w, v)).tangent
+    torch.testing.assert_close(u @ tangent, want, **tol)
+    f = lambda p: reciprocal_apply(p, g, w, v)
+    torch.testing.assert_close(u @ torch.func.jvp(f, (pos,), (t,))[1], want, **tol)
+    torch.testing.assert_close(torch.func.vmap(lambda k: reciprocal_apply(pos, g, w, k))(u),
+                               torch.stack([reciprocal_apply(pos, g, w, k) for k in u]), **tol)
+    (got,) = torch.autograd.grad(out, leaf, u, is_grads_batched=True)
+    torch.testing.assert_close(got, rows, **tol)

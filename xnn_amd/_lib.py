@@ -354,6 +354,14 @@ def ptr(t: Optional[torch.Tensor]) -> Optional[int]:
     return t.data_ptr()
 
 
+def transformed(*tensors: Optional[torch.Tensor]) -> bool:
+    """Whether a call is part of a forward-mode derivative or a functional transform: a custom
+    op has no tangent, so a function with a tensor form takes that one there."""
+    return torch._C._are_functorch_transforms_active() or any(
+        torch.autograd.forward_ad.unpack_dual(t).tangent is not None
+        for t in tensors if t is not None)
+
+
 def stream(device: torch.device) -> int:
     """The current HIP stream of ``device`` as an integer handle."""
     return torch.cuda.current_stream(device).cuda_stream

@@ -117,8 +117,9 @@ def reciprocal_apply(pos: Tensor, g: Tensor, w: Tensor, v: Tensor) -> Tensor:
     that carries gradients is recomputed in the backward instead of kept (memory
     ``O(LIVE_BUDGET)`` at any size). One vector ``v`` in float64 on the GPU goes through
     :func:`reciprocal_op`, which keeps no phases: 5,000 atoms and their forces 0.15 ms
-    against 1.6 ms."""
-    if pos.is_cuda and v.dim() == 1 and all(t.dtype == torch.float64 for t in (pos, g, w, v)):
+    against 1.6 ms; forward-mode derivatives and functional transforms take the tensor form."""
+    if (pos.is_cuda and v.dim() == 1 and all(t.dtype == torch.float64 for t in (pos, g, w, v))
+            and not _lib.transformed(pos, g, w, v)):
         return reciprocal_op(pos.contiguous(), g.contiguous(), w.contiguous(), v.contiguous())[0]
     return _reciprocal_blocks(pos, g, w, v)
 
@@ -162,6 +163,28 @@ def _recip_work(n: int, m: int, backward: bool, device) -> Tensor:
     return torch.empty(need.value, dtype=torch.uint8, device=device)
 
 
+@torch.library.custom_op(f"{_NS}::eeq_reciprocal_backward", mutates_args=())
+def reciprocal_backward_op(pos: Tensor, g: Tensor, w: Tensor, v: Tensor, factors: Tensor, u: Tensor,
+                           cell_side: bool) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
+    """The gradients of :func:`reciprocal_op` in ``pos``, ``g``, ``w`` (zeros unless
+    ``cell_side``) and ``v`` for the output's gradient ``u``; an op, so that a batch of ``u``
+    goes through it one by one."""
+    n, m = int(pos.shape[0]), int(g.shape[0])
+    u = u.contiguous()
+    grads = [torch.zeros_like(t) for t in (pos, g, w, v)]
+    work = _recip_work(n, m, True, pos.device)
+    _lib.call("xnn_eeq_recip_backward", _lib.ptr(pos), n, _lib.ptr(g), _lib.ptr(w), m, _lib.ptr(v),
+              _lib.ptr(factors), _lib.ptr(u), _lib.ptr(grads[0]),
+              _lib.ptr(grads[1] if cell_side else None), _lib.ptr(grads[2] if cell_side else None),
+              _lib.ptr(grads[3]), _lib.ptr(work), int(work.numel()), _lib.stream(pos.device))
+    return tuple(grads)
+
+
+@reciprocal_backward_op.register_fake
+def _(pos, g, w, v, factors, u, cell_side):
+    return tuple(torch.empty_like(t) for t in (pos, g, w, v))
+
+
 @reciprocal_op.register_fake
 def _(pos, g, w, v):
     return pos.new_empty(pos.shape[0]), pos.new_empty((2, g.shape[0]))
@@ -179,16 +202,9 @@ def _reciprocal_backward(ctx, u, _factors):
         wanted = [t for t, need in zip((pos, g, w, v), ctx.needs_input_grad) if need]
         grads = iter(torch.autograd.grad([out], wanted, [u], create_graph=True))
         return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
-    n, m = int(pos.shape[0]), int(g.shape[0])
     cell_side = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
-    grad_pos, grad_v = torch.zeros_like(pos), torch.zeros_like(v)
-    grad_g, grad_w = (torch.zeros_like(g), torch.zeros_like(w)) if cell_side else (None, None)
-    work = _recip_work(n, m, True, pos.device)
-    _lib.call("xnn_eeq_recip_backward", _lib.ptr(pos), n, _lib.ptr(g), _lib.ptr(w), m, _lib.ptr(v),
-              _lib.ptr(factors), _lib.ptr(u.contiguous()), _lib.ptr(grad_pos), _lib.ptr(grad_g),
-              _lib.ptr(grad_w), _lib.ptr(grad_v), _lib.ptr(work), int(work.numel()),
-              _lib.stream(pos.device))
-    return grad_pos, grad_g, grad_w, grad_v
+    grads = reciprocal_backward_op(pos, g, w, v, factors, u, cell_side)
+    return tuple(t if need else None for t, need in zip(grads, ctx.needs_input_grad))
 
 
 reciprocal_op.register_autograd(_reciprocal_backward, setup_context=_reciprocal_setup)
