@@ -80,3 +80,16 @@ def test_other_refusals_of_the_plan_are_not_hidden():
     ei = torch.tensor([[0, 1], [1, 0]], device=DEV)
     with pytest.raises(ValueError, match="sums to 6"):
         XD._triple_vectors(pos, None, ei, torch.zeros((2, 3), dtype=torch.long, device=DEV), [6])
+
+
+def test_vectors_have_a_tangent():
+    """Forward-mode derivatives: the vectors are linear in the positions and the cell."""
+    from torch.autograd import forward_ad as fw
+    from xnn_amd import dispersion as XD
+    gen = torch.Generator().manual_seed(6)
+    pos = (4.0 * torch.rand((9, 3), generator=gen, dtype=torch.float64)).to(DEV)
+    cell = (6.0 * torch.eye(3, dtype=torch.float64))[None].to(DEV)
+    with fw.dual_level():
+        _, v = XD.triple_graph(fw.make_dual(pos, pos), fw.make_dual(cell, cell), None, [9], 5.0)
+        value, tangent = fw.unpack_dual(v)
+    torch.testing.assert_close(tangent, value, rtol=0, atol=1e-14 * float(value.abs().max()))

@@ -1192,7 +1192,7 @@ def _triple_vectors(pos: Tensor, cell: Optional[Tensor], ei: Tensor, sh: Tensor,
     from .ops import edge_vectors
     from .plan import ShiftRangeError, build_plan
     node_ptr, batch32 = _batch_tensors(counts, pos.device)
-    if pos.is_cuda:
+    if pos.is_cuda and not _lib.transformed(pos, cell):
         try:
             plan = build_plan(ei, sh if cell is not None else None, pos.shape[0], batch32,
                               node_ptr[1:] - node_ptr[:-1])
