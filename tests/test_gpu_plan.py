@@ -86,3 +86,16 @@ def test_visit_order_follows_the_cell(dtype):
     t[5, 1] = float("nan")
     assert np.array_equal(np.sort(build_plan(none, None, n, pos=t, cell=c).visit.cpu().numpy()),
                           np.arange(n))
+
+
+def test_a_batch_or_positions_that_miss_atoms_are_refused():
+    """The plan's kernel reads one entry an atom; refused on the host, before any launch."""
+    from xnn_amd.plan import build_plan
+    none = torch.zeros((2, 0), dtype=torch.long, device=DEV)
+    with pytest.raises(ValueError, match="batch holds 4"):
+        build_plan(none, None, 5, torch.zeros(4, dtype=torch.long, device=DEV))
+    for shape in ((4, 3), (5, 2), (6, 3)):
+        with pytest.raises(ValueError, match="positions"):
+            build_plan(none, None, 5, pos=torch.zeros(shape, device=DEV))
+    plan = build_plan(none, None, 5, pos=torch.rand((5, 3)))           # from the host
+    assert sorted(plan.visit.tolist()) == [0, 1, 2, 3, 4]

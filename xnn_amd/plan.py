@@ -65,7 +65,8 @@ def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
     a space-filling curve (:attr:`EdgePlan.visit`; ``cell`` (B, 3, 3) or None).
 
     Raises ``ValueError`` for edge indices outside ``[0, n_nodes)``, image
-    shifts outside ``[-512, 511]`` (:class:`ShiftRangeError`) or atoms not grouped by structure.
+    shifts outside ``[-512, 511]`` (:class:`ShiftRangeError`), atoms not grouped by structure
+    and a ``batch`` or ``pos`` that does not cover the atoms.
     """
     device = edge_index.device
     if device.type != "cuda":
@@ -76,10 +77,14 @@ def build_plan(edge_index: Tensor, cell_shifts: Optional[Tensor], n_nodes: int,
     if cell_shifts is not None and cell_shifts.numel() > 0:
         shifts = _int64(cell_shifts, device)
     batch = None if batch is None else _int64(batch, device)
+    if batch is not None and batch.shape[0] < n_nodes:
+        raise ValueError(f"batch holds {batch.shape[0]} of the graph's {n_nodes} atoms")
     n_atoms = None if n_atoms is None else _int64(n_atoms, device)
     n_graphs = 1 if n_atoms is None else int(n_atoms.shape[0])
     if pos is not None and n_nodes > 0 and n_graphs > 0:
-        pos = pos.detach().contiguous()
+        if tuple(pos.shape) != (n_nodes, 3):
+            raise ValueError(f"positions {tuple(pos.shape)} of a graph of {n_nodes} atoms")
+        pos = pos.detach().to(device).contiguous()
         if pos.dtype not in (torch.float32, torch.float64):
             pos = pos.double()
         geom = _lib.dtype_code(pos.dtype)
