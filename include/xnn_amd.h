@@ -1004,7 +1004,7 @@ int xnn_scan_counts(int32_t* row_ptr, int64_t n, void* workspace, xnn_stream_t s
  * sender CSR (ptr_src, perm_src), both stable (edge order within a row).
  * Mirrors the orderings of common/models/csr.py:20-51. Shift fields outside
  * [-512, 511] fail with XNN_ECAPACITY (flag written to *overflow on device: bit 0 a shift
- * out of range, bit 1 an index out of [0, N), bit 2 edges not grouped by receiver). */
+ * out of range, bit 1 an index out of [0, N); 0 for every other list). */
 size_t xnn_edge_plan_workspace_bytes(int64_t n_edges, int64_t n_nodes);
 int xnn_edge_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t n_edges,
                   int64_t n_nodes, int32_t* src, int32_t* dst, int32_t* shift,
@@ -1017,8 +1017,9 @@ int xnn_edge_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t
  * for B = 1) -> node_ptr (B+1); visit (N, nullable): the atoms along a Morton curve of
  * bins of each structure (fractional coordinates of cell (B,3,3), or positions; ties in
  * atom order), an ordering hint for the force reductions. pos and cell in geom_dtype.
- * *flags (device): the bits of xnn_edge_plan, bit 3 batch not sorted, bit 4 batch outside
- * [0, B), bit 5 n_atoms not summing to N. */
+ * *flags (device): the bits of xnn_edge_plan, bit 2 the edges are not grouped by receiver (no
+ * error: perm_dst is needed then), bit 3 batch not sorted, bit 4 batch outside [0, B), bit 5
+ * n_atoms not summing to N. */
 size_t xnn_graph_plan_workspace_bytes(int64_t n_edges, int64_t n_nodes, int64_t n_graphs,
                                       int32_t with_visit);
 int xnn_graph_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t n_edges,

@@ -99,3 +99,22 @@ def test_a_batch_or_positions_that_miss_atoms_are_refused():
             build_plan(none, None, 5, pos=torch.zeros(shape, device=DEV))
     plan = build_plan(none, None, 5, pos=torch.rand((5, 3)))           # from the host
     assert sorted(plan.visit.tolist()) == [0, 1, 2, 3, 4]
+
+
+def test_edge_plan_reports_errors_only():
+    """``xnn_edge_plan``'s flag is 0 for a list that is not grouped by receiver."""
+    import ctypes
+    from xnn_amd import _lib
+    rng = np.random.default_rng(0)
+    n, e = 300, 5000
+    ei = torch.tensor(rng.integers(0, n, (2, e)), device=DEV)
+    out = [torch.empty(k, dtype=torch.int32, device=DEV) for k in (e, e, e, n + 1, e, n + 1, e, 1)]
+    need = int(_lib.load().xnn_edge_plan_workspace_bytes(e, n))
+    ws = torch.empty(need, dtype=torch.uint8, device=DEV)
+    _lib.call("xnn_edge_plan", _lib.ptr(ei), None, e, n, *[_lib.ptr(t) for t in out], _lib.ptr(ws),
+              ctypes.c_size_t(need), _lib.stream(torch.device(DEV)))
+    assert out[7].item() == 0
+    for row, ptr, perm in ((1, out[3], out[4]), (0, out[5], out[6])):
+        key = ei[row].cpu().numpy()
+        assert np.array_equal(ptr.cpu(), np.concatenate([[0], np.cumsum(np.bincount(key, minlength=n))]))
+        assert np.array_equal(perm.cpu(), np.argsort(key, kind="stable"))

@@ -492,3 +492,17 @@ def test_low_rank_preconditioner_inverts_its_matrix():
     M = torch.diag(1.0 / system.inv_d) + system.U @ torch.diag(torch.cat([wl, wl])) @ system.U.t()
     r = torch.randn(n, 2, dtype=torch.float64, generator=g0)
     torch.testing.assert_close(M @ system.precondition(r), r, rtol=0, atol=1e-11)
+
+
+def test_edge_plan_refuses_null_arrays_before_any_launch(lib_path):
+    from xnn_amd import _lib
+    lib = _lib.load()
+    buf = ctypes.create_string_buffer(1 << 16)
+    at = ctypes.cast(buf, ctypes.c_void_p)
+    sizes = (4, 3, int(lib.xnn_edge_plan_workspace_bytes(4, 3)))
+    names = ["edge_index", "src", "dst", "shift", "perm_dst", "perm_src"]
+    for missing in names + ["workspace"]:
+        p = {k: None if k == missing else at for k in names + ["workspace"]}
+        code = lib.xnn_edge_plan(p["edge_index"], None, 4, 3, p["src"], p["dst"], p["shift"], at,
+                                 p["perm_dst"], at, p["perm_src"], at, p["workspace"], sizes[2], None)
+        assert code == _lib.XNN_EINVAL, missing

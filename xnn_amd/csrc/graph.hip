@@ -879,7 +879,8 @@ __global__ __launch_bounds__(256) void plan_read_kernel(
     const int64_t* __restrict__ ei, const int64_t* __restrict__ sh, int64_t E, int64_t n,
     int32_t* __restrict__ src, int32_t* __restrict__ dst, int32_t* __restrict__ shift,
     int32_t* __restrict__ rank_src, int32_t* __restrict__ cnt_src, int32_t* __restrict__ cnt_dst,
-    PlanAtoms A, int64_t edge_blocks, int64_t atom_blocks, int32_t* __restrict__ flags) {
+    PlanAtoms A, int64_t edge_blocks, int64_t atom_blocks, int32_t* __restrict__ flags,
+    int32_t* __restrict__ grouping) {
   int bad = 0;
   if ((int64_t)blockIdx.x < edge_blocks) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -973,7 +974,10 @@ __global__ __launch_bounds__(256) void plan_read_kernel(
   int any = 0;
 #pragma unroll
   for (int k = 0; k < 6; ++k) any |= __ballot(bad & (1 << k)) ? 1 << k : 0;
-  if (any && threadIdx.x % kWave == 0) atomicOr(flags, any);
+  if (any && threadIdx.x % kWave == 0) {
+    if (any & kFlagUngrouped) atomicOr(grouping, kFlagUngrouped);
+    if (any & ~kFlagUngrouped) atomicOr(flags, any & ~kFlagUngrouped);
+  }
 }
 
 __device__ inline int32_t block_sum_1024(int32_t v, int32_t* wsum) {
@@ -1042,11 +1046,11 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(PlanJobs J, const int32
 }
 
 __global__ __launch_bounds__(256) void plan_scatter_kernel(PlanJobs J,
-                                                           const int32_t* __restrict__ flags) {
+                                                           const int32_t* __restrict__ grouping) {
   const PlanJob& j = J.job[blockIdx.y];
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= j.items) return;
-  if (j.rank == nullptr && !(*flags & kFlagUngrouped)) {
+  if (j.rank == nullptr && !(*grouping & kFlagUngrouped)) {
     j.perm[e] = (int32_t)e;
     return;
   }
@@ -1059,10 +1063,10 @@ __global__ __launch_bounds__(256) void plan_scatter_kernel(PlanJobs J,
 // comparison; up to 1,024: the same over tiles of 64; longer rows: three passes of a stable
 // radix sort of the row (digit counts in LDS, ranks within a wave by ballots).
 __global__ __launch_bounds__(kPlanWaves* kWave) void plan_row_sort_kernel(
-    PlanJobs J, const int32_t* __restrict__ flags, int digit) {
+    PlanJobs J, const int32_t* __restrict__ grouping, int digit) {
   __shared__ int32_t hist[kPlanWaves][1 << kPlanDigitMax];
   const PlanJob& j = J.job[blockIdx.y];
-  if (j.rank == nullptr && !(*flags & kFlagUngrouped)) return;
+  if (j.rank == nullptr && !(*grouping & kFlagUngrouped)) return;
   const int64_t row = (int64_t)blockIdx.x * kPlanWaves + threadIdx.x / kWave;
   if (row >= j.rows) return;
   const int lane = threadIdx.x % kWave;
@@ -1141,8 +1145,8 @@ __global__ void plan_iota_kernel(int32_t* __restrict__ iota, int64_t n) {
 }
 
 struct PlanWs {
-  size_t rank_src, tmp_src, tmp_dst, code, rank_vis, tmp_vis, ptr_vis, cnt, sums, cub, cub_bytes,
-      total;
+  size_t rank_src, tmp_src, tmp_dst, code, rank_vis, tmp_vis, ptr_vis, cnt, sums, grouping, cub,
+      cub_bytes, total;
   int64_t cnt_ints, bins, max_tiles;
   int bits;
   bool library;
@@ -1178,6 +1182,7 @@ static PlanWs plan_ws_layout(int64_t E, int64_t n, int64_t n_graphs, bool visit)
   ints(w.cnt, w.cnt_ints);
   w.max_tiles = (std::max(n, w.bins) + kPlanTile - 1) / kPlanTile;
   ints(w.sums, 3 * w.max_tiles);
+  ints(w.grouping, 1);
   if (w.library) {
     size_t sort_bytes = 0;
     (void)hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (int32_t*)nullptr,
@@ -1197,19 +1202,25 @@ static int end_bit_for(int64_t n) {
   return b;
 }
 
-__global__ void plan_zero_kernel(int32_t* __restrict__ cnt, int64_t n, int32_t* __restrict__ flags) {
+__global__ void plan_zero_kernel(int32_t* __restrict__ cnt, int64_t n, int32_t* __restrict__ flags,
+                                 int32_t* __restrict__ grouping) {
   const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) cnt[i] = 0;
-  if (i == 0) flags[0] = 0;
+  if (i == 0) flags[0] = grouping[0] = 0;
 }
 
+// grouping: where bit 2 goes (flags itself, or NULL: a word of the workspace)
 static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t E,
                             int64_t n, PlanAtoms A, int32_t* visit, int32_t* src, int32_t* dst,
                             int32_t* shift, int32_t* ptr_dst, int32_t* perm_dst, int32_t* ptr_src,
-                            int32_t* perm_src, int32_t* flags, void* ws, size_t ws_bytes,
-                            hipStream_t s) {
+                            int32_t* perm_src, int32_t* flags, int32_t* grouping, void* ws,
+                            size_t ws_bytes, hipStream_t s) {
+  XNN_REQUIRE(E == 0 || (edge_index && src && dst && shift && perm_dst && perm_src),
+              "NULL edge input or output");
   const PlanWs w = plan_ws_layout(E, n, A.n_graphs, visit != nullptr);
-  XNN_REQUIRE(ws_bytes >= w.total, "workspace too small: %zu < %zu", ws_bytes, w.total);
+  XNN_REQUIRE(ws != nullptr && ws_bytes >= w.total, "workspace too small: %zu < %zu", ws_bytes,
+              w.total);
+  if (grouping == nullptr) grouping = ws_at<int32_t>(ws, w.grouping);
   int32_t* cnt = ws_at<int32_t>(ws, w.cnt);
   int32_t* cnt_dst = cnt + (n + 1);
   int32_t* sums = ws_at<int32_t>(ws, w.sums);
@@ -1230,13 +1241,13 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
     A.pos = nullptr;
   }
   hipLaunchKernelGGL(plan_zero_kernel, dim3(grid_1d(w.cnt_ints, 256)), dim3(256), 0, s, cnt,
-                     w.cnt_ints, flags);
+                     w.cnt_ints, flags, grouping);
   const bool atoms = A.node_ptr != nullptr;
   const int64_t eb = grid_1d(E, 256), ab = atoms ? grid_1d(n, 256) : 0;
   if (eb + ab + (atoms ? 1 : 0) > 0)
     hipLaunchKernelGGL(plan_read_kernel, dim3((unsigned)(eb + ab + (atoms ? 1 : 0))), dim3(256), 0,
                        s, edge_index, cell_shifts, E, n, src, dst, shift, rank_src, cnt, cnt_dst, A,
-                       eb, ab, flags);
+                       eb, ab, flags, grouping);
   XNN_LAUNCH_CHECK();
   if (n == 0) {   // no rows: the pointers' single entry
     hipLaunchKernelGGL(set_first_zero_kernel, dim3(1), dim3(1), 0, s, ptr_dst);
@@ -1268,11 +1279,11 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
   const int64_t rows = std::max(J.job[0].rows, J.job[2].rows);
   if (items > 0) {
     hipLaunchKernelGGL(plan_scatter_kernel, dim3((unsigned)grid_1d(items, 256), jobs), dim3(256), 0,
-                       s, J, flags);
+                       s, J, grouping);
     int digit = 1;
     while ((int64_t(1) << (3 * digit)) < items && digit < kPlanDigitMax) ++digit;
     hipLaunchKernelGGL(plan_row_sort_kernel, dim3((unsigned)grid_1d(rows, kPlanWaves), jobs),
-                       dim3(kPlanWaves * kWave), 0, s, J, flags, digit);
+                       dim3(kPlanWaves * kWave), 0, s, J, grouping, digit);
     XNN_LAUNCH_CHECK();
   }
   return XNN_OK;
@@ -1791,8 +1802,8 @@ int xnn_edge_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_t
   PlanAtoms A{};
   A.n_graphs = 1;
   return build_graph_plan(edge_index, cell_shifts, n_edges, n_nodes, A, nullptr, src, dst, shift,
-                          ptr_dst, perm_dst, ptr_src, perm_src, overflow, workspace,
-                          workspace_bytes, as_hip(stream));
+                          ptr_dst, perm_dst, ptr_src, perm_src, overflow, nullptr,
+                          workspace, workspace_bytes, as_hip(stream));
 }
 
 size_t xnn_graph_plan_workspace_bytes(int64_t n_edges, int64_t n_nodes, int64_t n_graphs,
@@ -1812,8 +1823,6 @@ int xnn_graph_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_
               "int32 indices: at most 2^31 - 1 edges, atoms and structures");
   XNN_REQUIRE(ptr_dst && ptr_src && flags && node_ptr, "NULL output");
   XNN_REQUIRE(n_nodes == 0 || batch32, "NULL batch32");
-  XNN_REQUIRE(n_edges == 0 || (edge_index && src && dst && shift && perm_dst && perm_src),
-              "NULL edge input or output");
   XNN_REQUIRE(n_atoms || n_graphs <= 1, "n_atoms is needed for more than one structure");
   XNN_REQUIRE(visit == nullptr || n_nodes == 0 ||
                   (pos != nullptr && n_graphs >= 1 &&
@@ -1830,7 +1839,7 @@ int xnn_graph_plan(const int64_t* edge_index, const int64_t* cell_shifts, int64_
   A.geom = geom_dtype;
   return build_graph_plan(edge_index, cell_shifts, n_edges, n_nodes, A,
                           n_nodes > 0 ? visit : nullptr, src, dst, shift, ptr_dst, perm_dst, ptr_src,
-                          perm_src, flags, workspace, workspace_bytes, as_hip(stream));
+                          perm_src, flags, flags, workspace, workspace_bytes, as_hip(stream));
 }
 
 int xnn_nearest_edges_count(const int32_t* ptr_dst, int64_t n_nodes, int32_t k, int32_t* kept_ptr,
