@@ -118,3 +118,38 @@ def test_edge_plan_reports_errors_only():
         key = ei[row].cpu().numpy()
         assert np.array_equal(ptr.cpu(), np.concatenate([[0], np.cumsum(np.bincount(key, minlength=n))]))
         assert np.array_equal(perm.cpu(), np.argsort(key, kind="stable"))
+
+
+@pytest.mark.parametrize("e,hubs", [
+    (200_000, [1024, 1025, 1500, 90_000]),            # one window of 2^18 ids
+    (700_000, [1024, 1025, 5000, 2000, 300_000]),     # three, some of a row's empty
+    (300_000, [299_990]),                             # nearly all
+    (5_300_000, [1100, 5375, 5376, 6000, 40_000]),    # 21: a wave sorts up to 5,375 ids
+])
+@pytest.mark.parametrize("scattered", [True, False])
+def test_rows_of_any_length_are_sorted(e, hubs, scattered):
+    """A few long rows among short ones, their ids all over the list or in one stretch."""
+    from xnn_amd.plan import build_plan
+    rng = np.random.default_rng(e + len(hubs))
+    n = 5000
+    key = rng.integers(len(hubs), n, e)
+    at = rng.permutation(e) if scattered else np.roll(np.arange(e), e // 3)
+    s0 = 0
+    for row, length in enumerate(hubs):
+        key[at[s0:s0 + length]] = row
+        s0 += length
+    other = rng.permutation(key)
+    plan = build_plan(torch.tensor(np.stack([key, other]), device=DEV), None, n)
+    for k, ptr, perm in ((key, plan.ptr_src, plan.perm_src), (other, plan.ptr_dst, plan.perm_dst)):
+        assert np.array_equal(ptr.cpu(), np.concatenate([[0], np.cumsum(np.bincount(k, minlength=n))]))
+        assert np.array_equal(perm.cpu(), np.argsort(k, kind="stable"))
+
+
+def test_visit_order_of_one_crowded_bin():
+    """Atoms in one corner of a wide cell share a bin: they are visited in their order."""
+    from xnn_amd.plan import build_plan
+    none = torch.zeros((2, 0), dtype=torch.long, device=DEV)
+    pos = torch.rand((30_000, 3), device=DEV, dtype=torch.float64)
+    cell = torch.eye(3, device=DEV, dtype=torch.float64)[None] * 1e4
+    assert torch.equal(build_plan(none, None, 30_000, pos=pos, cell=cell).visit.cpu(),
+                       torch.arange(30_000, dtype=torch.int32))

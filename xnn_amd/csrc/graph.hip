@@ -765,30 +765,38 @@ __global__ __launch_bounds__(256) void molecule_search_kernel(
 // ---------------------------------------------------------------- edge plan
 // The orderings of an edge list: int32 copies, the receiver and sender CSR and (optional) a
 // space-filling order of the atoms. All three orderings are counting sorts that share their
-// launches (blockIdx.y = the job): the counts are taken while the list is read, one scan
-// turns them into row pointers, one pass scatters the ids into their rows in arrival order,
-// and a wave per row puts them in ascending order (the order of a stable sort by row, so
-// the plan does not depend on the order of the atomics). A list already grouped by
-// receiver (what the neighbor list returns) has its receiver counts taken from the runs'
-// ends, two atomics a row, and needs no receiver scatter or sort; whether it is grouped is
-// found by the read itself (flag bit 2), so the host need not know.
+// launches (blockIdx.y = the job): the counts and every item's arrival rank are taken while the
+// list is read, one scan turns them into row pointers, one pass scatters the ids into their rows
+// in arrival order, and they are put in ascending order there (the order of a stable sort by
+// row, so the plan does not depend on the order of the atomics). A list already grouped by
+// receiver (what the neighbor list returns) takes about two receiver atomics a row and needs no
+// receiver scatter or sort; whether it is grouped is found by the read itself (flag bit 2), so
+// the host need not know.
 // Bound by the sender counts' device-scope atomics (about one per edge) and, for small
 // lists, by the five launches. Measured against two library radix sorts, the per-edge
 // atomics of both orderings and the separate batch, grouping and Morton-order passes:
-// 620 -> 64 us of kernels (140 -> 6 launches) for 478k edges of 9,000 atoms, 1,116 -> 210 us
-// for 3.8M edges of 72,000 atoms (18 B read and 32 B written an edge: 0.9 TB/s there).
+// 620 -> 58 us of kernels (140 -> 6 launches) for 478k edges of 9,000 atoms, 1,116 -> 210 us
+// for 3.8M edges of 72,000 atoms (52 B read and 32 B written an edge: 1.5 TB/s there, the read
+// alone 2.6).
 constexpr int kPlanTile = 8192;       // counts scanned by one block
 constexpr int kPlanWaves = 4;         // rows sorted per block of the row sort
-constexpr int kPlanDigitMax = 11;     // id bits per pass of a long row's sort (3 passes)
-// Mean row length above which the orderings go to the library's radix sort: one wave sorts a
-// row, and rows of 8,192 ids take it about 0.2 ms while few waves run at once.
-constexpr int64_t kPlanRowMax = 8192;
+constexpr int kPlanThreads = kPlanWaves * kWave;
+constexpr int kPlanDigitMax = 11;     // id bits per pass of a wave's radix sort (3 passes)
+constexpr int kPlanLds = 8192;        // ints: the waves' digit counts, or one bitmap
+constexpr int kPlanRowShort = 1024;   // ids that a wave sorts by comparison
+constexpr int kPlanLongBlocks = 256;  // blocks after those of the rows, for long rows
+constexpr int kPlanWindowBits = 18;   // ids a bitmap holds: 32 x 8,192
+constexpr int kPlanWindow = 1 << kPlanWindowBits;
+constexpr int kPlanWindowShare = 256;  // ids for each window of the list that make a row long
+static_assert(kPlanLds * 32 == kPlanWindow && kPlanLds >= (1ll << (31 - kPlanWindowBits)) &&
+                  kPlanLds == kPlanWaves << kPlanDigitMax,
+              "the row sorts share their LDS");
 constexpr int kFlagShift = 1, kFlagIndex = 2, kFlagUngrouped = 4, kFlagBatchOrder = 8,
               kFlagBatchRange = 16, kFlagAtomCount = 32;
 
 struct PlanJob {
   const int32_t* key;   // row of each item
-  const int32_t* rank;  // arrival rank within the row (NULL: counted down in the scatter)
+  const int32_t* rank;  // arrival rank within the row
   int32_t* cnt;         // (rows + 1) counts
   int32_t* ptr;         // (rows + 1) row pointers
   int32_t* tmp;         // scattered ids
@@ -798,24 +806,34 @@ struct PlanJob {
 struct PlanJobs {
   PlanJob job[3];       // sender, receiver, visit order
 };
+constexpr int kJobReceiver = 1;
 
-// arrival rank of each lane's item in its row: one atomic per run of lanes with the same row
-__device__ inline int32_t wave_rank(int32_t* __restrict__ cnt, int32_t row, bool live) {
+// Arrival ranks of the lanes' items in their rows, one atomic per run of lanes with the same
+// row: wave_claim issues it, wave_rank takes its result (two claims can be in flight).
+struct WaveClaim {
+  int32_t base;
+  int lead;             // first lane of this lane's run
+};
+
+__device__ inline WaveClaim wave_claim(int32_t* __restrict__ cnt, int32_t row, bool live) {
   const int lane = threadIdx.x % kWave;
   const int32_t prev = __shfl_up(row, 1, kWave);
   const uint64_t alive = __ballot(live);
   const bool head = live && (lane == 0 || prev != row || !((alive >> (lane - 1)) & 1));
   const uint64_t heads = __ballot(head);
   const uint64_t below = heads & (~0ull >> (kWave - 1 - lane));      // heads at or below
-  const int lead = below ? kWave - 1 - __clzll((long long)below) : 0;
-  int32_t base = 0;
+  WaveClaim c{0, below ? kWave - 1 - __clzll((long long)below) : 0};
   if (head) {
     // the run ends at the next head or the first dead lane
     const uint64_t above = lane == kWave - 1 ? 0ull : ((heads | ~alive) >> (lane + 1)) << (lane + 1);
     const int end = above ? __ffsll((unsigned long long)above) - 1 : kWave;
-    base = atomicAdd(&cnt[row], end - lane);
+    c.base = atomicAdd(&cnt[row], end - lane);
   }
-  return __shfl(base, lead, kWave) + lane - lead;
+  return c;
+}
+
+__device__ inline int32_t wave_rank(const WaveClaim& c) {
+  return __shfl(c.base, c.lead, kWave) + threadIdx.x % kWave - c.lead;
 }
 
 __device__ inline uint32_t spread_bits(uint32_t q) {  // 10 bits to every third bit
@@ -878,9 +896,9 @@ __device__ inline int32_t visit_code(const PlanAtoms& A, int64_t i, int64_t b) {
 __global__ __launch_bounds__(256) void plan_read_kernel(
     const int64_t* __restrict__ ei, const int64_t* __restrict__ sh, int64_t E, int64_t n,
     int32_t* __restrict__ src, int32_t* __restrict__ dst, int32_t* __restrict__ shift,
-    int32_t* __restrict__ rank_src, int32_t* __restrict__ cnt_src, int32_t* __restrict__ cnt_dst,
-    PlanAtoms A, int64_t edge_blocks, int64_t atom_blocks, int32_t* __restrict__ flags,
-    int32_t* __restrict__ grouping) {
+    int32_t* __restrict__ rank_src, int32_t* __restrict__ rank_dst, int32_t* __restrict__ cnt_src,
+    int32_t* __restrict__ cnt_dst, PlanAtoms A, int64_t edge_blocks, int64_t atom_blocks,
+    int32_t* __restrict__ flags, int32_t* __restrict__ grouping) {
   int bad = 0;
   if ((int64_t)blockIdx.x < edge_blocks) {
     const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
@@ -902,22 +920,19 @@ __global__ __launch_bounds__(256) void plan_read_kernel(
       }
       if (x < -512 || x > 511 || y < -512 || y > 511 || z < -512 || z > 511) bad |= kFlagShift;
       shift[e] = pack_shift((int)x, (int)y, (int)z);
-      // a receiver's count: (end of a run) - (its start), summed over its runs
-      int32_t before = -1, after = -1;
+      int32_t before = -1;
       if (e > 0) {
         const int64_t p = ei[E + e - 1], q = ei[e - 1];
         before = p >= 0 && p < n && q >= 0 && q < n ? (int32_t)p : 0;
       }
-      if (e + 1 < E) {
-        const int64_t p = ei[E + e + 1], q = ei[e + 1];
-        after = p >= 0 && p < n && q >= 0 && q < n ? (int32_t)p : 0;
-      }
       if (before > d) bad |= kFlagUngrouped;
-      const int32_t add = (after != d ? (int32_t)(e + 1) : 0) - (before != d ? (int32_t)e : 0);
-      if (add != 0) atomicAdd(&cnt_dst[d], add);
     }
-    const int32_t r = wave_rank(cnt_src, s, live);
-    if (live) rank_src[e] = r;
+    const WaveClaim cs = wave_claim(cnt_src, s, live), cd = wave_claim(cnt_dst, d, live);
+    const int32_t r = wave_rank(cs), rd = wave_rank(cd);
+    if (live) {
+      rank_src[e] = r;
+      rank_dst[e] = rd;
+    }
   } else if ((int64_t)blockIdx.x < edge_blocks + atom_blocks) {
     const int64_t i = ((int64_t)blockIdx.x - edge_blocks) * 256 + threadIdx.x;
     const bool live = i < n;
@@ -934,7 +949,7 @@ __global__ __launch_bounds__(256) void plan_read_kernel(
     if (A.pos != nullptr) {
       const int32_t code = !live ? 0 : A.geom == XNN_F64 ? visit_code<double>(A, i, b)
                                                          : visit_code<float>(A, i, b);
-      const int32_t r = wave_rank(A.cnt, code, live);
+      const int32_t r = wave_rank(wave_claim(A.cnt, code, live));
       if (live) {
         A.code[i] = code;
         A.rank[i] = r;
@@ -1050,30 +1065,18 @@ __global__ __launch_bounds__(256) void plan_scatter_kernel(PlanJobs J,
   const PlanJob& j = J.job[blockIdx.y];
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e >= j.items) return;
-  if (j.rank == nullptr && !(*grouping & kFlagUngrouped)) {
+  if (blockIdx.y == kJobReceiver && !(*grouping & kFlagUngrouped)) {
     j.perm[e] = (int32_t)e;
     return;
   }
-  const int32_t row = j.key[e];
-  const int32_t slot = j.rank != nullptr ? j.rank[e] : atomicSub(&j.cnt[row], 1) - 1;
-  j.tmp[j.ptr[row] + slot] = (int32_t)e;
+  j.tmp[j.ptr[j.key[e]] + j.rank[e]] = (int32_t)e;
 }
 
-// One wave per row: its scattered ids in ascending order. Up to 64 ids: each lane's rank by
-// comparison; up to 1,024: the same over tiles of 64; longer rows: three passes of a stable
-// radix sort of the row (digit counts in LDS, ranks within a wave by ballots).
-__global__ __launch_bounds__(kPlanWaves* kWave) void plan_row_sort_kernel(
-    PlanJobs J, const int32_t* __restrict__ grouping, int digit) {
-  __shared__ int32_t hist[kPlanWaves][1 << kPlanDigitMax];
-  const PlanJob& j = J.job[blockIdx.y];
-  if (j.rank == nullptr && !(*grouping & kFlagUngrouped)) return;
-  const int64_t row = (int64_t)blockIdx.x * kPlanWaves + threadIdx.x / kWave;
-  if (row >= j.rows) return;
+// A wave's row of up to 64 ids: each lane's rank by comparison; up to 1,024: the same over
+// tiles of 64; longer: three passes of a stable radix sort of the row (digit counts in LDS,
+// ranks within a wave by ballots).
+__device__ inline void plan_sort_row(int32_t* a, int32_t* b, int len, int digit, int32_t* h) {
   const int lane = threadIdx.x % kWave;
-  const int r0 = __builtin_amdgcn_readfirstlane(j.ptr[row]);
-  const int len = __builtin_amdgcn_readfirstlane(j.ptr[row + 1]) - r0;
-  int32_t* a = j.tmp + r0;
-  int32_t* b = j.perm + r0;
   if (len <= kWave) {
     const int32_t id = lane < len ? a[lane] : 0x7fffffff;
     int rank = 0;
@@ -1081,16 +1084,25 @@ __global__ __launch_bounds__(kPlanWaves* kWave) void plan_row_sort_kernel(
     if (lane < len) b[rank] = id;
     return;
   }
-  if (len <= 1024) {
-    for (int t = lane; t < len; t += kWave) {
-      const int32_t id = a[t];
-      int rank = 0;
-      for (int k = 0; k < len; ++k) rank += a[k] < id ? 1 : 0;
+  if (len <= kPlanRowShort) {
+    // read once into LDS (the digit counts' place), from which four ids at a time go to all lanes
+    const int whole = (len + 3) & ~3;
+    for (int t = lane; t < whole; t += kWave) h[t] = t < len ? a[t] : 0x7fffffff;
+    wave_sync();
+    for (int t = lane; t < len; t += 2 * kWave) {
+      const bool two = t + kWave < len;
+      const int32_t id = h[t], id2 = two ? h[t + kWave] : 0;
+      int rank = 0, rank2 = 0;
+      for (int k = 0; k < whole; k += 4) {
+        const int4 q = *reinterpret_cast<const int4*>(h + k);
+        rank += (q.x < id) + (q.y < id) + (q.z < id) + (q.w < id);
+        rank2 += (q.x < id2) + (q.y < id2) + (q.z < id2) + (q.w < id2);
+      }
       b[rank] = id;
+      if (two) b[rank2] = id2;
     }
     return;
   }
-  int32_t* h = hist[threadIdx.x / kWave];
   const int bins = 1 << digit, per = (bins + kWave - 1) / kWave;
   for (int pass = 0; pass < 3; ++pass) {
     const int low = pass * digit;
@@ -1139,17 +1151,147 @@ __global__ __launch_bounds__(kPlanWaves* kWave) void plan_row_sort_kernel(
   }
 }
 
-__global__ void plan_iota_kernel(int32_t* __restrict__ iota, int64_t n) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e < n) iota[e] = (int32_t)e;
+// exclusive sum of v over the workgroup's threads, and the total; every thread calls it
+__device__ inline int32_t plan_block_scan(int32_t v, int32_t* wsum, int32_t& total) {
+  const int lane = threadIdx.x % kWave, w = threadIdx.x / kWave;
+  int32_t x = v;
+#pragma unroll
+  for (int o = 1; o < kWave; o <<= 1) {
+    const int32_t y = __shfl_up(x, o, kWave);
+    if (lane >= o) x += y;
+  }
+  __syncthreads();                                  // wsum's last reads
+  if (lane == kWave - 1) wsum[w] = x;
+  __syncthreads();
+  int32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (int k = 0; k < kPlanWaves; ++k) {
+    if (k < w) before += wsum[k];
+    total += wsum[k];
+  }
+  return before + x - v;
+}
+
+// A long row by the whole workgroup: its ids are put into windows of kPlanWindow ids (counts
+// and places in LDS), then each window's are marked in a bitmap and read off in order.
+__device__ inline void plan_sort_long_row(int32_t* __restrict__ a, int32_t* __restrict__ b,
+                                          int32_t len, int windows, int32_t* lds, int32_t* wsum) {
+  constexpr int kPer = kPlanLds / kPlanThreads;
+  const int t = threadIdx.x, lane = t % kWave, w = t / kWave;
+  const int32_t* ids = a;
+  if (windows > 1) {
+    for (int k = t; k < kPlanLds; k += kPlanThreads) lds[k] = 0;
+    __syncthreads();
+#pragma unroll 8
+    for (int32_t k = t; k < len; k += kPlanThreads) atomicAdd(&lds[a[k] >> kPlanWindowBits], 1);
+    __syncthreads();
+    int32_t n[kPer], sum = 0, total;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) sum += n[q] = lds[t * kPer + q];
+    int32_t at = plan_block_scan(sum, wsum, total);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      lds[t * kPer + q] = at;
+      at += n[q];
+    }
+    __syncthreads();
+#pragma unroll 8
+    for (int32_t k = t; k < len; k += kPlanThreads) {
+      const int32_t id = a[k];
+      b[atomicAdd(&lds[id >> kPlanWindowBits], 1)] = id;
+    }
+    __syncthreads();
+    for (int k = t; k < windows; k += kPlanThreads) a[k] = lds[k];   // the windows' ends
+    ids = b;
+  }
+  int32_t begin = 0;
+  for (int win = 0; win < windows; ++win) {
+    __syncthreads();                                // a's ends; the bitmap's last reads
+    const int32_t end = windows > 1 ? a[win] : len;
+    if (end == begin) continue;                     // uniform
+    for (int k = t; k < kPlanLds; k += kPlanThreads) lds[k] = 0;
+    __syncthreads();
+#pragma unroll 8
+    for (int32_t k = begin + t; k < end; k += kPlanThreads) {
+      const int32_t low = ids[k] & (kPlanWindow - 1);
+      atomicOr(&lds[low >> 5], 1 << (low & 31));
+    }
+    __syncthreads();
+    // wave w reads words [w kPer kWave, ..) in kPer rounds of one word a lane
+    int32_t n[kPer], sum = 0, total;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) sum += n[q] = __popc((unsigned)lds[(w * kPer + q) * kWave + lane]);
+    int32_t at = begin + __shfl(plan_block_scan(sum, wsum, total), 0, kWave);
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+      int32_t x = n[q];
+#pragma unroll
+      for (int o = 1; o < kWave; o <<= 1) {
+        const int32_t y = __shfl_up(x, o, kWave);
+        if (lane >= o) x += y;
+      }
+      const int word = (w * kPer + q) * kWave + lane;
+      int32_t to = at + x - n[q];
+      for (unsigned bits = (unsigned)lds[word]; bits != 0; bits &= bits - 1)
+        b[to++] = win * kPlanWindow + 32 * word + __ffs(bits) - 1;
+      at += __shfl(x, kWave - 1, kWave);
+    }
+    begin = end;
+  }
+}
+
+__device__ inline bool plan_long_row(int32_t len, int windows) {
+  return len > kPlanRowShort && len >= kPlanWindowShare * windows;
+}
+
+// The scattered ids of each row in ascending order: blocks [0, row_blocks) a wave a row, the
+// kPlanLongBlocks after them the long rows, a workgroup each: a wave takes 24 ns an id, so one row
+// could hold up the plan. Whole plans of 1,000,000 edges with one row of 16,000 ids: 835 -> 374
+// us, of 500,000: 20.3 -> 4.5 ms, most of it the row's atomics (sorting the list by a library
+// radix sort: 678 us, 6.2 ms); 40 rows of 25,000: 2.5 ms (2.9). kPlanWindowShare: of 4,000,000
+// edges (16 windows) a row of 2,000 ids takes 393 us by a wave and 529 by a workgroup, one of
+// 8,000 takes 648 and 570.
+__global__ __launch_bounds__(kPlanThreads) void plan_row_sort_kernel(
+    PlanJobs J, const int32_t* __restrict__ grouping, int digit, int64_t row_blocks) {
+  __shared__ __attribute__((aligned(16))) int32_t lds[kPlanLds];
+  const PlanJob& j = J.job[blockIdx.y];
+  if (blockIdx.y == kJobReceiver && !(*grouping & kFlagUngrouped)) return;   // uniform
+  const int windows = (int)((j.items + kPlanWindow - 1) >> kPlanWindowBits);
+  if ((int64_t)blockIdx.x < row_blocks) {
+    const int w = threadIdx.x / kWave;
+    const int64_t row = (int64_t)blockIdx.x * kPlanWaves + w;
+    if (row >= j.rows) return;
+    const int r0 = __builtin_amdgcn_readfirstlane(j.ptr[row]);
+    const int len = __builtin_amdgcn_readfirstlane(j.ptr[row + 1]) - r0;
+    if (!plan_long_row(len, windows))
+      plan_sort_row(j.tmp + r0, j.perm + r0, len, digit, lds + (w << kPlanDigitMax));
+    return;
+  }
+  __shared__ int32_t wsum[kPlanWaves], rows[kPlanThreads], count;
+  const int64_t b = (int64_t)blockIdx.x - row_blocks;
+  for (int64_t base = 0; base < j.rows; base += kPlanLongBlocks * kPlanThreads) {
+    __syncthreads();
+    if (threadIdx.x == 0) count = 0;
+    __syncthreads();
+    const int64_t row = base + (int64_t)threadIdx.x * kPlanLongBlocks + b;
+    if (row < j.rows && plan_long_row(j.ptr[row + 1] - j.ptr[row], windows))
+      rows[atomicAdd(&count, 1)] = (int32_t)row;
+    __syncthreads();
+    const int n = count;                                            // uniform
+    for (int k = 0; k < n; ++k) {
+      const int32_t r0 = j.ptr[rows[k]], len = j.ptr[rows[k] + 1] - r0;
+      __syncthreads();
+      plan_sort_long_row(j.tmp + r0, j.perm + r0, len, windows, lds, wsum);
+    }
+  }
 }
 
 struct PlanWs {
-  size_t rank_src, tmp_src, tmp_dst, code, rank_vis, tmp_vis, ptr_vis, cnt, sums, grouping, cub,
-      cub_bytes, total;
+  size_t rank_src, rank_dst, tmp_src, tmp_dst, code, rank_vis, tmp_vis, ptr_vis, cnt, sums, grouping,
+      total;
   int64_t cnt_ints, bins, max_tiles;
   int bits;
-  bool library;
 };
 
 // bins of the visit order per structure: 8^bits, about one atom a bin or more, 2^21 in all
@@ -1166,10 +1308,10 @@ static PlanWs plan_ws_layout(int64_t E, int64_t n, int64_t n_graphs, bool visit)
     field = at;
     at += align_up(sizeof(int32_t) * (size_t)count);
   };
-  w.library = E > kPlanRowMax * n;
   w.bits = visit ? visit_bits(n, n_graphs) : 0;
   w.bins = visit ? n_graphs << (3 * w.bits) : 0;
   ints(w.rank_src, E);
+  ints(w.rank_dst, E);
   ints(w.tmp_src, E);
   ints(w.tmp_dst, E);
   if (visit) {
@@ -1183,15 +1325,6 @@ static PlanWs plan_ws_layout(int64_t E, int64_t n, int64_t n_graphs, bool visit)
   w.max_tiles = (std::max(n, w.bins) + kPlanTile - 1) / kPlanTile;
   ints(w.sums, 3 * w.max_tiles);
   ints(w.grouping, 1);
-  if (w.library) {
-    size_t sort_bytes = 0;
-    (void)hipcub::DeviceRadixSort::SortPairs(nullptr, sort_bytes, (int32_t*)nullptr,
-                                             (int32_t*)nullptr, (int32_t*)nullptr,
-                                             (int32_t*)nullptr, (int)E);
-    w.cub = at;
-    w.cub_bytes = align_up(sort_bytes + 256);
-    at += w.cub_bytes;
-  }
   w.total = at;
   return w;
 }
@@ -1225,9 +1358,10 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
   int32_t* cnt_dst = cnt + (n + 1);
   int32_t* sums = ws_at<int32_t>(ws, w.sums);
   int32_t* rank_src = ws_at<int32_t>(ws, w.rank_src);
+  int32_t* rank_dst = ws_at<int32_t>(ws, w.rank_dst);
   PlanJobs J{};
   J.job[0] = PlanJob{src, rank_src, cnt, ptr_src, ws_at<int32_t>(ws, w.tmp_src), perm_src, E, n};
-  J.job[1] = PlanJob{dst, nullptr, cnt_dst, ptr_dst, ws_at<int32_t>(ws, w.tmp_dst), perm_dst, E, n};
+  J.job[1] = PlanJob{dst, rank_dst, cnt_dst, ptr_dst, ws_at<int32_t>(ws, w.tmp_dst), perm_dst, E, n};
   int jobs = 2;
   A.bits = w.bits;
   if (visit != nullptr) {
@@ -1246,8 +1380,8 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
   const int64_t eb = grid_1d(E, 256), ab = atoms ? grid_1d(n, 256) : 0;
   if (eb + ab + (atoms ? 1 : 0) > 0)
     hipLaunchKernelGGL(plan_read_kernel, dim3((unsigned)(eb + ab + (atoms ? 1 : 0))), dim3(256), 0,
-                       s, edge_index, cell_shifts, E, n, src, dst, shift, rank_src, cnt, cnt_dst, A,
-                       eb, ab, flags, grouping);
+                       s, edge_index, cell_shifts, E, n, src, dst, shift, rank_src, rank_dst, cnt,
+                       cnt_dst, A, eb, ab, flags, grouping);
   XNN_LAUNCH_CHECK();
   if (n == 0) {   // no rows: the pointers' single entry
     hipLaunchKernelGGL(set_first_zero_kernel, dim3(1), dim3(1), 0, s, ptr_dst);
@@ -1261,20 +1395,6 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
   hipLaunchKernelGGL(plan_scan_kernel, dim3((unsigned)w.max_tiles, jobs), dim3(1024), 0, s, J, sums,
                      w.max_tiles);
   XNN_LAUNCH_CHECK();
-  if (w.library) {
-    // few, very long rows: the library's stable sort of (row, id); the job's buffers hold the
-    // ids (rank_src, read no more) and the sorted rows (tmp)
-    void* cub = ws_at<char>(ws, w.cub);
-    size_t bytes = w.cub_bytes;
-    const int bit = end_bit_for(n);
-    hipLaunchKernelGGL(plan_iota_kernel, dim3(grid_1d(E, 256)), dim3(256), 0, s, rank_src, E);
-    XNN_LAUNCH_CHECK();
-    for (int k = 0; k < 2; ++k)
-      XNN_HIP_CHECK(hipcub::DeviceRadixSort::SortPairs(cub, bytes, J.job[k].key, J.job[k].tmp, rank_src,
-                                                       J.job[k].perm, (int)E, 0, bit, s));
-    J.job[0].items = J.job[1].items = 0;    // the visit order, if any, is left
-    J.job[0].rows = J.job[1].rows = 0;
-  }
   const int64_t items = std::max(J.job[0].items, J.job[2].items);
   const int64_t rows = std::max(J.job[0].rows, J.job[2].rows);
   if (items > 0) {
@@ -1282,8 +1402,10 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
                        s, J, grouping);
     int digit = 1;
     while ((int64_t(1) << (3 * digit)) < items && digit < kPlanDigitMax) ++digit;
-    hipLaunchKernelGGL(plan_row_sort_kernel, dim3((unsigned)grid_1d(rows, kPlanWaves), jobs),
-                       dim3(kPlanWaves * kWave), 0, s, J, grouping, digit);
+    const int64_t row_blocks = grid_1d(rows, kPlanWaves);
+    const int64_t long_blocks = items > kPlanRowShort ? kPlanLongBlocks : 0;
+    hipLaunchKernelGGL(plan_row_sort_kernel, dim3((unsigned)(row_blocks + long_blocks), jobs),
+                       dim3(kPlanThreads), 0, s, J, grouping, digit, row_blocks);
     XNN_LAUNCH_CHECK();
   }
   return XNN_OK;
