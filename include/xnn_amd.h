@@ -694,7 +694,8 @@ int xnn_eeq_store_apply(const double* values, const xnn_eeq_tiles* tiles, int64_
  * 2 K nrhs) summed and weighted by weights (C, K) into out (2 C, 2 K nrhs) = [[gr, gi], [gi,
  * -gr]]. gather: out (N, nrhs) += sum_k pr y_re + pi y_im + diag v with y (N, 2 K nrhs).
  * step: a = rz / p.ap, x += a p, res -= a ap, z = inv_d res. project: t (n_low, nrhs) = U^T z,
- * U (N, n_low <= 2048), work the queried bytes. search: z -= inv_d U t (U NULL: not), p = z + (res.z / rz) p (first: p = z), new_state = (res.z, |res| <= tol as 0 or 1); state and
+ * U (N, n_low), work the queried bytes. search: z -= inv_d U t (U NULL: not), p = z +
+ * (res.z / rz) p (first: p = z), new_state = (res.z, |res| <= tol as 0 or 1); state and
  * new_state are 2 nrhs doubles each, a column whose state says done takes a = 0 and p = z.
  * sums: 512 nrhs doubles, the same for a step and the search after it. */
 int xnn_eeq_cg_spread(const double* pr, const double* pi, const double* v, int64_t n_nodes,

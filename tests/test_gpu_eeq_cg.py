@@ -58,3 +58,20 @@ def test_solves_against_the_matrix(n, cell):
         res = torch.linalg.vector_norm(cols - dense.A @ out, dim=0)
         # the recurrence's residual against the true one: rounding of the product
         assert (res <= tol + 1e-12 * float(dense.A.abs().max()) * torch.linalg.vector_norm(out, dim=0)).all()
+
+
+@pytest.mark.parametrize("vectors", [1024, 1025, 1500])
+@pytest.mark.parametrize("R", [1, 2])
+def test_low_rank_parts_beyond_the_lds(monkeypatch, vectors, R):
+    """2,048 columns of the preconditioner are the most that a workgroup's LDS takes."""
+    E, gen, args, alpha, cutoff = _system(300, 5)
+    monkeypatch.setattr(E, "LOW_K_VECTORS", vectors)
+    cg = E.IterativeEEQSystem(*args, alpha, cutoff)
+    assert cg.U.shape[1] == 2 * vectors
+    dense = E.LargeEEQSystem(*args, alpha, cutoff)
+    b = torch.randn(300, R, dtype=torch.float64, generator=gen).to(DEV)
+    tol = torch.full((R,), 1e-11, dtype=torch.float64, device=DEV)
+    out = torch.empty_like(b)
+    out[cg.order] = cg.conjugate_gradient(b[cg.order], tol)
+    res = torch.linalg.vector_norm(b - dense.A @ out, dim=0)
+    assert (res <= tol + 1e-12 * float(dense.A.abs().max()) * torch.linalg.vector_norm(out, dim=0)).all()

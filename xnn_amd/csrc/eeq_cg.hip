@@ -208,7 +208,7 @@ __global__ __launch_bounds__(kCgThreads) void cg_step_kernel(
 // part[block][l][r] = sum over the block's rows of U[i][l] z[i][r], a thread per column l
 constexpr int kLowBlocks = 512;       // two workgroups a compute unit
 constexpr int kLowRows = 32;          // rows staged at a time
-constexpr int kLowMax = 2048;         // columns of U: t in LDS
+constexpr int kLowLds = 2048;         // columns of U up to which t is in LDS (32 KB at most)
 
 static int low_blocks(int64_t n) {
   return (int)std::min<int64_t>(kLowBlocks, (n + kLowRows - 1) / kLowRows);
@@ -272,10 +272,11 @@ __global__ __launch_bounds__(kCgThreads) void cg_project_sum_kernel(const double
   }
 }
 
-// U NULL: no low-rank part. A wave per row, lanes over the columns of U, t in LDS
+// U NULL: no low-rank part. A wave per row, lanes over the columns of U, t in LDS (LDS) or from
+// L2
 constexpr int kDirThreads = 1024;
 
-template <int R>
+template <int R, bool LDS>
 __global__ __launch_bounds__(kDirThreads) void cg_direction_kernel(
     const double* __restrict__ U, const double* __restrict__ t, int L,
     const double* __restrict__ inv_d, const double* __restrict__ res, int64_t n,
@@ -290,8 +291,10 @@ __global__ __launch_bounds__(kDirThreads) void cg_direction_kernel(
 #pragma unroll
       for (int r = 0; r < R; ++r) s[r] = fma(res[i * R + r], z[i * R + r], s[r]);
   } else {
-    for (int e = threadIdx.x; e < L * R; e += kDirThreads) st[(e % R) * L + e / R] = t[e];
-    __syncthreads();
+    if constexpr (LDS) {
+      for (int e = threadIdx.x; e < L * R; e += kDirThreads) st[(e % R) * L + e / R] = t[e];
+      __syncthreads();
+    }
     const int lane = threadIdx.x & (kWave - 1);
     constexpr int kWaves = kDirThreads / kWave;
     for (int64_t i = (int64_t)blockIdx.x * kWaves + threadIdx.x / kWave; i < n;
@@ -303,7 +306,7 @@ __global__ __launch_bounds__(kDirThreads) void cg_direction_kernel(
       for (int l = lane; l < L; l += kWave) {
         const double x = U[i * L + l];
 #pragma unroll
-        for (int r = 0; r < R; ++r) u[r] = fma(x, st[r * L + l], u[r]);
+        for (int r = 0; r < R; ++r) u[r] = fma(x, LDS ? st[r * L + l] : t[l * R + r], u[r]);
       }
 #pragma unroll
       for (int m = kWave / 2; m > 0; m >>= 1)
@@ -428,7 +431,7 @@ int xnn_eeq_cg_project_work_size(int64_t n_nodes, int32_t n_low, int32_t nrhs, s
 int xnn_eeq_cg_project(const double* U, const double* z, int64_t n_nodes, int32_t n_low,
                        int32_t nrhs, double* t, void* work, size_t work_bytes,
                        xnn_stream_t stream) {
-  XNN_REQUIRE(n_nodes >= 1 && n_low >= 1 && n_low <= kLowMax, "size out of range");
+  XNN_REQUIRE(n_nodes >= 1 && n_low >= 1 && n_low < (1 << 29), "size out of range");
   XNN_REQUIRE(nrhs == 1 || nrhs == 2, "one or two right-hand sides (got %d)", (int)nrhs);
   XNN_REQUIRE(U && z && t && work, "NULL input, output or work");
   const int want = low_blocks(n_nodes), m = n_low * nrhs;
@@ -457,17 +460,17 @@ int xnn_eeq_cg_search(const double* U, const double* t, int32_t n_low, const dou
   XNN_REQUIRE(nrhs == 1 || nrhs == 2, "one or two right-hand sides (got %d)", (int)nrhs);
   XNN_REQUIRE(inv_d && res && tol && (first || state) && z && p && new_state && sums,
               "NULL input or output");
-  XNN_REQUIRE(U == nullptr || (t && n_low >= 1 && n_low <= kLowMax), "1 to %d low-rank columns", kLowMax);
+  XNN_REQUIRE(U == nullptr || (t && n_low >= 1 && n_low < (1 << 29)), "NULL t or size out of range");
   XNN_REQUIRE(state != new_state, "the state is read while the new one is written");
   hipStream_t s = as_hip(stream);
   if (first) XNN_CG(cg_dot_kernel, n_nodes, res, res, n_nodes, sums + nrhs * kCgBlocks);
-  const size_t lds = U != nullptr ? sizeof(double) * (size_t)n_low * nrhs : 0;   // at most 32 KB
-  if (nrhs == 1)
-    hipLaunchKernelGGL(cg_direction_kernel<1>, dim3((unsigned)cg_blocks(n_nodes)), dim3(kDirThreads), lds,
-                       s, U, t, (int)n_low, inv_d, res, n_nodes, z, sums);
-  else
-    hipLaunchKernelGGL(cg_direction_kernel<2>, dim3((unsigned)cg_blocks(n_nodes)), dim3(kDirThreads), lds,
-                       s, U, t, (int)n_low, inv_d, res, n_nodes, z, sums);
+  const bool low_lds = U != nullptr && n_low <= kLowLds;
+  const size_t lds = low_lds ? sizeof(double) * (size_t)n_low * nrhs : 0;
+  const auto direction =
+      nrhs == 1 ? (low_lds ? cg_direction_kernel<1, true> : cg_direction_kernel<1, false>)
+                : (low_lds ? cg_direction_kernel<2, true> : cg_direction_kernel<2, false>);
+  hipLaunchKernelGGL(direction, dim3((unsigned)cg_blocks(n_nodes)), dim3(kDirThreads), lds, s, U, t,
+                     (int)n_low, inv_d, res, n_nodes, z, sums);
   XNN_CG(cg_search_kernel, n_nodes, sums, sums + nrhs * kCgBlocks, tol, state, first != 0, z, n_nodes, p,
          new_state);
   return XNN_OK;
