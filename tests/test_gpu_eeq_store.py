@@ -75,3 +75,44 @@ def test_far_tiles_are_left_out_and_the_fallback_agrees(monkeypatch):
     q2, mu2 = free.solve_augmented(x, zero)
     # both to a residual of 1e-12 |x|, the operator's smallest eigenvalue of order one
     assert float((q - q2).abs().max()) <= 2e-11 * float(x.norm())
+
+
+def _charges(n, solver, seed=7):
+    from xnn_amd import eeq as E
+    pos, cell, rad, v = _system(n, seed)
+    diag = torch.full((n,), 3.0, dtype=torch.float64, device=DEV)
+    leaves = [pos.clone().requires_grad_(True), cell.clone().requires_grad_(True)]
+    q = E.eeq_charges_large(leaves[0], leaves[1], rad, diag, v[:, 0].contiguous(), 0.0, 24.0,
+                            solver=solver)
+    return q, leaves, v[:, 1]
+
+
+def test_values_are_given_back_between_the_solves(monkeypatch):
+    """Neither the graph nor a second backward through it keeps the stored values."""
+    from xnn_amd import eeq as E
+    made = []
+    form = E.IterativeEEQSystem._form_store
+    monkeypatch.setattr(E.IterativeEEQSystem, "_form_store", lambda s: (made.append(s), form(s))[1])
+    q, leaves, u = _charges(300, "cg")
+    assert len(made) == 1 and made[0].store is None
+    got = torch.autograd.grad([q], leaves, [u], retain_graph=True)
+    assert len(made) == 2 and made[1] is made[0] and made[0].store is None
+    again = torch.autograd.grad([q], leaves, [u])
+    assert len(made) == 3 and made[0].store is None
+    ref_q, ref_leaves, _ = _charges(300, "lu")
+    want = torch.autograd.grad([ref_q], ref_leaves, [u])
+    # both solved to 1e-12 of the right-hand side, eigenvalues of order one
+    torch.testing.assert_close(q, ref_q, rtol=0, atol=1e-10)
+    for a, b, c in zip(got, again, want):
+        assert torch.equal(a, b)
+        torch.testing.assert_close(a, c, rtol=0, atol=1e-9 * float(c.abs().max()))
+
+
+def test_values_take_at_most_half_of_the_memory_left(monkeypatch):
+    from xnn_amd import eeq as E
+    pos, cell, rad, _ = _system(300)
+    args = (pos, E._host_cell(cell), rad, E.ewald_alpha(30.0), 30.0)
+    need = 8 * (E.RealTiles.build(*args).values.numel() - 1)
+    for left, kept in ((2 * need, True), (2 * need - 2, False)):
+        monkeypatch.setattr(E, "_device_left", lambda dev: left)
+        assert (E.RealTiles.build(*args) is not None) == kept

@@ -48,9 +48,9 @@ TABLE_BUDGET = 1 << 28
 #: (N, G) entries per block of the differentiable reciprocal sum (recomputed in the
 #: backward)
 LIVE_BUDGET = 1 << 23
-#: bytes of real-space values the conjugate-gradient regime keeps (8.2 B per unordered pair
-#: in reach: 1.3 GB at 24,000 atoms and 60 bohr); beyond it, or when the device has not that
-#: much left, every product evaluates its pairs again
+#: bytes of real-space values the conjugate-gradient regime keeps during its solves (8.2 B per
+#: unordered pair in reach: 1.3 GB at 24,000 atoms and 60 bohr); beyond it, or beyond half of
+#: what the device has left, every product evaluates its pairs again
 STORE_BYTES = 32 << 30
 STORE_TILE = 128
 #: reciprocal vectors (smallest |G|, largest weights) in the low-rank part of the
@@ -257,6 +257,12 @@ def real_apply(pos: Tensor, cell, rad: Tensor, alpha: float, cutoff_au: float,
     return out
 
 
+def _device_left(device) -> int:
+    """Bytes that allocations on ``device`` can still take: free, or kept by the allocator."""
+    return (torch.cuda.mem_get_info(device)[0] + torch.cuda.memory_reserved(device)
+            - torch.cuda.memory_allocated(device))
+
+
 class RealTiles:
     """The real-space matrix of ``N`` spatially ordered atoms, evaluated once: of the lower
     128 x 128 tiles the pairs with an image within the cutoff (``xnn_eeq_store_tiles``)."""
@@ -267,7 +273,7 @@ class RealTiles:
     @classmethod
     def build(cls, pos: Tensor, host_cell, rad: Tensor, alpha: float,
               cutoff_au: float) -> Optional["RealTiles"]:
-        """None where the values exceed :data:`STORE_BYTES` or do not fit the device."""
+        """None where the values exceed :data:`STORE_BYTES` or half of the device's memory left."""
         n, dev = int(pos.shape[0]), pos.device
         nt = -(-n // STORE_TILE)
         if n == 0 or nt * nt > 1 << 26:
@@ -299,7 +305,7 @@ class RealTiles:
             end = torch.cumsum(counts, 0)
             base = end - counts
             total = int(end[-1])
-            if total * 8 > STORE_BYTES:
+            if total * 8 > min(STORE_BYTES, _device_left(dev) // 2):
                 return None
             # one more: a tile without values starts at their end
             values = torch.empty(total + 1, dtype=torch.float64, device=dev)
@@ -499,6 +505,9 @@ class LargeEEQSystem:
             y1 = self._solve(b)[:, 0]
         mu = (y1.sum() - bottom) / self.y_ones.sum()
         return y1 - mu * self.y_ones, mu
+
+    def release(self) -> None:
+        """Nothing: the factor serves the backward's solve too."""
 
     def apply(self, v: Tensor) -> Tensor:
         """``A v`` at the detached geometry."""
@@ -736,9 +745,18 @@ class IterativeEEQSystem:
             self.inv_d = (1.0 / full[self.order]).contiguous()
         self.y_ones = None
         self.iterations = []                   # per conjugate-gradient solve
+        self._work = None
+        self._form_store()
+
+    def _form_store(self) -> None:
+        self.released = False
         self.store = (RealTiles.build(self.pos_s, self.cell_host, self.rad_s, self.alpha, self.cutoff)
                       if self.pos_s.is_cuda else None)
-        self._work = None
+
+    def release(self) -> None:
+        """Give the stored values back until the next solve, which forms them again (4 of the
+        44 ms of 24,000 atoms): nothing of their size waits for a backward pass."""
+        self.store, self._work, self.released = None, None, True
 
     def _low_rank(self, full_s: Tensor) -> None:
         """The preconditioner ``M = D + U W U^T`` (dispersion_fast/eeq.py:72-86): ``U = [cos,
@@ -772,6 +790,8 @@ class IterativeEEQSystem:
 
     def _matvec(self, v: Tensor) -> Tensor:
         """``A v`` in the spatial order, ``v`` (N, 1 or 2)."""
+        if self.released:
+            self._form_store()
         if self.store is not None:
             out = self.store.apply(v)
         else:
@@ -945,6 +965,7 @@ class _ConstantSolve(torch.autograd.Function):
     def backward(ctx, g):
         lam, kappa = ctx.system.solve_augmented(g, torch.zeros((), dtype=torch.float64,
                                                                device=g.device))
+        ctx.system.release()
         return None, lam.to(g.dtype), kappa.to(g.dtype)
 
 
@@ -978,6 +999,7 @@ def eeq_charges_large(pos: Tensor, cell: Optional[Tensor], rad: Tensor, diag: Te
         tol_abs = CG_TOL * float(torch.linalg.vector_norm(xd)) if iterative else None
         dq, dmu = system.solve_augmented(xd - system.apply(q0) - mu0, total - q0.sum(), tol_abs)
         q1, mu1 = q0 + dq, mu0 + dmu
+        system.release()
     live = x.requires_grad or pos.requires_grad or (periodic and cell.requires_grad)
     if not (live and torch.is_grad_enabled()):
         return q1.to(x.dtype)
