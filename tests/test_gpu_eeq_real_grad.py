@@ -43,3 +43,34 @@ def test_pairs_match_the_directed_sum(n, kind):
     if want:
         assert torch.equal(outs[0][1], outs[1][1])
         torch.testing.assert_close(outs[0][1], rows.sum(0), rtol=0, atol=tol * n)
+
+
+def test_without_room_for_the_pairs_the_directed_kernel_runs(monkeypatch):
+    from xnn_amd import _lib, eeq as E
+    gen = torch.Generator().manual_seed(1)
+    cell = 12.0 * torch.eye(3, dtype=torch.float64)
+    pos = (torch.rand(100, 3, dtype=torch.float64, generator=gen) * 12.0).to(DEV)
+    rad, u, v = (torch.rand(100, dtype=torch.float64, generator=gen).to(DEV) for _ in range(3))
+
+    def grads():
+        leaves = [pos.clone().requires_grad_(True), cell.to(DEV).requires_grad_(True)]
+        out = E.real_apply_op(leaves[0], leaves[1], rad, v, None, E.ewald_alpha(20.0), 20.0)
+        return torch.autograd.grad([out], leaves, [u])
+
+    want = grads()
+    need, empty = ctypes.c_size_t(0), torch.empty
+    _lib.call("xnn_eeq_real_grad_pairs_work_size", 100, ctypes.byref(need))
+
+    def full(*args, **kw):
+        if args[0] == need.value:
+            raise torch.cuda.OutOfMemoryError("no room")
+        return empty(*args, **kw)
+
+    before = _lib.calls.get("xnn_eeq_real_grad", 0)
+    monkeypatch.setattr(torch, "empty", full)
+    got = grads()
+    monkeypatch.undo()
+    assert _lib.calls.get("xnn_eeq_real_grad", 0) == before + 1
+    # as above: terms of order one, a hundred of them an atom
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a, b, rtol=0, atol=1e-14 * 16 * 100 * 100)

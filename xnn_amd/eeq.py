@@ -333,7 +333,8 @@ def real_apply_op(pos: Tensor, cell: Optional[Tensor], rad: Tensor, v: Tensor,
                   matrix: Optional[Tensor], alpha: float, cutoff_au: float) -> Tensor:
     """``R(pos, cell) v`` with the matrix formed at these positions, or without a matrix
     (``matrix`` None: the matrix-free HIP product); differentiable in ``pos`` and ``cell``
-    through ``xnn_eeq_real_grad_pairs`` (``v`` is held constant)."""
+    through ``xnn_eeq_real_grad_pairs``, or without its workspace (up to 1.2 GB)
+    ``xnn_eeq_real_grad`` (``v`` is held constant)."""
     if matrix is not None:
         return matrix @ v
     return real_apply(pos, cell, rad, alpha, cutoff_au, v.reshape(-1, 1)).reshape(v.shape)
@@ -348,6 +349,14 @@ def _real_apply_setup(ctx, inputs, output):
     pos, cell, rad, v, matrix, alpha, cutoff_au = inputs
     ctx.save_for_backward(pos, cell, rad, v)
     ctx.alpha, ctx.cutoff = alpha, cutoff_au
+
+
+def _room(n_bytes: int, device) -> Optional[Tensor]:
+    """A workspace, or None for no bytes or where the device has not that much left."""
+    try:
+        return torch.empty(n_bytes, dtype=torch.uint8, device=device) if n_bytes else None
+    except torch.cuda.OutOfMemoryError:
+        return None
 
 
 def _real_apply_backward(ctx, grad):
@@ -366,8 +375,8 @@ def _real_apply_backward(ctx, grad):
     g_cell = None
     need = ctypes.c_size_t(0)
     _lib.call("xnn_eeq_real_grad_pairs_work_size", n, ctypes.byref(need))
-    if need.value:
-        work = torch.empty(need.value, dtype=torch.uint8, device=dev)
+    work = _room(need.value, dev)
+    if work is not None:
         g_cell = torch.empty(9, dtype=torch.float64, device=dev) if want_cell else None
         _lib.call("xnn_eeq_real_grad_pairs", *args, _lib.ptr(g_cell), _lib.ptr(work),
                   int(work.numel()), _lib.stream(dev))
