@@ -51,3 +51,14 @@ def test_readout_weight_gradient(n, F, dtype, broadcast):
     # summed in float64 and rounded once
     bound = eps * want.abs() + (n + 1) * 2.3e-16 * (rows.double().abs().t() @ g.double().abs())
     assert ((got.cpu().double() - want).abs() <= bound).all()
+
+
+def test_readout_weight_gradient_of_a_batch_of_cotangents():
+    from xnn_amd.ops import node_readout_op
+    gen = torch.Generator().manual_seed(1)
+    rows, w, g = (torch.randn(*k, generator=gen).to(DEV) for k in ((50, 33), (33,), (4, 50)))
+    w.requires_grad_(True)
+    E = node_readout_op(rows, w, torch.zeros(50, dtype=torch.int64, device=DEV), torch.zeros(1, device=DEV))
+    (got,) = torch.autograd.grad([E], [w], [g], is_grads_batched=True)
+    bound = 52 * EPS * (g.double().abs() @ rows.double().abs())       # float32 products and sums
+    assert ((got.double() - g.double() @ rows.double()).abs() <= bound).all()

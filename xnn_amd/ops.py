@@ -975,9 +975,10 @@ def _readout_setup(ctx, inputs, output):
     ctx.n_bias, ctx.bias_dtype, ctx.weight_dtype = bias.shape[0], bias.dtype, weight.dtype
 
 
-def _readout_weight_grad(rows: Tensor, grad: Tensor) -> Tensor:
-    if rows.dtype != grad.dtype:
-        return rows.t() @ grad
+@torch.library.custom_op(f"{_NS}::node_readout_wgrad", mutates_args=())
+def node_readout_wgrad_op(rows: Tensor, grad: Tensor) -> Tensor:
+    """``rows^T grad`` (F,) of one dtype, summed in float64 (``xnn_node_readout_wgrad``, HIP); an
+    op, so that a batch of cotangents goes through it one by one."""
     F = rows.shape[1]
     rows = rows.contiguous()
     g = grad if (grad.dim() == 1 and grad.stride(0) == 0) else grad.contiguous()
@@ -987,6 +988,15 @@ def _readout_weight_grad(rows: Tensor, grad: Tensor) -> Tensor:
               _lib.ptr(g), 0 if g.stride(0) == 0 else 1, _lib.ptr(out), _lib.ptr(work),
               int(work.numel()), _lib.stream(rows.device))
     return out
+
+
+@node_readout_wgrad_op.register_fake
+def _(rows, grad):
+    return rows.new_empty(rows.shape[1])
+
+
+def _readout_weight_grad(rows: Tensor, grad: Tensor) -> Tensor:
+    return node_readout_wgrad_op(rows, grad) if rows.dtype == grad.dtype else rows.t() @ grad
 
 
 def _readout_backward(ctx, grad):
