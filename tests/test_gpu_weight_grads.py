@@ -62,3 +62,19 @@ def test_readout_weight_gradient_of_a_batch_of_cotangents():
     (got,) = torch.autograd.grad([E], [w], [g], is_grads_batched=True)
     bound = 52 * EPS * (g.double().abs() @ rows.double().abs())       # float32 products and sums
     assert ((got.double() - g.double() @ rows.double()).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("l_max", [1, 2, 3])
+def test_linear_message_weight_gradient_of_a_misaligned_cotangent(l_max):
+    """A cotangent that is a view one float into other memory is the same as any other."""
+    from xnn_amd.ops import sh_linear_message_sum_op
+    gen = torch.Generator().manual_seed(2)
+    vec, h, W = (torch.randn(*k, generator=gen).to(DEV) for k in ((60, 3), (60, 8), (8, 32)))
+    ptr = torch.arange(0, 61, 6, dtype=torch.int32, device=DEV)
+    W.requires_grad_(True)
+    A = sh_linear_message_sum_op(vec, h, W, ptr, None, l_max, 1)
+    G = torch.randn(A.shape, generator=gen).to(DEV)
+    view = torch.empty(A.numel() + 1, device=DEV)[1:].view_as(A).copy_(G)
+    assert view.data_ptr() % 16
+    want, got = (torch.autograd.grad([A], [W], [k], retain_graph=True)[0] for k in (G, view))
+    assert torch.equal(got, want)

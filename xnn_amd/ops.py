@@ -602,6 +602,8 @@ def _lin_msg_backward(ctx, d_out):
     d_W = None
     if need_W:
         d_W = torch.empty_like(W)
+        if d_out.data_ptr() % 16:              # a view into other memory; the kernel reads float4
+            d_out = d_out.clone()
         work = _work("xnn_sh_linear_message_wgrad_work_size", dev, n_nodes, K, C)
         _lib.call("xnn_sh_linear_message_wgrad", _lib.ptr(vec), n_nodes, vec.shape[0],
                   _lib.ptr(ptr_dst), _lib.ptr(perm_dst), ctx.l_max, ctx.sh_sign, K, C, _lib.ptr(h),
