@@ -98,3 +98,16 @@ def test_an_unsymmetric_table_takes_the_general_kernel():
     assert not XD.DFTD3(tables)._pair_tiles
     assert not XD.DFTD3(XD.load_d3_tables(os.path.join(GOLDEN, "d3_tables_hcnoar.npz")),
                         damping="zero")._pair_tiles
+
+
+@pytest.mark.parametrize("damping", ["zero", "mzero", "op"])
+def test_a_damping_set_afterwards_is_the_one_used(damping):
+    import xnn_amd.dispersion as XD
+    tables = XD.load_d3_tables(os.path.join(GOLDEN, "d3_tables_hcnoar.npz"))
+    z, pos, _ = _inputs([30], False)
+    args = (torch.tensor(z, device=DEV), torch.tensor(pos, device=DEV), None, None, torch.tensor([30]))
+    later, model = XD.DFTD3(tables).to(DEV), XD.DFTD3(tables, damping=damping).to(DEV)
+    later.damping = damping
+    later.s6, later.s8, later.a1, later.a2 = model.s6, model.s8, model.a1, model.a2
+    later.rs6, later.rs8, later.alp, later.bet = model.rs6, model.rs8, model.alp, model.bet
+    assert torch.equal(later.evaluate(*args)["node_energy"], model.evaluate(*args)["node_energy"])

@@ -1531,8 +1531,8 @@ class DFTD3(nn.Module):
         self.register_buffer("c6pair", torch.as_tensor(
             np.ascontiguousarray(np.asarray(tables["c6ref"]).transpose(2, 3, 0, 1)),
             dtype=torch.float64), persistent=False)
-        # the pair tiles take each unordered pair once: the rational damping, and a reference
-        # block that does not change when its two atoms change places
+        # the pair tiles take each unordered pair once: the rational damping (asked again at each
+        # call), and a reference block that does not change when its two atoms change places
         c6 = np.asarray(tables["c6ref"])
         self._pair_tiles = (damping == "bj" and len(self.elements) <= D3_TILE_SPECIES
                             and bool(np.array_equal(c6, c6.transpose(1, 0, 3, 2))))
@@ -1584,7 +1584,7 @@ class DFTD3(nn.Module):
         wants_grad = torch.is_grad_enabled() and (
             pos.requires_grad or (cell64 is not None and cell64.requires_grad))
         e2_b = None
-        plan = plan if self._pair_tiles else None
+        plan = plan if self._pair_tiles and self.damping == "bj" else None
         if fused_pair and wants_grad:
             e2_b, e2 = D3TwoBodyStructureEnergy.apply(
                 pos.contiguous(), cell64, w, species, batch32, node_ptr, images, self.r4r2,
