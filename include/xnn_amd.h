@@ -743,7 +743,8 @@ int xnn_eeq_recip_backward(const double* pos, int64_t n_nodes, const double* g, 
  * the trailing updates of the blocks before it. Written in place: the block's factor L
  * (lower; its upper triangle zeroed), and inv (b, b) = L^-1 (row-major, lower) for the
  * panel product L21 = A21 inv^T. A pivot that is not positive and finite stores k0 + j + 1 into the
- * device int *info when that still holds 0, and leaves the block unwritten. */
+ * device int *info when that still holds 0, and leaves the block unwritten. For a caller with
+ * trailing updates of its own; xnn_eeq_cholesky does the whole. */
 int xnn_eeq_cholesky_block(double* matrix, int64_t n, int64_t k0, int64_t b, double* inv,
                            int* info, xnn_stream_t stream);
 
@@ -755,9 +756,9 @@ int xnn_eeq_cholesky(double* matrix, int64_t n, double* inv_blocks, int* info,
                      xnn_stream_t stream);
 
 /* (L L^T) X = B in place: X (n, nrhs) row-major float64 on entry B, nrhs 1 or 2; L the
- * factor that xnn_eeq_cholesky_block left in the matrix (row-major, lower), inv_blocks the
+ * factor that xnn_eeq_cholesky left in the matrix (row-major, lower), inv_blocks the
  * inverses of its diagonal blocks (block j of rows [128 j, 128 j + b_j) at inv_blocks +
- * 128 * 128 j, row stride b_j, as xnn_eeq_cholesky_block wrote them); work: n * nrhs
+ * 128 * 128 j, row stride b_j, as it wrote them); work: n * nrhs
  * doubles. Blocked forward and backward substitution, one launch per block and direction;
  * sums in a fixed order. Stands in for the factorized solves of the large regime
  * (eeq.py:117-140: torch.linalg.lu_solve on the LU factors), here with the Cholesky factor

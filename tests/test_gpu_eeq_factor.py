@@ -36,3 +36,25 @@ def test_first_bad_pivot(at, value):
     A[299, 299] = min(float(A[299, 299]), -1.0) if value == value else -1.0
     _, info = _cholesky(A.to(DEV))
     assert int(info) == at + 1
+
+
+@pytest.mark.parametrize("k0,b", [(0, 128), (128, 128), (256, 44), (7, 1), (100, 77)])
+def test_one_block(k0, b):
+    """``xnn_eeq_cholesky_block`` by itself, anywhere in the matrix, and nothing beside it."""
+    from xnn_amd import _lib
+    g = torch.Generator().manual_seed(b)
+    M = torch.randn((300, 300), dtype=torch.float64, generator=g)
+    A = M @ M.T + 300 * torch.eye(300, dtype=torch.float64)
+    got, inv = A.to(DEV), torch.empty(b, b, dtype=torch.float64, device=DEV)
+    info = torch.zeros(1, dtype=torch.int32, device=DEV)
+    _lib.call("xnn_eeq_cholesky_block", _lib.ptr(got), 300, k0, b, _lib.ptr(inv), _lib.ptr(info),
+              _lib.stream(got.device))
+    want = torch.linalg.cholesky(A[k0:k0 + b, k0:k0 + b])
+    tol = 4 * b * torch.finfo(torch.float64).eps             # as above
+    block = got.cpu()[k0:k0 + b, k0:k0 + b]
+    torch.testing.assert_close(block, want, rtol=0, atol=tol * float(want.abs().max()))
+    inverse = torch.linalg.inv(want)
+    torch.testing.assert_close(inv.cpu(), inverse, rtol=0, atol=tol * float(inverse.abs().max()))
+    rest = got.cpu()
+    rest[k0:k0 + b, k0:k0 + b] = A[k0:k0 + b, k0:k0 + b]
+    assert int(info) == 0 and torch.equal(rest, A)

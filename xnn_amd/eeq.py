@@ -680,7 +680,8 @@ class FactorizedReciprocal:
         return out
 
     def apply(self, v: Tensor) -> Tensor:
-        """``A_rec v`` for ``v`` (N, R)."""
+        """``A_rec v`` for ``v`` (N, R) in tensor operations, on any device: the reference of
+        :meth:`add_to`, which the solves call."""
         n, R = v.shape
         K, KR = self.K, self.K * v.shape[1]
         pr, pi = self.tables[2]
