@@ -362,6 +362,15 @@ def transformed(*tensors: Optional[torch.Tensor]) -> bool:
         for t in tensors if t is not None)
 
 
+def addressable(t: torch.Tensor) -> bool:
+    """Whether the tensor has storage: not the wrapper of a batch (of cotangents, say)."""
+    try:
+        t.data_ptr()
+    except RuntimeError:
+        return False
+    return True
+
+
 def stream(device: torch.device) -> int:
     """The current HIP stream of ``device`` as an integer handle."""
     return torch.cuda.current_stream(device).cuda_stream

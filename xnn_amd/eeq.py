@@ -163,12 +163,10 @@ def _recip_work(n: int, m: int, backward: bool, device) -> Tensor:
     return torch.empty(need.value, dtype=torch.uint8, device=device)
 
 
-@torch.library.custom_op(f"{_NS}::eeq_reciprocal_backward", mutates_args=())
-def reciprocal_backward_op(pos: Tensor, g: Tensor, w: Tensor, v: Tensor, factors: Tensor, u: Tensor,
-                           cell_side: bool) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
+def _reciprocal_grads(pos: Tensor, g: Tensor, w: Tensor, v: Tensor, factors: Tensor, u: Tensor,
+                      cell_side: bool) -> Tuple[Tensor, Tensor, Tensor, Tensor]:
     """The gradients of :func:`reciprocal_op` in ``pos``, ``g``, ``w`` (zeros unless
-    ``cell_side``) and ``v`` for the output's gradient ``u``; an op, so that a batch of ``u``
-    goes through it one by one."""
+    ``cell_side``) and ``v`` for the output's gradient ``u``."""
     n, m = int(pos.shape[0]), int(g.shape[0])
     u = u.contiguous()
     grads = [torch.zeros_like(t) for t in (pos, g, w, v)]
@@ -178,6 +176,11 @@ def reciprocal_backward_op(pos: Tensor, g: Tensor, w: Tensor, v: Tensor, factors
               _lib.ptr(grads[1] if cell_side else None), _lib.ptr(grads[2] if cell_side else None),
               _lib.ptr(grads[3]), _lib.ptr(work), int(work.numel()), _lib.stream(pos.device))
     return tuple(grads)
+
+
+# as an op, which a batch of cotangents goes through one by one
+reciprocal_backward_op = torch.library.custom_op(f"{_NS}::eeq_reciprocal_backward",
+                                                 mutates_args=())(_reciprocal_grads)
 
 
 @reciprocal_backward_op.register_fake
@@ -203,7 +206,8 @@ def _reciprocal_backward(ctx, u, _factors):
         grads = iter(torch.autograd.grad([out], wanted, [u], create_graph=True))
         return tuple(next(grads) if need else None for need in ctx.needs_input_grad)
     cell_side = ctx.needs_input_grad[1] or ctx.needs_input_grad[2]
-    grads = reciprocal_backward_op(pos, g, w, v, factors, u, cell_side)
+    form = _reciprocal_grads if _lib.addressable(u) else reciprocal_backward_op
+    grads = form(pos, g, w, v, factors, u, cell_side)
     return tuple(t if need else None for t, need in zip(grads, ctx.needs_input_grad))
 
 

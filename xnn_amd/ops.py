@@ -977,10 +977,8 @@ def _readout_setup(ctx, inputs, output):
     ctx.n_bias, ctx.bias_dtype, ctx.weight_dtype = bias.shape[0], bias.dtype, weight.dtype
 
 
-@torch.library.custom_op(f"{_NS}::node_readout_wgrad", mutates_args=())
-def node_readout_wgrad_op(rows: Tensor, grad: Tensor) -> Tensor:
-    """``rows^T grad`` (F,) of one dtype, summed in float64 (``xnn_node_readout_wgrad``, HIP); an
-    op, so that a batch of cotangents goes through it one by one."""
+def _readout_wgrad(rows: Tensor, grad: Tensor) -> Tensor:
+    """``rows^T grad`` (F,) of one dtype, summed in float64 (``xnn_node_readout_wgrad``, HIP)."""
     F = rows.shape[1]
     rows = rows.contiguous()
     g = grad if (grad.dim() == 1 and grad.stride(0) == 0) else grad.contiguous()
@@ -992,13 +990,20 @@ def node_readout_wgrad_op(rows: Tensor, grad: Tensor) -> Tensor:
     return out
 
 
+# as an op, which a batch of cotangents goes through one by one
+node_readout_wgrad_op = torch.library.custom_op(f"{_NS}::node_readout_wgrad",
+                                                mutates_args=())(_readout_wgrad)
+
+
 @node_readout_wgrad_op.register_fake
 def _(rows, grad):
     return rows.new_empty(rows.shape[1])
 
 
 def _readout_weight_grad(rows: Tensor, grad: Tensor) -> Tensor:
-    return node_readout_wgrad_op(rows, grad) if rows.dtype == grad.dtype else rows.t() @ grad
+    if rows.dtype != grad.dtype:
+        return rows.t() @ grad
+    return (_readout_wgrad if _lib.addressable(grad) else node_readout_wgrad_op)(rows, grad)
 
 
 def _readout_backward(ctx, grad):
