@@ -153,3 +153,17 @@ def test_visit_order_of_one_crowded_bin():
     cell = torch.eye(3, device=DEV, dtype=torch.float64)[None] * 1e4
     assert torch.equal(build_plan(none, None, 30_000, pos=pos, cell=cell).visit.cpu(),
                        torch.arange(30_000, dtype=torch.int32))
+
+
+@pytest.mark.parametrize("n,e", [(1, 1), (64, 60), (65, 130), (1000, 3999), (1000, 4000), (40_000, 9000)])
+def test_rows_of_few_ids(n, e):
+    """A lane a row below four ids a row on the average; some rows are longer than its eight."""
+    from xnn_amd.plan import build_plan
+    rng = np.random.default_rng(n + e)
+    key, other = rng.integers(0, n, e), rng.integers(0, n, e)
+    key[rng.permutation(e)[:e // 3]] = n // 2
+    other[rng.permutation(e)[:min(e, 9)]] = n - 1
+    plan = build_plan(torch.tensor(np.stack([key, other]), device=DEV), None, n)
+    for k, perm in ((key, plan.perm_src), (other, plan.perm_dst)):
+        got = np.arange(e) if perm is None else perm.cpu()
+        assert np.array_equal(got, np.argsort(k, kind="stable"))
