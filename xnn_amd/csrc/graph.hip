@@ -775,22 +775,20 @@ __global__ __launch_bounds__(256) void molecule_search_kernel(
 // Bound by the sender counts' device-scope atomics (about one per edge) and, for small
 // lists, by the five launches. Measured against two library radix sorts, the per-edge
 // atomics of both orderings and the separate batch, grouping and Morton-order passes:
-// 620 -> 58 us of kernels (140 -> 6 launches) for 478k edges of 9,000 atoms, 1,116 -> 210 us
+// 620 -> 56 us of kernels (140 -> 6 launches) for 478k edges of 9,000 atoms, 1,116 -> 205 us
 // for 3.8M edges of 72,000 atoms (52 B read and 32 B written an edge: 1.5 TB/s there, the read
 // alone 2.6).
 constexpr int kPlanTile = 8192;       // counts scanned by one block
 constexpr int kPlanWaves = 4;         // rows sorted per block of the row sort
 constexpr int kPlanThreads = kPlanWaves * kWave;
-constexpr int kPlanDigitMax = 11;     // id bits per pass of a wave's radix sort (3 passes)
-constexpr int kPlanLds = 8192;        // ints: the waves' digit counts, or one bitmap
+constexpr int kPlanDigitMax = 10;     // id bits per pass of a wave's radix sort
+constexpr int kPlanLds = 31 * kPlanThreads;  // ints: the waves' digit counts, or one bitmap (five
+                                             // blocks a compute unit)
 constexpr int kPlanRowShort = 1024;   // ids that a wave sorts by comparison
 constexpr int kPlanLongBlocks = 256;  // blocks after those of the rows, for long rows
-constexpr int kPlanWindowBits = 18;   // ids a bitmap holds: 32 x 8,192
-constexpr int kPlanWindow = 1 << kPlanWindowBits;
+constexpr int kPlanWindow = 32 * kPlanLds;  // ids that a bitmap holds
 constexpr int kPlanWindowShare = 256;  // ids for each window of the list that make a row long
-static_assert(kPlanLds * 32 == kPlanWindow && kPlanLds >= (1ll << (31 - kPlanWindowBits)) &&
-                  kPlanLds == kPlanWaves << kPlanDigitMax,
-              "the row sorts share their LDS");
+static_assert(kPlanLds >= kPlanWaves << kPlanDigitMax, "the row sorts share their LDS");
 constexpr int kFlagShift = 1, kFlagIndex = 2, kFlagUngrouped = 4, kFlagBatchOrder = 8,
               kFlagBatchRange = 16, kFlagAtomCount = 32;
 
@@ -1073,9 +1071,13 @@ __global__ __launch_bounds__(256) void plan_scatter_kernel(PlanJobs J,
 }
 
 // A wave's row of up to 64 ids: each lane's rank by comparison; up to 1,024: the same over
-// tiles of 64; longer: three passes of a stable radix sort of the row (digit counts in LDS,
-// ranks within a wave by ballots).
-__device__ inline void plan_sort_row(int32_t* a, int32_t* b, int len, int digit, int32_t* h) {
+// tiles of 64; longer: an odd number of passes of a stable radix sort of the row (digit counts in
+// LDS, ranks within a wave by ballots).
+struct PlanRadix {
+  int passes, digit;
+};
+
+__device__ inline void plan_sort_row(int32_t* a, int32_t* b, int len, PlanRadix radix, int32_t* h) {
   const int lane = threadIdx.x % kWave;
   if (len <= kWave) {
     const int32_t id = lane < len ? a[lane] : 0x7fffffff;
@@ -1103,8 +1105,8 @@ __device__ inline void plan_sort_row(int32_t* a, int32_t* b, int len, int digit,
     }
     return;
   }
-  const int bins = 1 << digit, per = (bins + kWave - 1) / kWave;
-  for (int pass = 0; pass < 3; ++pass) {
+  const int digit = radix.digit, bins = 1 << digit, per = (bins + kWave - 1) / kWave;
+  for (int pass = 0; pass < radix.passes; ++pass) {
     const int low = pass * digit;
     for (int k = lane; k < bins; k += kWave) h[k] = 0;
     wave_sync();
@@ -1184,22 +1186,23 @@ __device__ inline void plan_sort_long_row(int32_t* __restrict__ a, int32_t* __re
     for (int k = t; k < kPlanLds; k += kPlanThreads) lds[k] = 0;
     __syncthreads();
 #pragma unroll 8
-    for (int32_t k = t; k < len; k += kPlanThreads) atomicAdd(&lds[a[k] >> kPlanWindowBits], 1);
+    for (int32_t k = t; k < len; k += kPlanThreads) atomicAdd(&lds[a[k] / kPlanWindow], 1);
     __syncthreads();
-    int32_t n[kPer], sum = 0, total;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) sum += n[q] = lds[t * kPer + q];
+    int32_t sum = 0, total;
+#pragma unroll 4
+    for (int q = 0; q < kPer; ++q) sum += lds[t * kPer + q];
     int32_t at = plan_block_scan(sum, wsum, total);
-#pragma unroll
+#pragma unroll 4
     for (int q = 0; q < kPer; ++q) {
+      const int32_t c = lds[t * kPer + q];
       lds[t * kPer + q] = at;
-      at += n[q];
+      at += c;
     }
     __syncthreads();
 #pragma unroll 8
     for (int32_t k = t; k < len; k += kPlanThreads) {
       const int32_t id = a[k];
-      b[atomicAdd(&lds[id >> kPlanWindowBits], 1)] = id;
+      b[atomicAdd(&lds[id / kPlanWindow], 1)] = id;
     }
     __syncthreads();
     for (int k = t; k < windows; k += kPlanThreads) a[k] = lds[k];   // the windows' ends
@@ -1214,27 +1217,29 @@ __device__ inline void plan_sort_long_row(int32_t* __restrict__ a, int32_t* __re
     __syncthreads();
 #pragma unroll 8
     for (int32_t k = begin + t; k < end; k += kPlanThreads) {
-      const int32_t low = ids[k] & (kPlanWindow - 1);
+      const int32_t low = ids[k] - win * kPlanWindow;
       atomicOr(&lds[low >> 5], 1 << (low & 31));
     }
     __syncthreads();
     // wave w reads words [w kPer kWave, ..) in kPer rounds of one word a lane
-    int32_t n[kPer], sum = 0, total;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) sum += n[q] = __popc((unsigned)lds[(w * kPer + q) * kWave + lane]);
+    const unsigned* words = reinterpret_cast<const unsigned*>(lds) + w * kPer * kWave + lane;
+    int32_t sum = 0, total;
+#pragma unroll 4
+    for (int q = 0; q < kPer; ++q) sum += __popc(words[q * kWave]);
     int32_t at = begin + __shfl(plan_block_scan(sum, wsum, total), 0, kWave);
-#pragma unroll
+#pragma unroll 1
     for (int q = 0; q < kPer; ++q) {
-      int32_t x = n[q];
+      const unsigned word = words[q * kWave];
+      const int32_t own = __popc(word);
+      int32_t x = own;
 #pragma unroll
       for (int o = 1; o < kWave; o <<= 1) {
         const int32_t y = __shfl_up(x, o, kWave);
         if (lane >= o) x += y;
       }
-      const int word = (w * kPer + q) * kWave + lane;
-      int32_t to = at + x - n[q];
-      for (unsigned bits = (unsigned)lds[word]; bits != 0; bits &= bits - 1)
-        b[to++] = win * kPlanWindow + 32 * word + __ffs(bits) - 1;
+      const int32_t first = win * kPlanWindow + 32 * ((w * kPer + q) * kWave + lane);
+      int32_t to = at + x - own;
+      for (unsigned bits = word; bits != 0; bits &= bits - 1) b[to++] = first + __ffs(bits) - 1;
       at += __shfl(x, kWave - 1, kWave);
     }
     begin = end;
@@ -1242,7 +1247,7 @@ __device__ inline void plan_sort_long_row(int32_t* __restrict__ a, int32_t* __re
 }
 
 __device__ inline bool plan_long_row(int32_t len, int windows) {
-  return len > kPlanRowShort && len >= kPlanWindowShare * windows;
+  return len > kPlanRowShort && windows <= kPlanLds && len >= kPlanWindowShare * windows;
 }
 
 // Rows of few ids on the average: a lane a row of up to kPlanLaneIds, the others of its 64 by
@@ -1255,8 +1260,8 @@ __host__ __device__ inline bool plan_lane_rows(const PlanJob& j) {
   return j.items < kPlanLaneMean * j.rows;
 }
 
-__device__ inline void plan_sort_lane_rows(const PlanJob& j, int64_t first, int windows, int digit,
-                                           int32_t* h) {
+__device__ inline void plan_sort_lane_rows(const PlanJob& j, int64_t first, int windows,
+                                           PlanRadix radix, int32_t* h) {
   const int64_t row = first + threadIdx.x % kWave;
   int32_t r0 = 0, len = 0;
   if (row < j.rows) {
@@ -1279,7 +1284,7 @@ __device__ inline void plan_sort_lane_rows(const PlanJob& j, int64_t first, int 
   for (; left != 0; left &= left - 1) {
     const int l = __ffsll((unsigned long long)left) - 1;
     const int at = __builtin_amdgcn_readlane(r0, l);
-    plan_sort_row(j.tmp + at, j.perm + at, __builtin_amdgcn_readlane(len, l), digit, h);
+    plan_sort_row(j.tmp + at, j.perm + at, __builtin_amdgcn_readlane(len, l), radix, h);
     wave_sync();
   }
 }
@@ -1292,15 +1297,15 @@ __device__ inline void plan_sort_lane_rows(const PlanJob& j, int64_t first, int 
 // edges (16 windows) a row of 2,000 ids takes 393 us by a wave and 529 by a workgroup, one of
 // 8,000 takes 648 and 570.
 __global__ __launch_bounds__(kPlanThreads) void plan_row_sort_kernel(
-    PlanJobs J, const int32_t* __restrict__ grouping, int digit, int64_t row_blocks) {
+    PlanJobs J, const int32_t* __restrict__ grouping, PlanRadix radix, int64_t row_blocks) {
   __shared__ __attribute__((aligned(16))) int32_t lds[kPlanLds];
   const PlanJob& j = J.job[blockIdx.y];
   if (blockIdx.y == kJobReceiver && !(*grouping & kFlagUngrouped)) return;   // uniform
-  const int windows = (int)((j.items + kPlanWindow - 1) >> kPlanWindowBits);
+  const int windows = (int)((j.items + kPlanWindow - 1) / kPlanWindow);
   if ((int64_t)blockIdx.x < row_blocks) {
     const int w = threadIdx.x / kWave;
     if (plan_lane_rows(j)) {
-      plan_sort_lane_rows(j, ((int64_t)blockIdx.x * kPlanWaves + w) * kWave, windows, digit,
+      plan_sort_lane_rows(j, ((int64_t)blockIdx.x * kPlanWaves + w) * kWave, windows, radix,
                           lds + (w << kPlanDigitMax));
       return;
     }
@@ -1309,25 +1314,27 @@ __global__ __launch_bounds__(kPlanThreads) void plan_row_sort_kernel(
     const int r0 = __builtin_amdgcn_readfirstlane(j.ptr[row]);
     const int len = __builtin_amdgcn_readfirstlane(j.ptr[row + 1]) - r0;
     if (!plan_long_row(len, windows))
-      plan_sort_row(j.tmp + r0, j.perm + r0, len, digit, lds + (w << kPlanDigitMax));
+      plan_sort_row(j.tmp + r0, j.perm + r0, len, radix, lds + (w << kPlanDigitMax));
     return;
   }
-  __shared__ int32_t wsum[kPlanWaves], rows[kPlanThreads], count;
+  __shared__ int32_t wsum[kPlanWaves];
+  __shared__ uint64_t found[kPlanWaves];
   const int64_t b = (int64_t)blockIdx.x - row_blocks;
-  for (int64_t base = 0; base < j.rows; base += kPlanLongBlocks * kPlanThreads) {
+  for (int64_t base = b; base < j.rows; base += kPlanLongBlocks * kPlanThreads) {
+    const int64_t row = base + (int64_t)threadIdx.x * kPlanLongBlocks;
+    const uint64_t mine =
+        __ballot(row < j.rows && plan_long_row(j.ptr[row + 1] - j.ptr[row], windows));
+    __syncthreads();                                // found's last reads
+    if (threadIdx.x % kWave == 0) found[threadIdx.x / kWave] = mine;
     __syncthreads();
-    if (threadIdx.x == 0) count = 0;
-    __syncthreads();
-    const int64_t row = base + (int64_t)threadIdx.x * kPlanLongBlocks + b;
-    if (row < j.rows && plan_long_row(j.ptr[row + 1] - j.ptr[row], windows))
-      rows[atomicAdd(&count, 1)] = (int32_t)row;
-    __syncthreads();
-    const int n = count;                                            // uniform
-    for (int k = 0; k < n; ++k) {
-      const int32_t r0 = j.ptr[rows[k]], len = j.ptr[rows[k] + 1] - r0;
-      __syncthreads();
-      plan_sort_long_row(j.tmp + r0, j.perm + r0, len, windows, lds, wsum);
-    }
+    for (int w = 0; w < kPlanWaves; ++w)
+      for (uint64_t left = found[w]; left != 0; left &= left - 1) {   // uniform
+        const int64_t q =
+            base + (int64_t)(w * kWave + __ffsll((unsigned long long)left) - 1) * kPlanLongBlocks;
+        const int32_t r0 = j.ptr[q];
+        __syncthreads();                            // the last row's use of the LDS
+        plan_sort_long_row(j.tmp + r0, j.perm + r0, j.ptr[q + 1] - r0, windows, lds, wsum);
+      }
   }
 }
 
@@ -1443,15 +1450,16 @@ static int build_graph_plan(const int64_t* edge_index, const int64_t* cell_shift
   if (items > 0) {
     hipLaunchKernelGGL(plan_scatter_kernel, dim3((unsigned)grid_1d(items, 256), jobs), dim3(256), 0,
                        s, J, grouping);
-    int digit = 1;
-    while ((int64_t(1) << (3 * digit)) < items && digit < kPlanDigitMax) ++digit;
+    // an odd number of passes ends in perm
+    const int bits = end_bit_for(items), passes = bits <= 3 * kPlanDigitMax ? 3 : 5;
+    const PlanRadix radix{passes, (bits + passes - 1) / passes};
     int64_t row_blocks = 0;
     for (int k = 0; k < jobs; ++k)
       row_blocks = std::max<int64_t>(row_blocks, grid_1d(J.job[k].rows, plan_lane_rows(J.job[k])
                                                                             ? kPlanThreads : kPlanWaves));
     const int64_t long_blocks = items > kPlanRowShort ? kPlanLongBlocks : 0;
     hipLaunchKernelGGL(plan_row_sort_kernel, dim3((unsigned)(row_blocks + long_blocks), jobs),
-                       dim3(kPlanThreads), 0, s, J, grouping, digit, row_blocks);
+                       dim3(kPlanThreads), 0, s, J, grouping, radix, row_blocks);
     XNN_LAUNCH_CHECK();
   }
   return XNN_OK;
