@@ -124,7 +124,7 @@ def test_edge_plan_reports_errors_only():
     (200_000, [1024, 1025, 1500, 90_000]),            # one window of 253,952 ids
     (700_000, [1024, 1025, 5000, 2000, 300_000]),     # three, some of a row's empty
     (300_000, [299_990]),                             # nearly all
-    (5_300_000, [1100, 5375, 5376, 6000, 40_000]),    # 21: a wave sorts up to 5,375 ids
+    (5_300_000, [1100, 10_751, 10_752, 12_000, 40_000]),  # 21: a wave sorts up to 10,751 ids
 ])
 @pytest.mark.parametrize("scattered", [True, False])
 def test_rows_of_any_length_are_sorted(e, hubs, scattered):

@@ -787,7 +787,7 @@ constexpr int kPlanLds = 31 * kPlanThreads;  // ints: the waves' digit counts, o
 constexpr int kPlanRowShort = 1024;   // ids that a wave sorts by comparison
 constexpr int kPlanLongBlocks = 256;  // blocks after those of the rows, for long rows
 constexpr int kPlanWindow = 32 * kPlanLds;  // ids that a bitmap holds
-constexpr int kPlanWindowShare = 256;  // ids for each window of the list that make a row long
+constexpr int kPlanWindowShare = 512;  // ids for each window of the list that make a row long
 static_assert(kPlanLds >= kPlanWaves << kPlanDigitMax, "the row sorts share their LDS");
 constexpr int kFlagShift = 1, kFlagIndex = 2, kFlagUngrouped = 4, kFlagBatchOrder = 8,
               kFlagBatchRange = 16, kFlagAtomCount = 32;
@@ -1293,9 +1293,10 @@ __device__ inline void plan_sort_lane_rows(const PlanJob& j, int64_t first, int 
 // kPlanLongBlocks after them the long rows, a workgroup each: a wave takes 24 ns an id, so one row
 // could hold up the plan. Whole plans of 1,000,000 edges with one row of 16,000 ids: 835 -> 374
 // us, of 500,000: 20.3 -> 4.5 ms, most of it the row's atomics (sorting the list by a library
-// radix sort: 678 us, 6.2 ms); 40 rows of 25,000: 2.5 ms (2.9). kPlanWindowShare: of 4,000,000
-// edges (16 windows) a row of 2,000 ids takes 393 us by a wave and 529 by a workgroup, one of
-// 8,000 takes 648 and 570.
+// radix sort: 678 us, 6.2 ms); 40 rows of 25,000: 2.5 ms (2.9).
+// kPlanWindowShare: a workgroup takes about 11 us a window and far fewer of them run at once:
+// of 4,000,000 edges (16 windows) a row of 2,000 ids takes 393 us by a wave and 529 by a
+// workgroup, one of 8,000 takes 636 and 581; sorting 700 rows of 3,150 (9 windows) 194 and 413.
 __global__ __launch_bounds__(kPlanThreads) void plan_row_sort_kernel(
     PlanJobs J, const int32_t* __restrict__ grouping, PlanRadix radix, int64_t row_blocks) {
   __shared__ __attribute__((aligned(16))) int32_t lds[kPlanLds];
