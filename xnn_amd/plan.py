@@ -1,7 +1,7 @@
 """Edge plans: the int32 edge streams and CSR orderings the HIP kernels walk.
 
 An :class:`EdgePlan` is built once per edge list (on the device, by
-``xnn_edge_plan``) and cached on the graph. It holds
+``xnn_graph_plan``) and cached on the graph. It holds
 
 * ``src``, ``dst`` (int32) and ``shift`` (three signed 10-bit fields in one
   int32) for every edge, in the edge list's own order;
